@@ -386,7 +386,7 @@ static int check_abort(Context &c, const char *what)
     if (flag) {
         int y = flag - 1;
         double m = 0.0;
-        (void) hipMemcpy(&m, c.cflmax + c.d.qpts, sizeof(double), hipMemcpyDeviceToHost);
+        (void) hipMemcpy(&m, c.cflmax + (size_t) c.d.qpts * CFL_STRIDE, sizeof(double), hipMemcpyDeviceToHost);
         printf("Pass1:  CFL[%d]:%e, Max:%e dt:%e.  CFL condition violated.\n", y, m * c.d.dt,
                2.8, c.d.dt);
         printf("%s failure\n", what);
@@ -698,7 +698,7 @@ int c_init(int Nx, int Ny, int Nz, double Lx, double Lz, double Re, double flux,
         {(void **) &c.W2b, sizeof(cplx) * (size_t) d.qpts * 6 * d.Pz * d.Mx, true, false},
         {(void **) &c.SP, sizeof(cplx) * 6 * (size_t) d.Nz * d.qpts * d.Mx, true, false},
         {(void **) &c.flowdev, sizeof(double) * 3 * (size_t) d.Px * d.qpts * d.Pz, false, false},
-        {(void **) &c.cflmax, sizeof(double) * (d.qpts + 1), false, false},
+        {(void **) &c.cflmax, sizeof(double) * (d.qpts + 1) * CFL_STRIDE, false, false},
         {(void **) &c.dotpart, sizeof(double) * ndot, false, false},
         {(void **) &c.scal, sizeof(double) * 8 * nm, false, false},
         {(void **) &c.abort_flag, 4 * sizeof(int), false, false},
@@ -852,7 +852,7 @@ static int primal_run(int ru_steps, sc_complex *C_given, hipMemcpyKind in, hipMe
     if (int rc = copy_to_slots(c, c.MC, 0, c.C)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     // each CFL check clears the maxima it read; a run starts from zero
-    SC_HIP(hipMemsetAsync(c.cflmax, 0, sizeof(double) * c.d.qpts, c.stream));
+    SC_HIP(hipMemsetAsync(c.cflmax, 0, sizeof(double) * c.d.qpts * CFL_STRIDE, c.stream));
     c.status = 0;
     // the stage working on stored state j = 3(n - ru) + k writes the cached
     // fields of that state (its fields equal those of rebuild(MC[j])), except
@@ -950,7 +950,7 @@ static int tangent_run(int start, int end, sc_complex *IC_given, unsigned inhomo
     if (int rc = copy_to_slots(c, c.MIC, 3L * start, c.IC)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     // each CFL check clears the maxima it read; a run starts from zero
-    SC_HIP(hipMemsetAsync(c.cflmax, 0, sizeof(double) * c.d.qpts, c.stream));
+    SC_HIP(hipMemsetAsync(c.cflmax, 0, sizeof(double) * c.d.qpts * CFL_STRIDE, c.stream));
     // member windows: a member is zero from the end of its window on (a
     // zero tangent stays zero without the mean-velocity source), so the
     // stored states after its window are zero and its result stays at

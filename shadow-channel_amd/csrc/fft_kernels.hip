@@ -389,7 +389,7 @@ __global__ __launch_bounds__(BLK) void k_xmix(XmixArgs a, PlanDev px, const real
             double b = cw[0];
 #pragma unroll
             for (int w = 1; w < BLK / 64; ++w) b = fmax(b, cw[w]);
-            atomic_max_nonneg(&a.cflmax[y], b);
+            atomic_max_nonneg(&a.cflmax[y * CFL_STRIDE], b);
         }
     }
     if constexpr (MODE == XM_PHYS) return;

@@ -191,22 +191,22 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
     if constexpr (MODE == XM_PRIMAL || MODE == XM_TANGENT) {
         if (a.check_cfl) {
             // block maxima: within each wave by lane exchanges, then the
-            // waves' maxima through LDS (a maximum is exact in any order)
+            // waves' maxima through LDS (a maximum is exact in any order); the
+            // second plane only where the block meets it
             __shared__ double cw[2][T / 64];
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
+            const int np = z0 + nr > Pz ? 2 : 1;
+            for (int p = 0; p < np; ++p) {
                 double m = cmax[p];
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
                 if ((threadIdx.x & 63) == 0) cw[p][threadIdx.x >> 6] = m;
             }
             __syncthreads();
-            if (threadIdx.x < 2) {
+            if ((int) threadIdx.x < np) {
                 double b = cw[threadIdx.x][0];
 #pragma unroll
                 for (int w = 1; w < T / 64; ++w) b = fmax(b, cw[threadIdx.x][w]);
-                const int y = y0 + threadIdx.x;
-                if (y < a.qpts) atomic_max_nonneg(&a.cflmax[y], b);
+                atomic_max_nonneg(&a.cflmax[(y0 + threadIdx.x) * CFL_STRIDE], b);
             }
         }
     }

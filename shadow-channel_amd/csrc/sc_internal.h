@@ -26,6 +26,10 @@ typedef double2 cplx;
 // kernel error bits in abort_flag[2]
 constexpr int SC_KERR_SOLVE_WAIT = 1;   // band solve: factor staging never signalled
 
+// doubles between the planes' CFL maxima: a cache line each, as the blocks of a
+// launch update them with atomics (145 planes in 10 lines: 4 us of the primal x
+// kernel's 27 at 64x64x97)
+constexpr int CFL_STRIDE = 16;
 constexpr int MAXF = 12;        // fields in one z-inverse launch
 constexpr int FFT_TILE = 2048;  // complex values (data + twiddles) in one transform block
 constexpr int FFT_BLOCK = 256;  // threads of a transform block
@@ -189,8 +193,9 @@ struct Context {
     size_t wslot = 0;                           // complex values per state
     std::vector<char> wvalid;                   // entry j holds MC[j]'s fields
     double *flowdev = nullptr;                  // [3][Px][qpts][Pz]
-    // [qpts + 1]: per-plane CFL maxima of the running check (zero between
-    // checks), then the maximum of the plane that stopped a run
+    // [qpts + 1][CFL_STRIDE]: per-plane CFL maxima of the running check (zero
+    // between checks), then the maximum of the plane that stopped a run; the
+    // first value of each
     double *cflmax = nullptr;
     double *dotpart = nullptr;                  // partial sums
     size_t ndotpart = 0;                        // doubles in dotpart
@@ -410,17 +415,17 @@ __device__ __forceinline__ void cfl_check_block(double *cflmax, int qpts, double
     __syncthreads();
     const bool live = *abort_flag == 0;
     for (int y = threadIdx.x; y < qpts; y += blockDim.x) {
-        if (live && cflmax[y] * dt >= 2.8) atomicMin(&first, y);
+        if (live && cflmax[y * sc::CFL_STRIDE] * dt >= 2.8) atomicMin(&first, y);
     }
     __syncthreads();
     const int y0 = first;
     if (y0 < qpts && threadIdx.x == 0) {
-        cflmax[qpts] = cflmax[y0];
+        cflmax[qpts * sc::CFL_STRIDE] = cflmax[y0 * sc::CFL_STRIDE];
         abort_flag[1] = slot;
         abort_flag[0] = 1 + y0;
     }
     __syncthreads();
-    for (int y = threadIdx.x; y < qpts; y += blockDim.x) cflmax[y] = 0.0;
+    for (int y = threadIdx.x; y < qpts; y += blockDim.x) cflmax[y * sc::CFL_STRIDE] = 0.0;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs in launch order, and
