@@ -365,20 +365,6 @@ static void pass2_adjoint_pair(Context &c, const cplx *AUb, const cplx *wa, cons
     }
 }
 
-// Kernel error bits (abort_flag[2]) left by the last run: reported once
-// through last_error() and cleared.
-static int check_kernel_error(Context &c)
-{
-    int e = 0;
-    SC_HIP(hipMemcpy(&e, c.abort_flag + 2, sizeof(int), hipMemcpyDeviceToHost));
-    if (!e) return SC_OK;
-    SC_HIP(hipMemset(c.abort_flag + 2, 0, sizeof(int)));
-    last_error() = "kernel error " + std::to_string(e) +
-                   ((e & SC_KERR_SOLVE_WAIT) ? ": band solve factor staging never signalled" : "");
-    fprintf(stderr, "shadow-channel: %s\n", last_error().c_str());
-    return SC_EDEVICE;
-}
-
 static int check_abort(Context &c, const char *what)
 {
     int flag = 0;
@@ -890,7 +876,6 @@ static int primal_run(int ru_steps, sc_complex *C_given, hipMemcpyKind in, hipMe
         return SC_OK;
     });
     if (!rc) rc = stream_sync(c);
-    if (!rc) rc = check_kernel_error(c);
     if (rc) return rc;
     // after an abort the queued launches did nothing: no cached field is
     // valid, and the states from the stopped step on were not written
@@ -1002,7 +987,6 @@ static int tangent_run(int start, int end, sc_complex *IC_given, unsigned inhomo
     return SC_OK;
     });
     if (!rc) rc = stream_sync(c);
-    if (!rc) rc = check_kernel_error(c);
     if (rc) return rc;
     check_abort(c, "Pass1");
     SC_HIP(hipMemcpy(IC_given, c.IC, cbm, out));
@@ -1156,7 +1140,6 @@ static int adjoint_run(int start, int end, sc_complex *AC_given, double strength
         return SC_OK;
     });
     if (!rc) rc = stream_sync(c);
-    if (!rc) rc = check_kernel_error(c);
     if (rc) return rc;
     SC_HIP(hipMemcpy(AC_given, c.AC, cbm, out));
     return SC_OK;
@@ -1190,7 +1173,6 @@ static int adjoint_objective_run(int start, int end, sc_complex *AC_given, doubl
     }
     if (windows) zero_pending(c, end + 1);   // never started: win <= end
     int rc = stream_sync(c);
-    if (!rc) rc = check_kernel_error(c);
     if (rc) return rc;
     SC_HIP(hipMemcpy(AC_given, c.AC, cbm, out));
     return SC_OK;

@@ -67,8 +67,8 @@ struct IadjArgs {
     const double *Kx, *Kz, *Qs, *Qps, *Qpps, *Rs, *Rps, *Rp0;
     const double *tRw, *tRpw;   // [q][dimR]: Rw, Rpw transposed
     // LU factors of the stage's implicit operators (the adjoint's): the solve
-    // images of the setup (alpha La, beta Lb: [block][parity][chain row][W][sbt]
-    // over columns z Mx + x, rows z <= Nz/2 only when mirror) and the mean's [dimR][5]
+    // images of the setup (alpha La, beta Lb: blocks of sbt columns over columns
+    // z Mx + x, rows z <= Nz/2 only when mirror) and the mean's
     const double *La, *Lb, *Lm;
     int sbt, mirror;
     const double *lift;    // [4][q]: lv, lv', lv'', lg
@@ -81,26 +81,27 @@ __device__ __forceinline__ cplx cadd(cplx a, cplx b) { return make_double2(a.x +
 __device__ __forceinline__ cplx cscale(cplx a, double s) { return make_double2(a.x * s, a.y * s); }
 
 // Forward and back substitution on the rows of parity p of a stride-2 band
-// system, in place on vec (row i at vec[i]), with the LU factors of the
-// setup (no pivoting; per matrix row W = 2 DL + 1 entries: j < DL the
-// multiplier L(i, i - 2(DL - j)), DL the reciprocal of U(i, i), j > DL
-// U(i, i + 2(j - DL)), zero outside the matrix).  Chain row r (matrix row
-// p + 2r) has its entry j at f0[r rs + j js].  The last DL values stay in
-// registers, so one row waits only on the row before it.
+// system, in place on vec (row i at vec[i]), with column cc of a factor image
+// of the setup (sbt columns, both parities one after the other: see dLa in
+// sc_internal.h; no pivoting).  The last DL values stay in registers, so one
+// row waits only on the row before it.
 template <int DL>
-__device__ void chain_subst(cplx *vec, const double *f0, size_t rs, size_t js, int N, int p)
+__device__ void chain_subst(cplx *vec, const double *img, int sbt, int cc, int N, int p)
 {
-    const int nr = (N - p + 1) / 2;
+    const int nr = (N - p + 1) / 2, nrp = solve_rows(N);
+    const double *L = img + (size_t) p * nrp * sbt * (2 * DL + 1) + cc * DL;
+    const double *U = L + (size_t) nrp * sbt * DL, *D = U + (size_t) nrp * sbt * DL - cc * (DL - 1);
+    const size_t rs = (size_t) sbt * DL;
     cplx y[DL];
 #pragma unroll
     for (int m = 0; m < DL; ++m) y[m] = make_double2(0.0, 0.0);
 #pragma unroll 4
     for (int r = 0; r < nr; ++r) {
-        const double *f = f0 + r * rs;
         cplx b = vec[p + 2 * r];
 #pragma unroll
         for (int m = 1; m <= DL; ++m) {
-            const double l = f[(DL - m) * js];
+            // L(r, m); rows before the first multiply zeros
+            const double l = L[max(r - m + 1, 0) * rs + m - 1];
             b.x -= l * y[m - 1].x;
             b.y -= l * y[m - 1].y;
         }
@@ -113,15 +114,14 @@ __device__ void chain_subst(cplx *vec, const double *f0, size_t rs, size_t js, i
     for (int m = 0; m < DL; ++m) y[m] = make_double2(0.0, 0.0);
 #pragma unroll 4
     for (int r = nr - 1; r >= 0; --r) {
-        const double *f = f0 + r * rs;
         cplx v = vec[p + 2 * r];
 #pragma unroll
         for (int t = 1; t <= DL; ++t) {
-            const double u = f[(DL + t) * js];
+            const double u = U[r * rs + t - 1];
             v.x -= u * y[t - 1].x;
             v.y -= u * y[t - 1].y;
         }
-        v = cscale(v, f[DL * js]);
+        v = cscale(v, D[(size_t) r * sbt]);
 #pragma unroll
         for (int m = DL - 1; m > 0; --m) y[m] = y[m - 1];
         y[0] = v;
@@ -275,7 +275,7 @@ __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
     __syncthreads();
     if (r < dR) (isb ? sbe : sal)[r] = c;
     __syncthreads();
-    if (tid < 4) chain_subst<2>(tid < 2 ? sal : sbe, a.Lm + (tid & 1) * 5, 10, 1, dR, tid & 1);
+    if (tid < 4) chain_subst<2>(tid < 2 ? sal : sbe, a.Lm, 1, 0, dR, tid & 1);
     __syncthreads();
     // the mean's Gauss-point values sum all dimR coefficients
     for (int i = tid; i < dR; i += IA_THREADS) {
@@ -435,17 +435,12 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
         const int kind = tid / IA_XG, t = tid % IA_XG;
         if (valid(t)) {
             const int zi = (a.mirror && z > Nz / 2) ? Nz - z : z;
-            const size_t col = (size_t) zi * Mx + x0 + t, blk = col / a.sbt, cc = col % a.sbt;
-            const int par = kind & 1, sbt = a.sbt;
-            if (kind < 2) {
-                const size_t rmax = (dQ + 1) / 2;
-                chain_subst<4>(sal + t * dR, a.La + ((blk * 2 + par) * rmax * 9) * sbt + cc,
-                               (size_t) 9 * sbt, sbt, dQ, par);
-            } else {
-                const size_t rmax = (dR + 1) / 2;
-                chain_subst<2>(sbe + t * dR, a.Lb + ((blk * 2 + par) * rmax * 5) * sbt + cc,
-                               (size_t) 5 * sbt, sbt, dR, par);
-            }
+            const size_t col = (size_t) zi * Mx + x0 + t, blk = col / a.sbt;
+            const int cc = (int) (col % a.sbt);
+            if (kind < 2)
+                chain_subst<4>(sal + t * dR, a.La + blk * 2 * solve_rows(dQ) * 9 * a.sbt, a.sbt, cc, dQ, kind & 1);
+            else
+                chain_subst<2>(sbe + t * dR, a.Lb + blk * 2 * solve_rows(dR) * 5 * a.sbt, a.sbt, cc, dR, kind & 1);
         }
     }
     __syncthreads();

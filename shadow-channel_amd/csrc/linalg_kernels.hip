@@ -1513,28 +1513,39 @@ void launch_force(Context &c, const cplx *Usrc, int adj) { launch_force(c, Usrc,
 // the state), the LU solve with the stage's implicit operator, then
 // C <- E' X + dt d_{k+1} F2, the next stage's carried right-hand side.  The
 // even and odd rows of the stride-2 bands decouple, so one chain is one
-// (column, field, parity).
+// (column, field, parity), and the real and imaginary parts are chains of
+// their own.
 //
-// The LU factors are formed once at init with the pivots inverted, so a chain
-// is a pure multiply-add recurrence.  A block stages the factors and vectors
-// of SBT columns of one (field, parity) in LDS with all its threads, runs the
-// SBT chains with one thread each (the last DL solved values in registers),
-// and writes back with all its threads.  The loops over rows stay rolled: the
-// kernel fits the instruction cache at every grid size.
+// A block solves SBT columns of one (field, parity) for up to MB members, which
+// all have the same operator.  One wave runs the chains (2 SBT lanes a member,
+// the last DL values in registers); the other three, the workers, own the rows:
+// they form the right-hand sides, bring the U factors into LDS and form the next
+// stage's operator entries while the chain wave runs its forward sweep, and write
+// the results.  The chain is what the kernel waits for, and a lone wave issues
+// one instruction every four or five clocks, so its cost is its instructions: the
+// factors are laid out (setup.cpp) so that a row's operands are whole 16-byte LDS
+// reads at immediate offsets, rows and vectors are padded with zeros to groups
+// of eight so that nothing is clamped or predicated.  Two sweeps of 48 rows took
+// 7 us with a row-major image and clamped rows, and take 4.2 with four blocks'
+// chains on a CU (10000 clocks; 32 rows 2 us).  Measured, stage average: one
+// 64x97x64 solution 23.0 -> 16.0 us, 32 members 455 -> 232 us, 32x65x32 12.7 ->
+// 8.0 us, 128x129x128 with two members 185 -> 143 us; the members' launch is
+// bound by its 0.8 GB of vectors (4.9 TB/s of a large copy: 165 us).
 //
 // The mean mode (kz = kx = 0; channel/project0.c:22-271,
-// channel/increproject0.c:14-312, channel/adjproject0.c:8-310) runs in one
-// extra block: real-part-only forcing fa = Re(Hx)-projection and
-// fb = Re(Hz)-projection, read as the pair Fb(0,0) = (fa, fb); the flux
-// correction alpha += (target - sum_i rowsum_i Re alpha_i) add / 2.
+// channel/increproject0.c:14-312, channel/adjproject0.c:8-310): real-part-only
+// forcing fa = Re(Hx)-projection and fb = Re(Hz)-projection, read as the pair
+// Fb(0,0) = (fa, fb); the flux correction
+// alpha += (target - sum_i rowsum_i Re alpha_i) add / 2.
 struct SolveArgs {
     const double *Qs, *Qps, *Qpps, *Rs, *Rps, *Kx, *Kz;
-    const double *La, *Lb;             // factors of this stage, [z][row][2DL+1][x]
-    const double *Lm, *add, *rowsum;   // mean mode: factors [row][5], flux vector, row sums
+    const double *La, *Lb;             // factor images of this stage (SolveImage)
+    const double *Lm, *add, *rowsum;   // mean mode: its image, flux vector, row sums
     const cplx *Fa, *Fb;               // projection for this stage's RHS
     const cplx *Fa2, *Fb2;             // projection for the next-stage RHS
     int Nz, Mx, dimR, dimQ, k, has_next;
     int nblk;                          // column blocks of SBT columns
+    int ngrp;                          // groups of MB members
     int nyq_mean;                      // the mean mode runs in the Nyquist blocks' first (1) or in an extra block (0)
     int mirror;                        // factor images of rows z > Nz/2 are those of row Nz - z
     double dtc, dtd;                   // dt c_k, dt d_{k+1}
@@ -1543,8 +1554,7 @@ struct SolveArgs {
     double target_alt;                 // ... of the members m with bit m of alt_mask set
     unsigned alt_mask;
     const int *abort_flag;
-    int *err;                          // device error word (SC_KERR_* bits)
-    // member strides (grid z = member) of C, Cs, Fa, Fb, Fa2, Fb2, Src
+    // member strides of C, Cs, Fa, Fb, Fa2, Fb2, Src
     size_t ms_c, ms_cs, ms_fa, ms_fb, ms_fa2, ms_fb2, ms_src;
     // optional right-hand-side source of the stage (C layout), added after
     // the explicit part and the forcing, before the solve (all modes)
@@ -1555,380 +1565,216 @@ struct SolveArgs {
     // follows the solve (the host loop applies P at each step's start)
     int exact_mean;
     const double *add_mass;            // Rs^{-1} w1
-    int nm;                            // members of the launch (grid z: groups of them)
+    int nm;                            // members of the launch
 };
 
-// explicit band operator row entry A(i, i+2m)
-__device__ __forceinline__ double op_entry(const SolveArgs &a, int var, int i, int m, double k2, double coef)
+// Entries A(i, i + 2m), m = -DL .. DL, of the explicit operator of a row: the v
+// operator -(k2 Qs + Qps) + coef (k2^2 Qs + 2 k2 Qps + Qpps) (DL = 4), the omega_y
+// operator Rs + coef (Rps + k2 Rs) (DL = 2).  The Gram bands are zero outside the
+// matrix; Qs reaches |m| = 4, Qps 3, Qpps 2, Rs 2 and Rps 1.  Which product of
+// k2^2 Qs + 2 k2 Qps is rounded is written out, so that every block shape forms
+// the same bits.
+template <int DL>
+__device__ __forceinline__ void op_row(const SolveArgs &a, int i, double k2, double coef, double *e)
 {
-    if (var == 0) {
-        int e = i * 9 + 4 + m;
-        double s = k2 * k2;
-        return -(k2 * a.Qs[e] + a.Qps[e]) + coef * (s * a.Qs[e] + 2. * k2 * a.Qps[e] + a.Qpps[e]);
+    if constexpr (DL == 4) {
+        const double s = k2 * k2, t = 2. * k2;
+        const double *qs = a.Qs + i * 9, *qp = a.Qps + i * 9, *qq = a.Qpps + i * 9;
+#pragma unroll
+        for (int j = 0; j < 9; ++j) {
+            const bool p = j > 0 && j < 8, q = j > 1 && j < 7;
+            double v = p ? __builtin_fma(s, qs[j], t * qp[j]) : s * qs[j];
+            if (q) v += qq[j];
+            e[j] = __builtin_fma(coef, v, -(p ? __builtin_fma(k2, qs[j], qp[j]) : k2 * qs[j]));
+        }
+    } else {
+        const double *rs = a.Rs + i * 5, *rp = a.Rps + i * 5;
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            e[j] = __builtin_fma(coef, j > 0 && j < 4 ? __builtin_fma(k2, rs[j], rp[j]) : k2 * rs[j], rs[j]);
     }
-    int e = i * 5 + 2 + m;
-    return a.Rs[e] + coef * (a.Rps[e] + k2 * a.Rs[e]);
 }
 
-// Forward and back substitution of one chain held in LDS.  Factors of row r:
-// f[r*fr + j*fj], j = DL - m for L(r, r-m), j = DL for 1/U(r, r),
-// j = DL + u for U(r, r+u); entries that fall outside the matrix are zero.
-// v: right-hand side in, solution out, row r at v[r*vr].
+// Forward and back substitution of one part (real or imaginary) of one column
+// held in LDS: fl, bu, bi the image's factors of the column (rows SBT DL, SBT DL
+// and SBT apart), v its part of the vector, rows vr apart, nrp rows (a multiple
+// of eight) between rows of zeros.  Factors of rows past the chain are zero.
 //
 // Forward sweep, row s: x_s = v_s - L(s,DL) x_{s-DL} - ... - L(s,1) x_{s-1},
 // the terms applied farthest first (the reference's order).  It runs skewed:
-// the iteration that produces x_{r-1} applies it to the rows r .. r+DL-1 at
-// once (term m = k+1 of row r+k), so the DL multiply-adds of an iteration are
-// independent and only one of them waits for the previous iteration.  Every
-// row still sees its terms in the same order, so the result is the same as
-// the row-by-row sweep.  P[k] holds row r+k with its terms DL .. k+2 applied.
+// the step that produces x_r applies it to the rows r+1 .. r+DL at once, so its
+// DL multiply-adds are independent and only one of them is on the path to the
+// next step.  P[k] holds row r+k with its terms DL .. k+2 applied;
+// fl[r][k] = L(r+k, k+1).
 //
-// Operands stream from LDS through two register buffers of two rows each,
-// used in turn by a body of four rows: the loads for rows r+4, r+5 go into
-// the buffer rows r, r+1 have just used, issued before the arithmetic of rows
-// r+2, r+3 (a scheduling barrier keeps them there), with no register copies
-// that would wait for them.  Row indices are clamped into the chain; values
-// of rows past the end are never stored.
-template <int DL>
-struct FwdOps {
-    double c[2][DL];   // c[i][k] = L(r+i+k, k+1)
-    double2 vn[2];     // right-hand side of row r+i+DL-1
-};
-
-template <int DL>
-__device__ __forceinline__ void fwd_load(FwdOps<DL> &o, const double *f, int fr, int fj,
-                                         const double2 *v, int vr, int r, int nr)
-{
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int k = 0; k < DL; ++k) o.c[i][k] = f[min(r + i + k, nr - 1) * fr + (DL - 1 - k) * fj];
-        o.vn[i] = v[min(r + i + DL - 1, nr - 1) * vr];
-    }
-}
-
-template <int DL>
-__device__ __forceinline__ void fwd_step(const double *c, double2 vn, double2 *P, double2 &xm1,
-                                         double2 *v, int vr, int r)
-{
-    double2 x = P[0];
-    x.x -= c[0] * xm1.x;
-    x.y -= c[0] * xm1.y;
-#pragma unroll
-    for (int k = 1; k < DL - 1; ++k) {
-        P[k - 1].x = P[k].x - c[k] * xm1.x;
-        P[k - 1].y = P[k].y - c[k] * xm1.y;
-    }
-    P[DL - 2].x = vn.x - c[DL - 1] * xm1.x;
-    P[DL - 2].y = vn.y - c[DL - 1] * xm1.y;
-    v[r * vr] = x;
-    xm1 = x;
-}
-
-template <int DL>
-__device__ __forceinline__ void chain_forward(const double *f, int fr, int fj, double2 *v, int vr,
-                                              int nr)
-{
-    double2 P[DL - 1];
-#pragma unroll
-    for (int k = 0; k < DL - 1; ++k) P[k] = v[min(k, nr - 1) * vr];
-    double2 xm1 = make_double2(0.0, 0.0);
-    FwdOps<DL> X, Y;
-    fwd_load<DL>(X, f, fr, fj, v, vr, 0, nr);
-    fwd_load<DL>(Y, f, fr, fj, v, vr, 2, nr);
-    int r = 0;
-    for (; r + 4 <= nr; r += 4) {
-        fwd_step<DL>(X.c[0], X.vn[0], P, xm1, v, vr, r);
-        fwd_step<DL>(X.c[1], X.vn[1], P, xm1, v, vr, r + 1);
-        fwd_load<DL>(X, f, fr, fj, v, vr, r + 4, nr);
-        __builtin_amdgcn_sched_barrier(0);
-        fwd_step<DL>(Y.c[0], Y.vn[0], P, xm1, v, vr, r + 2);
-        fwd_step<DL>(Y.c[1], Y.vn[1], P, xm1, v, vr, r + 3);
-        fwd_load<DL>(Y, f, fr, fj, v, vr, r + 6, nr);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    // fewer than four rows left: X holds rows r, r+1, Y rows r+2, r+3
-    if (r < nr) fwd_step<DL>(X.c[0], X.vn[0], P, xm1, v, vr, r);
-    if (r + 1 < nr) fwd_step<DL>(X.c[1], X.vn[1], P, xm1, v, vr, r + 1);
-    if (r + 2 < nr) fwd_step<DL>(Y.c[0], Y.vn[0], P, xm1, v, vr, r + 2);
-}
-
 // Backward sweep, row r: x_r = (v_r - U(r,1) x_{r+1} - ... - U(r,DL) x_{r+DL})
-// / U(r,r), nearest term first (the reference's order).  Same two-buffer
-// stream of operands as the forward sweep, rows descending.
-template <int DL>
-struct BwdOps {
-    double u[2][DL + 1];   // U(r-i, r-i+1..r-i+DL), then 1/U(r-i, r-i)
-    double2 v[2];          // right-hand side of row r-i
+// / U(r,r), nearest term first (the reference's order); bu[r][m-1] = U(r, r+m),
+// bi[r] = 1 / U(r, r).
+//
+// Operands stream through two register buffers of four rows each: the loads of
+// the next four rows are issued before the arithmetic of the current ones (a
+// scheduling barrier keeps them there).
+// (one row's operands are named values: arrays of rows would be kept in
+// scratch memory)
+template <int DL> struct RowFactors;
+template <> struct RowFactors<4> {
+    double2 p, q;
+    __device__ __forceinline__ void load(const double *f)
+    {
+        p = ((const double2 *) f)[0];
+        q = ((const double2 *) f)[1];
+    }
+    template <int K> __device__ __forceinline__ double get() const
+    {
+        return K == 0 ? p.x : K == 1 ? p.y : K == 2 ? q.x : q.y;
+    }
+};
+template <> struct RowFactors<2> {
+    double2 p;
+    __device__ __forceinline__ void load(const double *f) { p = ((const double2 *) f)[0]; }
+    template <int K> __device__ __forceinline__ double get() const { return K == 0 ? p.x : p.y; }
+};
+
+template <int DL> struct FwdRow {
+    RowFactors<DL> c;
+    double vn;
+};
+template <int DL, int FR, int VR> struct FwdRows {
+    FwdRow<DL> a, b, c, d;
+    __device__ __forceinline__ void load1(FwdRow<DL> &o, const double *fl, const double *v)
+    {
+        o.c.load(fl);
+        o.vn = v[(DL - 1) * VR];
+    }
+    __device__ __forceinline__ void load(const double *fl, const double *v)
+    {
+        load1(a, fl, v);
+        load1(b, fl + FR * DL, v + VR);
+        load1(c, fl + 2 * FR * DL, v + 2 * VR);
+        load1(d, fl + 3 * FR * DL, v + 3 * VR);
+    }
+};
+
+// P0 .. P2 (P0 only for DL = 2): the next rows with their terms applied so far
+struct FwdState {
+    double P0, P1, P2, x;
 };
 
 template <int DL>
-__device__ __forceinline__ void bwd_load(BwdOps<DL> &o, const double *f, int fr, int fj,
-                                         const double2 *v, int vr, int r)
+__device__ __forceinline__ void fwd_step(const FwdRow<DL> &o, FwdState &s, double *v)
 {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rr = max(r - i, 0);
-#pragma unroll
-        for (int k = 1; k <= DL; ++k) o.u[i][k - 1] = f[rr * fr + (DL + k) * fj];
-        o.u[i][DL] = f[rr * fr + DL * fj];
-        o.v[i] = v[rr * vr];
+    const double x = __builtin_fma(-o.c.template get<0>(), s.x, s.P0);
+    if constexpr (DL == 4) {
+        s.P0 = __builtin_fma(-o.c.template get<1>(), s.x, s.P1);
+        s.P1 = __builtin_fma(-o.c.template get<2>(), s.x, s.P2);
+        s.P2 = __builtin_fma(-o.c.template get<3>(), s.x, o.vn);
+    } else {
+        s.P0 = __builtin_fma(-o.c.template get<1>(), s.x, o.vn);
     }
+    v[0] = x;
+    s.x = x;
 }
 
-template <int DL>
-__device__ __forceinline__ void bwd_step(const double *u, double2 x, double2 *w, double2 *v,
-                                         int vr, int r)
+template <int DL, int FR, int VR>
+__device__ __forceinline__ void chain_forward(const double *fl, double *v, int nrp)
 {
-#pragma unroll
-    for (int k = 1; k <= DL; ++k) {
-        x.x -= u[k - 1] * w[k - 1].x;
-        x.y -= u[k - 1] * w[k - 1].y;
-    }
-    x.x *= u[DL];
-    x.y *= u[DL];
-#pragma unroll
-    for (int m = DL - 1; m > 0; --m) w[m] = w[m - 1];
-    w[0] = x;
-    v[r * vr] = x;
-}
-
-template <int DL>
-__device__ __forceinline__ void chain_backward(const double *f, int fr, int fj, double2 *v, int vr,
-                                               int nr)
-{
-    double2 w[DL];
-#pragma unroll
-    for (int m = 0; m < DL; ++m) w[m] = make_double2(0.0, 0.0);
-    BwdOps<DL> X, Y;
-    bwd_load<DL>(X, f, fr, fj, v, vr, nr - 1);
-    bwd_load<DL>(Y, f, fr, fj, v, vr, nr - 3);
-    int r = nr - 1;
-    // rows below r - 3 still hold forward values until their own step
-    for (; r >= 3; r -= 4) {
-        bwd_step<DL>(X.u[0], X.v[0], w, v, vr, r);
-        bwd_step<DL>(X.u[1], X.v[1], w, v, vr, r - 1);
-        bwd_load<DL>(X, f, fr, fj, v, vr, r - 4);
+    FwdState s{v[0], DL == 4 ? v[VR] : 0.0, DL == 4 ? v[2 * VR] : 0.0, 0.0};
+    FwdRows<DL, FR, VR> A, B;
+    A.load(fl, v);
+    for (int r = 0; r < nrp; r += 8) {
+        B.load(fl + 4 * FR * DL, v + 4 * VR);
         __builtin_amdgcn_sched_barrier(0);
-        bwd_step<DL>(Y.u[0], Y.v[0], w, v, vr, r - 2);
-        bwd_step<DL>(Y.u[1], Y.v[1], w, v, vr, r - 3);
-        bwd_load<DL>(Y, f, fr, fj, v, vr, r - 6);
+        fwd_step<DL>(A.a, s, v);
+        fwd_step<DL>(A.b, s, v + VR);
+        fwd_step<DL>(A.c, s, v + 2 * VR);
+        fwd_step<DL>(A.d, s, v + 3 * VR);
+        // past the last row: the rows after the image and the vector's padding,
+        // loaded and not used
+        A.load(fl + 8 * FR * DL, v + 8 * VR);
         __builtin_amdgcn_sched_barrier(0);
-    }
-    // fewer than four rows left: X holds rows r, r-1, Y rows r-2, r-3
-    if (r >= 0) bwd_step<DL>(X.u[0], X.v[0], w, v, vr, r);
-    if (r >= 1) bwd_step<DL>(X.u[1], X.v[1], w, v, vr, r - 1);
-    if (r >= 2) bwd_step<DL>(Y.u[0], Y.v[0], w, v, vr, r - 2);
-}
-
-// inlined at every call site: the pointers then stay LDS pointers (a call
-// would pass them as generic addresses, and every access would go through
-// the flat path)
-template <int DL>
-__device__ __forceinline__ void chain_subst(const double *f, int fr, int fj, double2 *v, int vr,
-                                            int nr)
-{
-    if (nr <= 0) return;
-    chain_forward<DL>(f, fr, fj, v, vr, nr);
-    chain_backward<DL>(f, fr, fj, v, vr, nr);
-}
-
-// The same sweeps with NB operand buffers of two rows (prefetch distance
-// 2 NB - 2 rows): the chain waits less on LDS latency.
-template <int DL, int NB>
-__device__ __forceinline__ void chain_forward_n(const double *f, int fr, int fj, double2 *v, int vr,
-                                                int nr)
-{
-    double2 P[DL - 1];
-#pragma unroll
-    for (int k = 0; k < DL - 1; ++k) P[k] = v[min(k, nr - 1) * vr];
-    double2 xm1 = make_double2(0.0, 0.0);
-    FwdOps<DL> B[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) fwd_load<DL>(B[b], f, fr, fj, v, vr, 2 * b, nr);
-    int r = 0;
-    for (; r + 2 * NB <= nr; r += 2 * NB) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            fwd_step<DL>(B[b].c[0], B[b].vn[0], P, xm1, v, vr, r + 2 * b);
-            fwd_step<DL>(B[b].c[1], B[b].vn[1], P, xm1, v, vr, r + 2 * b + 1);
-            fwd_load<DL>(B[b], f, fr, fj, v, vr, r + 2 * b + 2 * NB, nr);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    // fewer than 2 NB rows left: B[b] holds rows r + 2b, r + 2b + 1
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (r + 2 * b < nr) fwd_step<DL>(B[b].c[0], B[b].vn[0], P, xm1, v, vr, r + 2 * b);
-        if (r + 2 * b + 1 < nr) fwd_step<DL>(B[b].c[1], B[b].vn[1], P, xm1, v, vr, r + 2 * b + 1);
+        fwd_step<DL>(B.a, s, v + 4 * VR);
+        fwd_step<DL>(B.b, s, v + 5 * VR);
+        fwd_step<DL>(B.c, s, v + 6 * VR);
+        fwd_step<DL>(B.d, s, v + 7 * VR);
+        fl += 8 * FR * DL;
+        v += 8 * VR;
     }
 }
 
-// Real-valued forms of the sweeps: the real and imaginary parts of a
-// complex right-hand side are independent chains with the same factors, so
-// two lanes share a column (one part each) and every step issues half the
-// multiply-adds of the complex form.  v: one part of the vector (row r at
-// v[r*vr]); operands stream through NB buffers of two rows.
-template <int DL>
-struct FwdOpsR {
-    double c[2][DL];
-    double vn[2];
+template <int DL> struct BwdRow {
+    RowFactors<DL> u;
+    double d, v;
+};
+template <int DL, int FR, int VR> struct BwdRows {
+    BwdRow<DL> a, b, c, d;
+    __device__ __forceinline__ void load1(BwdRow<DL> &o, const double *bu, const double *bi, const double *v)
+    {
+        o.u.load(bu);
+        o.d = bi[0];
+        o.v = v[0];
+    }
+    __device__ __forceinline__ void load(const double *bu, const double *bi, const double *v)
+    {
+        load1(a, bu, bi, v);
+        load1(b, bu - FR * DL, bi - FR, v - VR);
+        load1(c, bu - 2 * FR * DL, bi - 2 * FR, v - 2 * VR);
+        load1(d, bu - 3 * FR * DL, bi - 3 * FR, v - 3 * VR);
+    }
+};
+
+// w0 .. w3: the solutions of the rows above, nearest first
+struct BwdState {
+    double w0, w1, w2, w3;
 };
 
 template <int DL>
-__device__ __forceinline__ void fwd_load_r(FwdOpsR<DL> &o, const double *f, int fr, int fj,
-                                           const double *v, int vr, int r, int nr)
+__device__ __forceinline__ void bwd_step(const BwdRow<DL> &o, BwdState &s, double *v)
 {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int k = 0; k < DL; ++k) o.c[i][k] = f[min(r + i + k, nr - 1) * fr + (DL - 1 - k) * fj];
-        o.vn[i] = v[min(r + i + DL - 1, nr - 1) * vr];
+    double x = __builtin_fma(-o.u.template get<0>(), s.w0, o.v);
+    x = __builtin_fma(-o.u.template get<1>(), s.w1, x);
+    if constexpr (DL == 4) {
+        x = __builtin_fma(-o.u.template get<2>(), s.w2, x);
+        x = __builtin_fma(-o.u.template get<3>(), s.w3, x);
+    }
+    x *= o.d;
+    s.w3 = s.w2;
+    s.w2 = s.w1;
+    s.w1 = s.w0;
+    s.w0 = x;
+    v[0] = x;
+}
+
+template <int DL, int FR, int VR>
+__device__ __forceinline__ void chain_backward(const double *bu, const double *bi, double *v, int nrp)
+{
+    BwdState s{0.0, 0.0, 0.0, 0.0};
+    bu += (nrp - 1) * FR * DL;
+    bi += (nrp - 1) * FR;
+    v += (nrp - 1) * VR;
+    BwdRows<DL, FR, VR> A, B;
+    A.load(bu, bi, v);
+    for (int r = nrp; r > 0; r -= 8) {
+        B.load(bu - 4 * FR * DL, bi - 4 * FR, v - 4 * VR);
+        __builtin_amdgcn_sched_barrier(0);
+        bwd_step<DL>(A.a, s, v);
+        bwd_step<DL>(A.b, s, v - VR);
+        bwd_step<DL>(A.c, s, v - 2 * VR);
+        bwd_step<DL>(A.d, s, v - 3 * VR);
+        if (r > 8) A.load(bu - 8 * FR * DL, bi - 8 * FR, v - 8 * VR);
+        __builtin_amdgcn_sched_barrier(0);
+        bwd_step<DL>(B.a, s, v - 4 * VR);
+        bwd_step<DL>(B.b, s, v - 5 * VR);
+        bwd_step<DL>(B.c, s, v - 6 * VR);
+        bwd_step<DL>(B.d, s, v - 7 * VR);
+        bu -= 8 * FR * DL;
+        bi -= 8 * FR;
+        v -= 8 * VR;
     }
 }
 
-template <int DL>
-__device__ __forceinline__ void fwd_step_r(const double *c, double vn, double *P, double &xm1,
-                                           double *v, int vr, int r)
-{
-    const double x = P[0] - c[0] * xm1;
-#pragma unroll
-    for (int k = 1; k < DL - 1; ++k) P[k - 1] = P[k] - c[k] * xm1;
-    P[DL - 2] = vn - c[DL - 1] * xm1;
-    v[r * vr] = x;
-    xm1 = x;
-}
-
-template <int DL, int NB>
-__device__ __forceinline__ void chain_forward_r(const double *f, int fr, int fj, double *v, int vr,
-                                                int nr)
-{
-    double P[DL - 1];
-#pragma unroll
-    for (int k = 0; k < DL - 1; ++k) P[k] = v[min(k, nr - 1) * vr];
-    double xm1 = 0.0;
-    FwdOpsR<DL> B[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) fwd_load_r<DL>(B[b], f, fr, fj, v, vr, 2 * b, nr);
-    int r = 0;
-    for (; r + 2 * NB <= nr; r += 2 * NB) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            fwd_step_r<DL>(B[b].c[0], B[b].vn[0], P, xm1, v, vr, r + 2 * b);
-            fwd_step_r<DL>(B[b].c[1], B[b].vn[1], P, xm1, v, vr, r + 2 * b + 1);
-            fwd_load_r<DL>(B[b], f, fr, fj, v, vr, r + 2 * b + 2 * NB, nr);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (r + 2 * b < nr) fwd_step_r<DL>(B[b].c[0], B[b].vn[0], P, xm1, v, vr, r + 2 * b);
-        if (r + 2 * b + 1 < nr) fwd_step_r<DL>(B[b].c[1], B[b].vn[1], P, xm1, v, vr, r + 2 * b + 1);
-    }
-}
-
-template <int DL>
-struct BwdOpsR {
-    double u[2][DL + 1];
-    double v[2];
-};
-
-template <int DL>
-__device__ __forceinline__ void bwd_load_r(BwdOpsR<DL> &o, const double *f, int fr, int fj,
-                                           const double *v, int vr, int r)
-{
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rr = max(r - i, 0);
-#pragma unroll
-        for (int k = 1; k <= DL; ++k) o.u[i][k - 1] = f[rr * fr + (DL + k) * fj];
-        o.u[i][DL] = f[rr * fr + DL * fj];
-        o.v[i] = v[rr * vr];
-    }
-}
-
-template <int DL>
-__device__ __forceinline__ void bwd_step_r(const double *u, double x, double *w, double *v, int vr,
-                                           int r)
-{
-#pragma unroll
-    for (int k = 1; k <= DL; ++k) x -= u[k - 1] * w[k - 1];
-    x *= u[DL];
-#pragma unroll
-    for (int m = DL - 1; m > 0; --m) w[m] = w[m - 1];
-    w[0] = x;
-    v[r * vr] = x;
-}
-
-// Rows of the factor image whose U parts arrive while the chain runs: chunk
-// c holds the rows [nr - (c+1) cr, nr - c cr) (last rows first); ready[c]
-// counts the waves that have stored their share of it.
-struct StagedRows {
-    const int *ready;
-    int cr, nchunk, nwriters;
-    int *err;          // device error word (SC_KERR_* bits)
-};
-
-// Polls of one chunk's counter before the wait gives up: each poll sleeps
-// 64 clocks, so the limit is ~30 ms, against waits of a few microseconds.
-constexpr int SOLVE_SPIN_LIMIT = 1 << 20;
-
-// wait until the U parts of rows >= row are in LDS (chunks in order).  A
-// counter that never reaches the writer count (a staging wave that did not
-// signal) sets SC_KERR_SOLVE_WAIT in the error word and ends the wait, so
-// the kernel still exits; the host reports the error after the run.
-__device__ __forceinline__ void wait_rows(const StagedRows &sr, int row, int &low, int &next)
-{
-    while (row < low && next < sr.nchunk) {
-        int spins = 0;
-        while (__hip_atomic_load(&sr.ready[next], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
-               sr.nwriters) {
-            if (++spins > SOLVE_SPIN_LIMIT) {
-                __hip_atomic_fetch_or(sr.err, SC_KERR_SOLVE_WAIT, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-                next = sr.nchunk;
-                low = 0;
-                return;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        ++next;
-        low = max(low - sr.cr, 0);
-    }
-}
-
-// real-valued backward sweep with NB operand buffers, the operand stream
-// waiting for staged rows
-template <int DL, int NB>
-__device__ __forceinline__ void chain_backward_staged(const double *f, int fr, int fj, double *v,
-                                                      int vr, int nr, const StagedRows &sr)
-{
-    int low = nr, next = 0;
-    double w[DL];
-#pragma unroll
-    for (int m = 0; m < DL; ++m) w[m] = 0.0;
-    BwdOpsR<DL> B[NB];
-    wait_rows(sr, max(nr - 2 * NB, 0), low, next);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) bwd_load_r<DL>(B[b], f, fr, fj, v, vr, nr - 1 - 2 * b);
-    int r = nr - 1;
-    // B[b] holds rows r - 2b, r - 2b - 1
-    for (; r >= 2 * NB - 1; r -= 2 * NB) {
-        wait_rows(sr, max(r - 4 * NB + 1, 0), low, next);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            bwd_step_r<DL>(B[b].u[0], B[b].v[0], w, v, vr, r - 2 * b);
-            bwd_step_r<DL>(B[b].u[1], B[b].v[1], w, v, vr, r - 2 * b - 1);
-            bwd_load_r<DL>(B[b], f, fr, fj, v, vr, r - 2 * b - 2 * NB);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (r - 2 * b >= 0) bwd_step_r<DL>(B[b].u[0], B[b].v[0], w, v, vr, r - 2 * b);
-        if (r - 2 * b - 1 >= 0) bwd_step_r<DL>(B[b].u[1], B[b].v[1], w, v, vr, r - 2 * b - 1);
-    }
-}
+// 16 bytes of an image (a plain vector: arrays of double2 copied whole stay in
+// scratch memory)
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 struct ColumnOf {
     int z, x;
@@ -1945,513 +1791,400 @@ __device__ __forceinline__ ColumnOf column_of(const SolveArgs &a, int col)
     return c;
 }
 
-// rows of one thread in a block of SOLVE_THREADS: r = tid / SBT + t * (SOLVE_THREADS / SBT),
-// t < VR (a chain has at most VR * SOLVE_THREADS / SBT rows)
-constexpr int SOLVE_THREADS = 256;
+constexpr int SOLVE_THREADS = 256, SOLVE_WORKERS = 192;
 constexpr int SOLVE_VR_MAX = 4;
-// factor values in flight per thread and batch (16-byte loads)
-constexpr int SOLVE_FBAT = 8;
+// zero rows before a vector (the operator's reach) and after it (that, and the
+// forward sweep's read ahead)
+constexpr int SOLVE_LEAD = 4, SOLVE_TAIL = 12;
+
+// The wave that runs the chains: the one whose SIMD equals the block's workgroup
+// slot on the CU (mod 4), so that the blocks resident on one CU run their chains
+// on different SIMDs (wave 0 when no wave matches).
+__device__ __forceinline__ int pick_chain_wave()
+{
+    __shared__ int chain_wave[1];
+    if (threadIdx.x == 0) chain_wave[0] = 0;
+    __syncthreads();
+    // HW_ID: SIMD in bits 5:4, workgroup slot in bits 19:16
+    const unsigned hw = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (31 << 11));
+    if ((threadIdx.x & 63) == 0 && ((hw >> 4) & 3) == ((hw >> 16) & 3)) chain_wave[0] = threadIdx.x >> 6;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(chain_wave[0]);
+}
 
 // One (field, parity) of SBT consecutive columns, for the members m0 ..
-// m0 + nmb - 1 (nmb <= MB), which all solve with the same operator.  The
-// factors of the block are one contiguous image [nr][W][SBT] (laid out so at
-// init) copied to LDS once with 16-byte loads and shared by the members;
-// every thread owns the column tid % SBT, so its rows are tid / SBT + t *
-// (SOLVE_THREADS / SBT).  lds: [nr][W][SBT] factors, then [MB][nr][SBT]
-// right-hand sides, then [MB][nr][SBT] stage-0 copies of C.  The chain wave
-// runs 2 SBT lanes per member (real and imaginary part of each column): with
-// several members one staged image feeds up to 64 chains at once.
+// m0 + nmb - 1 (nmb <= MB).  lds: the factor image (L, then U and the inverse
+// pivots), then per member SOLVE_LEAD + nrp + SOLVE_TAIL vector rows of SBT
+// complex values.  Worker w owns column w % SBT and the rows w / SBT + t RSTEP,
+// t < VR.
 template <int DL, int SBT, int VR, int MB>
-__device__ void solve_block(const SolveArgs &a, int var, int par, int blk, int m0, int nmb,
-                            cplx *C, cplx *Cs, double *lds)
+__device__ __forceinline__ void solve_block(const SolveArgs &a, int var, int par, int blk, int m0, int nmb,
+                            int stop, cplx *C, cplx *Cs, double *lds)
 {
-    constexpr int W = 2 * DL + 1;
-    constexpr int RSTEP = SOLVE_THREADS / SBT;
+    constexpr int RSTEP = SOLVE_WORKERS / SBT, NE = 2 * DL + 1;
     static_assert(2 * SBT * MB <= 64, "one chain lane per member, part and column");
     const int Mx = a.Mx, nR = a.dimR, nQ = a.dimQ;
     const int N = var == 0 ? nQ : nR;
-    const int nr = (N - par + 1) / 2, nrmax = (N + 1) / 2;
+    const int nr = (N - par + 1) / 2, nrp = solve_rows(N);
     const int tid = threadIdx.x;
-    double *lf = lds;
-    double2 *vec = (double2 *) (lds + (size_t) nr * W * SBT);
-    double2 *raw = vec + MB * nr * SBT;
-    const double ce0 = a.ce0[var], cn = a.cn[var];
-    // the members' arrays (member m0 + mb; uniform across the block)
-    auto Cm = [&](int mb) { return C + (size_t) (m0 + mb) * a.ms_c; };
-    auto Csm = [&](int mb) { return Cs + (size_t) (m0 + mb) * a.ms_cs; };
-    auto Fm = [&](int mb) {
-        return var == 0 ? a.Fa + (size_t) (m0 + mb) * a.ms_fa : a.Fb + (size_t) (m0 + mb) * a.ms_fb;
-    };
-    auto F2m = [&](int mb) {
-        return var == 0 ? a.Fa2 + (size_t) (m0 + mb) * a.ms_fa2 : a.Fb2 + (size_t) (m0 + mb) * a.ms_fb2;
-    };
-    auto Sm = [&](int mb) { return a.Src + (size_t) (m0 + mb) * a.ms_src; };
-
-    constexpr int NCHU = 4;                 // chunks of rows whose U parts stream in
-    __shared__ int chain_wave[1];
-    __shared__ int ready[NCHU];
-    if (tid == 0) chain_wave[0] = 0;
-    if (tid < NCHU) ready[tid] = 0;
-    __syncthreads();
-    {
-        // HW_ID: SIMD in bits 5:4, workgroup slot in bits 19:16
-        const unsigned hw = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (31 << 11));
-        if ((tid & 63) == 0 && ((hw >> 4) & 3) == ((hw >> 16) & 3)) chain_wave[0] = tid >> 6;
-    }
-    const int cc = tid % SBT, rt = tid / SBT;
-    const ColumnOf co = column_of(a, blk * SBT + cc);
-    const double kx = a.Kx[co.x], kz = a.Kz[co.z], k2 = kz * kz + kx * kx;
-    const size_t cbase = (((size_t) co.z * 2 + var) * nR + par) * Mx + co.x;   // C row par
-    const size_t fbase = ((size_t) co.z * N + par) * Mx + co.x;                 // F row par
-    const size_t rs = (size_t) 2 * Mx;                                          // next chain row
-
-    // right-hand side rows: member 0's loads first (before the factor copy);
-    // the other members' after it, one member at a time
-    double2 cv[VR], fv[VR], sv[VR];
-    auto load_rows = [&](int mb) {
-#pragma unroll
-        for (int t = 0; t < VR; ++t) {
-            const int r = min(rt + t * RSTEP, nr - 1);
-            cv[t] = Cm(mb)[cbase + r * rs];
-            fv[t] = Fm(mb)[fbase + r * rs];
-            sv[t] = a.Src ? Sm(mb)[cbase + r * rs] : make_double2(0.0, 0.0);
-        }
-    };
-    auto store_rows = [&](int mb) {
-#pragma unroll
-        for (int t = 0; t < VR; ++t) {
-            const int r = rt + t * RSTEP;
-            if (r >= nr || !co.chain) continue;
-            if (a.k == 0) {
-                raw[(mb * nr + r) * SBT + cc] = cv[t];
-            } else {
-                double2 v = cv[t];
-                v.x += a.dtc * fv[t].x;
-                v.y += a.dtc * fv[t].y;
-                v.x += sv[t].x;
-                v.y += sv[t].y;
-                vec[(mb * nr + r) * SBT + cc] = v;
-            }
-        }
-    };
-    load_rows(0);
-    // The factor image ([row][W][SBT], 16-byte loads): the L parts (columns
-    // j < DL) of every row before the barrier, for the forward sweep; the U
-    // parts (j >= DL) after it, last rows first in NCHU chunks, each wave
-    // signalling a chunk once its share is in LDS, so that the backward
-    // sweep starts while the upper rows still stream in.
-    constexpr int RPR = W * SBT / 2, LPR = DL * SBT / 2, UPR = RPR - LPR;
+    const int vrows = SOLVE_LEAD + nrp + SOLVE_TAIL;
+    double *fl = lds, *bu = fl + nrp * DL * SBT, *bi = bu + nrp * DL * SBT;
+    double2 *vec = (double2 *) (bi + nrp * SBT) + SOLVE_LEAD * SBT;     // row 0 of member 0
+    const int vm = vrows * SBT;                                          // member stride
+    // the factor image: mirror rows kz <-> Nz - kz share one
     int fb = blk;
     if (a.mirror) {
-        // factor image of the mirror row Nz - z for z > Nz/2
         const int z = blk * SBT / Mx;
         if (z > a.Nz / 2) fb = blk - (2 * z - a.Nz) * (Mx / SBT);
     }
-    const double2 *src = (const double2 *) (var == 0 ? a.La : a.Lb) +
-                         ((size_t) fb * 2 + par) * nrmax * RPR;
-    double2 *dst = (double2 *) lf;
-    {
-        const int nl = nr * LPR;
-        for (int b0 = 0; b0 < nl; b0 += SOLVE_FBAT * SOLVE_THREADS) {
-            double2 t[SOLVE_FBAT];
-            int o[SOLVE_FBAT];
+
+    // L factors: every thread, in flight while the chain wave is chosen (LB and
+    // UB 16-byte loads a thread cover the rows that VR slots hold)
+    constexpr int LB = DL == 4 ? (3 * VR + 1) / 2 : VR, UB = DL == 4 ? (5 * VR + 1) / 2 : (3 * VR + 1) / 2;
+    const v2d *src = (const v2d *) (var == 0 ? a.La : a.Lb) + ((size_t) fb * 2 + par) * (nrp * NE * SBT / 2);
+    const int nl = nrp * DL * SBT / 2, nu = nrp * (DL + 1) * SBT / 2;
+    v2d lt[LB], ut[UB];
 #pragma unroll
-            for (int i = 0; i < SOLVE_FBAT; ++i) {
-                const int e = min(b0 + tid + i * SOLVE_THREADS, nl - 1), r = e / LPR;
-                o[i] = r * RPR + (e - r * LPR);
-                t[i] = src[o[i]];
-            }
+    for (int i = 0; i < LB; ++i) lt[i] = src[min(tid + i * SOLVE_THREADS, nl - 1)];
+    const int cw = pick_chain_wave();
+    if (stop) return;                                    // (its load is under the others')
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto store_L = [&]() {
 #pragma unroll
-            for (int i = 0; i < SOLVE_FBAT; ++i)
-                if (b0 + tid + i * SOLVE_THREADS < nl) dst[o[i]] = t[i];
-        }
-    }
-    store_rows(0);
-    // member 0's forcing rows kept for the stage-0 operator (with one member
-    // they stay where they are)
-    constexpr int KV = MB > 1 ? VR : 1;
-    double2 fv0[KV], sv0[KV];
-    if constexpr (MB > 1) {
-#pragma unroll
-        for (int t = 0; t < VR; ++t) {
-            fv0[t] = fv[t];
-            sv0[t] = sv[t];
-        }
-    }
-    for (int mb = 1; mb < nmb; ++mb) {
-        load_rows(mb);
-        store_rows(mb);
-    }
-    __syncthreads();
-    if (a.k == 0) {
-        // E C + dt c_0 F with the stage-0 explicit operator
-        if constexpr (MB <= 2) {
-            // each band entry formed once for the block's members; their
-            // forcing rows are still in registers (member 0's in fv0/sv0
-            // when MB > 1, the last member's in fv/sv)
-#pragma unroll
-            for (int t = 0; t < VR; ++t) {
-                const int r = rt + t * RSTEP, i = par + 2 * r;
-                if (r >= nr || !co.chain) continue;
-                double2 acc[MB];
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[mb] = make_double2(0.0, 0.0);
-#pragma unroll
-                for (int m = -DL; m <= DL; ++m)
-                    if (r + m >= 0 && r + m < nr) {
-                        const double ev = op_entry(a, var, i, m, k2, ce0);
-#pragma unroll
-                        for (int mb = 0; mb < MB; ++mb)
-                            if (mb < nmb) {
-                                const double2 y = raw[(mb * nr + r + m) * SBT + cc];
-                                acc[mb].x += ev * y.x;
-                                acc[mb].y += ev * y.y;
-                            }
-                    }
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) {
-                    if (mb >= nmb) continue;
-                    double2 f = fv[t], sf = sv[t];
-                    if constexpr (MB > 1) {
-                        if (mb == 0) {
-                            f = fv0[t];
-                            sf = sv0[t];
-                        }
-                    }
-                    acc[mb].x += a.dtc * f.x;
-                    acc[mb].y += a.dtc * f.y;
-                    acc[mb].x += sf.x;
-                    acc[mb].y += sf.y;
-                    vec[(mb * nr + r) * SBT + cc] = acc[mb];
-                }
-            }
-        } else {
-            // member 0's forcing rows still in registers, the others'
-            // loaded again (one member's at a time)
-            for (int mb = 0; mb < nmb; ++mb) {
-                if (mb > 0) load_rows(mb);
-#pragma unroll
-                for (int t = 0; t < VR; ++t) {
-                    const int r = rt + t * RSTEP, i = par + 2 * r;
-                    if (r >= nr || !co.chain) continue;
-                    double2 f = fv[t], sf = sv[t];
-                    if (mb == 0) {
-                        f = fv0[t];
-                        sf = sv0[t];
-                    }
-                    const double2 *rm = raw + mb * nr * SBT;
-                    double2 acc = make_double2(0.0, 0.0);
-#pragma unroll
-                    for (int m = -DL; m <= DL; ++m)
-                        if (r + m >= 0 && r + m < nr) {
-                            double ev = op_entry(a, var, i, m, k2, ce0);
-                            double2 y = rm[(r + m) * SBT + cc];
-                            acc.x += ev * y.x;
-                            acc.y += ev * y.y;
-                        }
-                    acc.x += a.dtc * f.x;
-                    acc.y += a.dtc * f.y;
-                    acc.x += sf.x;
-                    acc.y += sf.y;
-                    vec[(mb * nr + r) * SBT + cc] = acc;
-                }
-            }
+        for (int i = 0; i < LB; ++i)
+            if (tid + i * SOLVE_THREADS < nl) ((v2d *) fl)[tid + i * SOLVE_THREADS] = lt[i];
+        for (int e = tid + LB * SOLVE_THREADS; e < nl; e += SOLVE_THREADS) ((v2d *) fl)[e] = src[e];
+    };
+    // The chain wave and the workers take separate paths with the same barriers
+    // (each is uniform in its waves), so that neither holds the other's values in
+    // registers.
+    if (wave == cw) {
+        store_L();
+        // lane cl < 2 SBT nmb: member cl / (2 SBT), part (cl / SBT) % 2 (real,
+        // imaginary) of column cl % SBT
+        const int cl = tid & 63, mb = cl / (2 * SBT), col = cl % SBT;
+        double *vd = (double *) (vec + mb * vm) + 2 * col + ((cl / SBT) & 1);
+        if (a.k == 0) {
+            __syncthreads();
+            __syncthreads();
         }
         __syncthreads();
+        if (mb < nmb) chain_forward<DL, SBT, 2 * SBT>(fl + col * DL, vd, nrp);
+        __syncthreads();
+        if (mb < nmb) chain_backward<DL, SBT, 2 * SBT>(bu + col * DL, bi + col, vd, nrp);
+        __syncthreads();
+        return;
     }
-    // The chains run in one wave of the block: the wave whose SIMD equals the
-    // block's workgroup slot on the CU (mod 4), so that the blocks resident on
-    // one CU run their chains on different SIMDs (wave 0 when no wave matches).
-    // The other waves stage the U parts meanwhile, chunk by chunk, and signal.
-    const int cl = tid & 63, cw = chain_wave[0];
-    const int cr = (nr + NCHU - 1) / NCHU;
-    // Every wave but the chain wave stages: each signals every chunk exactly
-    // once (both staging paths below), so a chunk is complete at NWR signals.
-    constexpr int NWR = SOLVE_THREADS / 64 - 1;          // staging waves
-    static_assert(NWR >= 1 && SOLVE_THREADS % 64 == 0, "one chain wave, the rest stage");
-    const StagedRows sr{ready, cr, NCHU, NWR, a.err};
-    if ((tid >> 6) == cw) {
-        // lane cl < 2 SBT nmb: member cl / (2 SBT), part (cl / SBT) % 2
-        // (real, imaginary) of column cl % SBT
-        if (cl < 2 * SBT * nmb && co.chain && nr > 0) {
-            const int mb = cl / (2 * SBT), col = cl % SBT, part = (cl / SBT) & 1;
-            double *vd = (double *) (vec + mb * nr * SBT) + 2 * col + part;
-            chain_forward_r<DL, 3>(lf + col, W * SBT, SBT, vd, 2 * SBT, nr);
-            chain_backward_staged<DL, 3>(lf + col, W * SBT, SBT, vd, 2 * SBT, nr, sr);
+    const int wt = tid - (wave > cw ? 64 : 0);
+    const int cc = wt % SBT, rt = wt / SBT;
+    const ColumnOf co = column_of(a, blk * SBT + cc);
+    const double kx = a.Kx[co.x], kz = a.Kz[co.z], k2 = __builtin_fma(kz, kz, kx * kx);
+    const size_t cbase = (((size_t) co.z * 2 + var) * nR + par) * Mx + co.x;   // C row par
+    const size_t fbase = ((size_t) co.z * N + par) * Mx + co.x;                 // F row par
+    const size_t rs = (size_t) 2 * Mx;                                          // next chain row
+    // the members' arrays (member m0 + mb; the last one again past the group)
+    auto of = [&](int mb) { return (size_t) (m0 + min(mb, nmb - 1)); };
+    auto Cm = [&](int mb) { return C + of(mb) * a.ms_c; };
+    auto Csm = [&](int mb) { return Cs + of(mb) * a.ms_cs; };
+    auto Fm = [&](int mb) { return var == 0 ? a.Fa + of(mb) * a.ms_fa : a.Fb + of(mb) * a.ms_fb; };
+    auto F2m = [&](int mb) { return var == 0 ? a.Fa2 + of(mb) * a.ms_fa2 : a.Fb2 + of(mb) * a.ms_fb2; };
+
+    double2 cv[MB][VR], fv[MB][VR];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int t = 0; t < VR; ++t) {
+            const int r = max(min(rt + t * RSTEP, nr - 1), 0);
+            cv[mb][t] = Cm(mb)[cbase + r * rs];
+            fv[mb][t] = Fm(mb)[fbase + r * rs];
         }
-    } else {
-        // element e of the U parts counts from the last row up (row
-        // nr - 1 - e / UPR); chunk c holds e in [c cr UPR, (c+1) cr UPR).
-        // The staging waves' threads wt take e = c cr UPR + wt + j NT of
-        // every chunk, all loads issued before the first store (chains of
-        // up to 48 rows; longer ones copy directly).
-        constexpr int NT = NWR * 64;
-        constexpr int CRMAX = (48 + NCHU - 1) / NCHU;
-        static_assert(CRMAX * UPR <= 2 * NT, "two elements per thread and chunk");
-        const int wt = tid - ((tid >> 6) > cw ? 64 : 0);
-        const int nu = nr * UPR, ce = cr * UPR;
-        const bool regs = cr <= CRMAX;
-        // a chunk's two elements per thread in named registers (arrays of
-        // them stay in scratch memory next to the signalling atomic); the
-        // loads of chunk c+1 are issued before the stores of chunk c
-        struct UC {
-            double2 v0, v1;
-            int o0, o1;
-            bool s0, s1;
-        };
-        auto ld = [&](int c) {
-            UC u;
-            const int e0 = c * ce, e1 = min(e0 + ce, nu);
-            const int ea = e0 + wt, eb = ea + NT;
-            u.s0 = ea < e1;
-            u.s1 = eb < e1;
-            const int ca = max(min(ea, e1 - 1), 0), cb = max(min(eb, e1 - 1), 0);
-            const int ra = ca / UPR, rb = cb / UPR;
-            // (no rows at all: read the image's first element, store nothing)
-            u.o0 = max((nr - 1 - ra) * RPR + LPR + (ca - ra * UPR), 0);
-            u.o1 = max((nr - 1 - rb) * RPR + LPR + (cb - rb * UPR), 0);
-            u.v0 = src[u.o0];
-            u.v1 = src[u.o1];
-            return u;
-        };
-        auto st = [&](const UC &u, int c) {
-            if (u.s0) dst[u.o0] = u.v0;
-            if (u.s1) dst[u.o1] = u.v1;
-            if (cl == 0) __hip_atomic_fetch_add(&ready[c], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        };
-        if (regs) {
-            static_assert(NCHU == 4, "four chunks below");
-            UC a0 = ld(0), a1 = ld(1);
-            st(a0, 0);
-            a0 = ld(2);
-            st(a1, 1);
-            a1 = ld(3);
-            st(a0, 2);
-            st(a1, 3);
-        } else {
-            for (int c = 0; c < NCHU; ++c) {
-                const int e0 = c * ce, e1 = min(e0 + ce, nu);
-                for (int e = e0 + wt; e < e1; e += NT) {
-                    const int rb = e / UPR, o = (nr - 1 - rb) * RPR + LPR + (e - rb * UPR);
-                    dst[o] = src[o];
+    // U factors and pivots, stored after the barrier
+#pragma unroll
+    for (int i = 0; i < UB; ++i) ut[i] = src[nl + min(wt + i * SOLVE_WORKERS, nu - 1)];
+    store_L();
+    // right-hand sides (at stage 0 the state itself first, for the explicit
+    // operator), zero outside the chain and its column set
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        if (mb >= nmb) break;
+        double2 *vv = vec + mb * vm + cc;
+#pragma unroll
+        for (int t = 0; t < VR; ++t) {
+            const int r = rt + t * RSTEP;
+            if (r >= nr) continue;
+            double2 v = cv[mb][t];
+            if (a.k != 0) {
+                v.x = __builtin_fma(a.dtc, fv[mb][t].x, v.x);
+                v.y = __builtin_fma(a.dtc, fv[mb][t].y, v.y);
+                if (a.Src) {
+                    const double2 s = a.Src[of(mb) * a.ms_src + cbase + r * rs];
+                    v.x += s.x;
+                    v.y += s.y;
                 }
-                if (cl == 0) __hip_atomic_fetch_add(&ready[c], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
+            vv[r * SBT] = co.chain ? v : make_double2(0.0, 0.0);
+        }
+        const int npad = vrows - nr;
+        for (int p = rt; p < npad; p += RSTEP)
+            vv[(p < SOLVE_LEAD ? p - SOLVE_LEAD : nr + p - SOLVE_LEAD) * SBT] = make_double2(0.0, 0.0);
+    }
+    if (a.k == 0) {
+        // E C + dt c_0 F with the stage-0 explicit operator, its entries formed
+        // once for the members
+        __syncthreads();
+        double2 acc[MB][VR];
+#pragma unroll
+        for (int t = 0; t < VR; ++t) {
+            const int r = max(min(rt + t * RSTEP, nr - 1), 0);
+            double e[NE] = {};
+            if (nr > 0) op_row<DL>(a, par + 2 * r, k2, a.ce0[var], e);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                const double2 *vv = vec + min(mb, nmb - 1) * vm + r * SBT + cc;
+                double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+                for (int m = -DL; m <= DL; ++m) {
+                    const double2 y = vv[m * SBT];
+                    s.x = __builtin_fma(e[DL + m], y.x, s.x);
+                    s.y = __builtin_fma(e[DL + m], y.y, s.y);
+                }
+                s.x = __builtin_fma(a.dtc, fv[mb][t].x, s.x);
+                s.y = __builtin_fma(a.dtc, fv[mb][t].y, s.y);
+                if (a.Src) {
+                    const double2 q = a.Src[of(mb) * a.ms_src + cbase + r * rs];
+                    s.x += q.x;
+                    s.y += q.y;
+                }
+                acc[mb][t] = s;
+            }
+            __builtin_amdgcn_sched_barrier(0);       // one row's bands at a time
+        }
+        __syncthreads();
+        if (co.chain) {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int t = 0; t < VR; ++t)
+                    if (mb < nmb && rt + t * RSTEP < nr) vec[mb * vm + (rt + t * RSTEP) * SBT + cc] = acc[mb][t];
         }
     }
     __syncthreads();
-    // write the solutions and the next stage's right-hand sides
-    if constexpr (MB <= 2) {
-        // each band entry of the next stage's operator formed once for the
-        // block's members
+    double2 f2[MB][VR];
+    double en[VR][NE];
+    v2d *dst = (v2d *) bu;
+#pragma unroll
+    for (int i = 0; i < UB; ++i)
+        if (wt + i * SOLVE_WORKERS < nu) dst[wt + i * SOLVE_WORKERS] = ut[i];
+    for (int e = wt + UB * SOLVE_WORKERS; e < nu; e += SOLVE_WORKERS) dst[e] = src[nl + e];
+    if (a.has_next && nr > 0) {
 #pragma unroll
         for (int t = 0; t < VR; ++t) {
-            const int r = rt + t * RSTEP, i = par + 2 * r;
-            if (r >= nr || !co.chain) continue;
+            const int r = max(min(rt + t * RSTEP, nr - 1), 0);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) f2[mb][t] = F2m(mb)[fbase + r * rs];
+            op_row<DL>(a, par + 2 * r, k2, a.cn[var], en[t]);
+            __builtin_amdgcn_sched_barrier(0);       // one row's bands at a time
+        }
+    }
+    __syncthreads();
+    __syncthreads();
+    // the solutions and the next stage's right-hand sides
+    if (co.chain) {
+#pragma unroll
+        for (int t = 0; t < VR; ++t) {
+            const int r = rt + t * RSTEP;
+            if (r >= nr) continue;
             const size_t gi = cbase + r * rs;
-            double2 f2[MB], acc[MB];
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) {
-                acc[mb] = make_double2(0.0, 0.0);
-                if (mb < nmb && a.has_next) f2[mb] = F2m(mb)[fbase + r * rs];
-            }
-            if (a.has_next) {
-#pragma unroll
-                for (int m = -DL; m <= DL; ++m)
-                    if (r + m >= 0 && r + m < nr) {
-                        const double ev = op_entry(a, var, i, m, k2, cn);
-#pragma unroll
-                        for (int mb = 0; mb < MB; ++mb)
-                            if (mb < nmb) {
-                                const double2 y = vec[(mb * nr + r + m) * SBT + cc];
-                                acc[mb].x += ev * y.x;
-                                acc[mb].y += ev * y.y;
-                            }
-                    }
-            }
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
                 if (mb >= nmb) continue;
-                const double2 sol = vec[(mb * nr + r) * SBT + cc];
+                const double2 *vv = vec + mb * vm + r * SBT + cc;
+                const double2 sol = vv[0];
                 Csm(mb)[gi] = sol;
+                double2 s = sol;
                 if (a.has_next) {
-                    acc[mb].x += a.dtd * f2[mb].x;
-                    acc[mb].y += a.dtd * f2[mb].y;
-                    Cm(mb)[gi] = acc[mb];
-                } else {
-                    Cm(mb)[gi] = sol;
+                    s = make_double2(0.0, 0.0);
+#pragma unroll
+                    for (int m = -DL; m <= DL; ++m) {
+                        const double2 y = vv[m * SBT];
+                        s.x = __builtin_fma(en[t][DL + m], y.x, s.x);
+                        s.y = __builtin_fma(en[t][DL + m], y.y, s.y);
+                    }
+                    s.x = __builtin_fma(a.dtd, f2[mb][t].x, s.x);
+                    s.y = __builtin_fma(a.dtd, f2[mb][t].y, s.y);
                 }
+                Cm(mb)[gi] = s;
             }
         }
-    } else {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int t = 0; t < VR; ++t) {
-                const int r = rt + t * RSTEP, i = par + 2 * r;
-                if (mb >= nmb || r >= nr || !co.chain) continue;
-                const double2 *vm = vec + mb * nr * SBT;
-                const size_t gi = cbase + r * rs;
-                const double2 sol = vm[r * SBT + cc];
-                Csm(mb)[gi] = sol;
-                if (a.has_next) {
-                    const double2 f2 = F2m(mb)[fbase + r * rs];
-                    double2 acc = make_double2(0.0, 0.0);
-#pragma unroll
-                    for (int m = -DL; m <= DL; ++m)
-                        if (r + m >= 0 && r + m < nr) {
-                            double ev = op_entry(a, var, i, m, k2, cn);
-                            double2 y = vm[(r + m) * SBT + cc];
-                            acc.x += ev * y.x;
-                            acc.y += ev * y.y;
-                        }
-                    acc.x += a.dtd * f2.x;
-                    acc.y += a.dtd * f2.y;
-                    Cm(mb)[gi] = acc;
-                } else {
-                    Cm(mb)[gi] = sol;
-                }
-            }
     }
     // rows of v beyond dimQ are carried unchanged; the Nyquist row is zeroed
     const int nrest = (nR - par + 1) / 2;
     if (!co.valid || (co.z == 0 && co.x == 0)) return;
     for (int mb = 0; mb < nmb; ++mb)
         for (int r = rt; r < nrest; r += RSTEP) {
-            const int i = par + 2 * r;
             const size_t gi = cbase + r * rs;
             if (co.z == a.Nz / 2)
                 Cm(mb)[gi] = make_double2(0.0, 0.0);
-            else if (var == 0 && i >= nQ)
+            else if (var == 0 && par + 2 * r >= nQ)
                 Csm(mb)[gi] = Cm(mb)[gi];
         }
 }
 
-// explicit mean operator Rs + coef Rps applied to v (row i)
-__device__ double2 mean_mult(const SolveArgs &a, const double2 *v, int i, double coef)
+// Sum of red[0 .. 255] by halving (128, 64, ..., 1), the same order in every
+// call; every thread gets it.
+__device__ __forceinline__ double halving_sum(double v, double *red)
 {
-    const int N = a.dimR;
-    double2 t = make_double2(0.0, 0.0);
-    int m0 = -min(2, i / 2), m1 = min(2, (N - i + 1) / 2 - 1);
-    for (int m = m0; m <= m1; ++m) {
-        double c = op_entry(a, 1, i, m, 0.0, coef);
-        t.x += c * v[i + 2 * m].x;
-        t.y += c * v[i + 2 * m].y;
+    const int tid = threadIdx.x;
+    __syncthreads();
+    red[tid] = v;
+    __syncthreads();
+    if (tid < 64) {
+        double s = (red[tid] + red[tid + 128]) + (red[tid + 64] + red[tid + 192]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
+        if (tid == 0) red[0] = s;
     }
-    return t;
+    __syncthreads();
+    return red[0];
 }
 
-// the mean mode: alpha (streamwise mean) and beta (spanwise mean) columns.
-// Every global load (state, both forcings, factors) is issued up front; the
-// two explicit products of a pass run together.  Rows per thread:
-// i = tid + MEAN_ROWS_STEP t, t < MEAN_ROWS (dimR <= 512).
+// The mean mode of the members m0 .. m0 + nmb - 1: alpha (streamwise mean) and
+// beta (spanwise mean) columns as the two columns of one chain image.  lds: the
+// image ([parity]: L, U, inverse pivots), then per member and parity the padded
+// rows of (alpha, beta), then 256 partial sums.  Rows per thread:
+// i = tid + 256 t, t < MEAN_ROWS (dimR <= 512).
 constexpr int MEAN_ROWS = 2;
-__device__ void solve_mean(const SolveArgs &a, cplx *C, cplx *Cs, double *lds)
+__device__ __forceinline__ void solve_mean(const SolveArgs &a, int m0, int nmb, cplx *C, cplx *Cs, double *lds)
 {
-    const int nR = a.dimR, Mx = a.Mx, T = SOLVE_THREADS, tid = threadIdx.x;
-    double2 *al = (double2 *) lds, *be = al + nR, *ta = be + nR, *tb = ta + nR;
-    double *lm = (double *) (tb + nR), *red = lm + 5 * nR;
-    cplx *Ca = C, *Cb = C + (size_t) nR * Mx;
-    const cplx *Fm = a.Fb, *Fm2 = a.Fb2;   // column (0, 0): (fa, fb)
-    double2 fr[MEAN_ROWS], f2r[MEAN_ROWS];
+    constexpr int T = SOLVE_THREADS;
+    const int nR = a.dimR, Mx = a.Mx, tid = threadIdx.x;
+    const int nrp = solve_rows(nR), img = nrp * 5, vrows = SOLVE_LEAD + nrp + SOLVE_TAIL;
+    double2 *vec = (double2 *) (lds + 2 * img);
+    const int pv = vrows * 2, mv = 2 * pv;                 // parity and member strides
+    double *red = (double *) (vec + nmb * mv);
+    // row i of member mb: (alpha, beta)
+    auto row = [&](int mb, int i) { return vec + mb * mv + (i & 1) * pv + (SOLVE_LEAD + (i >> 1)) * 2; };
+    for (int e = tid; e < 2 * img; e += T) lds[e] = a.Lm[e];
+    for (int e = tid; e < nmb * mv; e += T) vec[e] = make_double2(0.0, 0.0);
+    __syncthreads();
+    // Rs + coef Rps of the rows' two columns
+    auto mult = [&](int mb, int i, double coef, double2 &al, double2 &be) {
+        double e[5];
+        const double *rs = a.Rs + i * 5, *rp = a.Rps + i * 5;
 #pragma unroll
-    for (int t = 0; t < MEAN_ROWS; ++t) {
-        const int i = tid + T * t;
-        if (i < nR) {
-            al[i] = Ca[(size_t) i * Mx];
-            be[i] = Cb[(size_t) i * Mx];
+        for (int j = 0; j < 5; ++j) e[j] = __builtin_fma(coef, rp[j], rs[j]);
+        const double2 *v = row(mb, i);
+        al = be = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int m = -2; m <= 2; ++m) {
+            const double2 x = v[2 * m], y = v[2 * m + 1];
+            al.x = __builtin_fma(e[m + 2], x.x, al.x);
+            al.y = __builtin_fma(e[m + 2], x.y, al.y);
+            be.x = __builtin_fma(e[m + 2], y.x, be.x);
+            be.y = __builtin_fma(e[m + 2], y.y, be.y);
+        }
+    };
+    for (int mb = 0; mb < nmb; ++mb) {
+        const size_t m = m0 + mb;
+        const cplx *Ca = C + m * a.ms_c, *Cb = Ca + (size_t) nR * Mx;
+        const cplx *Fm = a.Fb + m * a.ms_fb, *Sm = a.Src ? a.Src + m * a.ms_src : nullptr;
+        double2 fr[MEAN_ROWS], al[MEAN_ROWS], be[MEAN_ROWS];
+#pragma unroll
+        for (int t = 0; t < MEAN_ROWS; ++t) {
+            const int i = tid + T * t;
+            if (i >= nR) continue;
+            al[t] = Ca[(size_t) i * Mx];
+            be[t] = Cb[(size_t) i * Mx];
             fr[t] = Fm[(size_t) i * Mx];
-            f2r[t] = a.has_next ? Fm2[(size_t) i * Mx] : make_double2(0.0, 0.0);
         }
-    }
-    for (int e = tid; e < 5 * nR; e += T) lm[e] = a.Lm[e];
-    __syncthreads();
-    if (a.k == 0) {
+        if (a.k == 0) {
 #pragma unroll
-        for (int t = 0; t < MEAN_ROWS; ++t) {
-            const int i = tid + T * t;
-            if (i < nR) {
-                ta[i] = mean_mult(a, al, i, a.ce0[1]);
-                tb[i] = mean_mult(a, be, i, a.ce0[1]);
+            for (int t = 0; t < MEAN_ROWS; ++t) {
+                const int i = tid + T * t;
+                if (i >= nR) continue;
+                row(mb, i)[0] = al[t];
+                row(mb, i)[1] = be[t];
             }
-        }
-        __syncthreads();
+            __syncthreads();
 #pragma unroll
-        for (int t = 0; t < MEAN_ROWS; ++t) {
-            const int i = tid + T * t;
-            if (i < nR) {
-                al[i] = ta[i];
-                be[i] = tb[i];
+            for (int t = 0; t < MEAN_ROWS; ++t) {
+                const int i = tid + T * t;
+                if (i < nR) mult(mb, i, a.ce0[1], al[t], be[t]);
             }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < MEAN_ROWS; ++t) {
-        const int i = tid + T * t;
-        if (i < nR) {
-            al[i].x += a.dtc * fr[t].x;
-            be[i].x += a.dtc * fr[t].y;
-            if (a.Src) {
-                const double2 sa = a.Src[(size_t) i * Mx], sb = a.Src[(size_t) (nR + i) * Mx];
-                al[i].x += sa.x;
-                al[i].y += sa.y;
-                be[i].x += sb.x;
-                be[i].y += sb.y;
-            }
-        }
-    }
-    __syncthreads();
-    if (a.exact_mean && a.k < 2) {
-        // the transpose of the flux correction on the right-hand side
-        double q = 0.0;
-        for (int i = tid; i < nR; i += T) q += a.add_mass[i] * al[i].x;
-        red[tid] = q;
-        __syncthreads();
-        for (int o = T / 2; o > 0; o >>= 1) {
-            if (tid < o) red[tid] += red[tid + o];
             __syncthreads();
         }
-        const double h = 0.5 * red[0];
-        __syncthreads();
-        for (int i = tid; i < nR; i += T) al[i].x -= h * a.rowsum[i];
-        __syncthreads();
-    }
-    const int n0 = (nR + 1) / 2, n1 = nR / 2;
-    if (tid == 0) chain_subst<2>(lm, 10, 1, al, 2, n0);
-    if (tid == 64) chain_subst<2>(lm + 5, 10, 1, al + 1, 2, n1);
-    if (tid == 128) chain_subst<2>(lm, 10, 1, be, 2, n0);
-    if (tid == 192) chain_subst<2>(lm + 5, 10, 1, be + 1, 2, n1);
-    __syncthreads();
-    double p = 0.0;
-    for (int i = tid; i < nR; i += T) p += a.rowsum[i] * al[i].x;
-    red[tid] = p;
-    __syncthreads();
-    for (int o = T / 2; o > 0; o >>= 1) {
-        if (tid < o) red[tid] += red[tid + o];
-        __syncthreads();
-    }
-    const double flux_t = a.target - red[0];
-    for (int i = tid; i < nR; i += T) {
-        if (!a.exact_mean) {
-            al[i].x = al[i].x + flux_t * a.add[i] * 0.5;
-            al[i].y = al[i].y + flux_t * 0.0 * 0.5;
-        }
-        Cs[(size_t) i * Mx] = al[i];
-        Cs[(size_t) (nR + i) * Mx] = be[i];
-    }
-    __syncthreads();
+        double q = 0.0;
 #pragma unroll
-    for (int t = 0; t < MEAN_ROWS; ++t) {
-        const int i = tid + T * t;
-        if (i >= nR) continue;
-        if (a.has_next) {
-            const double2 f = f2r[t];
-            double2 xa = mean_mult(a, al, i, a.cn[1]), xb = mean_mult(a, be, i, a.cn[1]);
-            Ca[(size_t) i * Mx] = make_double2(xa.x + a.dtd * f.x, xa.y + a.dtd * 0.0);
-            Cb[(size_t) i * Mx] = make_double2(xb.x + a.dtd * f.y, xb.y + a.dtd * 0.0);
-        } else {
-            Ca[(size_t) i * Mx] = al[i];
-            Cb[(size_t) i * Mx] = be[i];
+        for (int t = 0; t < MEAN_ROWS; ++t) {
+            const int i = tid + T * t;
+            if (i >= nR) continue;
+            al[t].x = __builtin_fma(a.dtc, fr[t].x, al[t].x);
+            be[t].x = __builtin_fma(a.dtc, fr[t].y, be[t].x);
+            if (Sm) {
+                const double2 sa = Sm[(size_t) i * Mx], sb = Sm[(size_t) (nR + i) * Mx];
+                al[t].x += sa.x;
+                al[t].y += sa.y;
+                be[t].x += sb.x;
+                be[t].y += sb.y;
+            }
+            if (a.exact_mean) q = __builtin_fma(a.add_mass[i], al[t].x, q);
+        }
+        double h = 0.0;
+        // the transpose of the flux correction on the right-hand side
+        if (a.exact_mean && a.k < 2) h = 0.5 * halving_sum(q, red);
+#pragma unroll
+        for (int t = 0; t < MEAN_ROWS; ++t) {
+            const int i = tid + T * t;
+            if (i >= nR) continue;
+            if (a.exact_mean && a.k < 2) al[t].x = __builtin_fma(-h, a.rowsum[i], al[t].x);
+            row(mb, i)[0] = al[t];
+            row(mb, i)[1] = be[t];
+        }
+    }
+    __syncthreads();
+    // eight chains a member: parity, column, part
+    if (tid < 8 * nmb) {
+        const int mb = tid >> 3, p = (tid >> 2) & 1;
+        double *v = (double *) row(mb, p) + (tid & 3);
+        const double *f = lds + p * img;
+        chain_forward<2, 1, 4>(f, v, nrp);
+        chain_backward<2, 1, 4>(f + nrp * 2, f + nrp * 4, v, nrp);
+    }
+    __syncthreads();
+    for (int mb = 0; mb < nmb; ++mb) {
+        const size_t m = m0 + mb;
+        cplx *Ca = C + m * a.ms_c, *Cb = Ca + (size_t) nR * Mx, *Sa = Cs + m * a.ms_cs;
+        const cplx *Fm2 = a.Fb2 + m * a.ms_fb2;
+        double p = 0.0;
+        for (int i = tid; i < nR; i += T) p = __builtin_fma(a.rowsum[i], row(mb, i)[0].x, p);
+        const double target = (a.alt_mask >> m) & 1u ? a.target_alt : a.target;
+        const double flux_t = target - halving_sum(p, red);
+#pragma unroll
+        for (int t = 0; t < MEAN_ROWS; ++t) {
+            const int i = tid + T * t;
+            if (i >= nR) continue;
+            double2 v = row(mb, i)[0];
+            if (!a.exact_mean) {
+                v.x = __builtin_fma(flux_t * a.add[i], 0.5, v.x);
+                row(mb, i)[0] = v;
+            }
+            Sa[(size_t) i * Mx] = v;
+            Sa[(size_t) (nR + i) * Mx] = row(mb, i)[1];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MEAN_ROWS; ++t) {
+            const int i = tid + T * t;
+            if (i >= nR) continue;
+            double2 xa = row(mb, i)[0], xb = row(mb, i)[1];
+            if (a.has_next) {
+                const double2 f = Fm2[(size_t) i * Mx];
+                mult(mb, i, a.cn[1], xa, xb);
+                xa.x = __builtin_fma(a.dtd, f.x, xa.x);
+                xb.x = __builtin_fma(a.dtd, f.y, xb.x);
+            }
+            Ca[(size_t) i * Mx] = xa;
+            Cb[(size_t) i * Mx] = xb;
         }
     }
 }
@@ -2468,48 +2201,43 @@ __device__ void nyquist_clear(const SolveArgs &a, int var, int par, int blk, cpl
         C[base + (size_t) (e / SBT) * 2 * Mx + e % SBT] = make_double2(0.0, 0.0);
 }
 
-// grid (nblk, 4, member groups), or (nblk + 1, 4, member groups) when the
-// mean mode needs a block of its own: blockIdx.y = field*2 + parity,
-// blockIdx.z = group of MB members (the last group may hold fewer: a.nm
-// members in all).  With Mx % SBT == 0 the blocks of the Nyquist row hold no
-// chains, and the first of them with blockIdx.y == 0 runs the mean mode (so
-// the grid is exactly the column blocks); otherwise the extra x-block nblk
-// with blockIdx.y == 0 does.  The mean mode runs member after member.
+// Tiles (column block, field and parity, group of MB members), groups fastest and
+// XCD-aware: the groups of a column block read the same factor image from one L2.
+// With Mx % SBT == 0 the blocks of the Nyquist row hold no chains; they come
+// first, and the first of them with field 0 and parity 0 runs the mean mode (so
+// the grid is exactly the column blocks, and the long mean chains start early);
+// otherwise the extra column block nblk does.  The registers are bounded for the
+// blocks that a CU's LDS holds: 36 KB a block at 48 rows, one member; 44 KB with
+// two, 47 KB at 64 rows; 57 KB and more beyond.
 template <int SBT, int VR, int MB>
-__global__ __launch_bounds__(SOLVE_THREADS, MB == 1 ? 4 : MB == 2 ? 3 : 2) void k_solve(SolveArgs a, cplx *C, cplx *Cs)
+__global__ __launch_bounds__(SOLVE_THREADS, VR <= 2 && MB == 1 ? 4 : VR * MB <= 4 && VR <= 3 && MB <= 2 ? 3 : 2)
+void k_solve(SolveArgs a, cplx *C, cplx *Cs)
 {
-    extern __shared__ double lds_solve[];
-    if (*a.abort_flag) return;
-    const int m0 = blockIdx.z * MB, nmb = min(MB, a.nm - m0);
-    const int var = blockIdx.y >> 1, par = blockIdx.y & 1, blk = blockIdx.x;
-    auto mean = [&]() {
-        for (int mb = 0; mb < nmb; ++mb) {
-            const int m = m0 + mb;
-            SolveArgs b = a;
-            if ((a.alt_mask >> m) & 1u) b.target = a.target_alt;
-            b.Fa += m * a.ms_fa;
-            b.Fb += m * a.ms_fb;
-            b.Fa2 += m * a.ms_fa2;
-            b.Fb2 += m * a.ms_fb2;
-            if (b.Src) b.Src += m * a.ms_src;
-            if (mb) __syncthreads();                 // the previous member's LDS reads done
-            solve_mean(b, C + m * a.ms_c, Cs + m * a.ms_cs, lds_solve);
-        }
-    };
-    if (blk == a.nblk) {
-        if (blockIdx.y == 0) mean();
-        return;
+    extern __shared__ __align__(16) double lds_solve[];
+    const int stop = *a.abort_flag;
+    const int ncol = a.nblk + (a.nyq_mean ? 0 : 1);
+    const int tile = xcd_tile(ncol * 4 * a.ngrp);
+    if (tile < 0) return;
+    const int cv = tile / a.ngrp, m0 = (tile - cv * a.ngrp) * MB, nmb = min(MB, a.nm - m0);
+    const int var = (cv & 3) >> 1, par = cv & 1, nyq = (a.Nz / 2) * a.Mx / SBT;
+    int blk = cv >> 2;
+    if (a.nyq_mean) {
+        const int per = a.Mx / SBT;                        // blocks of a kz row
+        blk = blk < per ? nyq + blk : blk < nyq + per ? blk - per : blk;
     }
-    if (a.nyq_mean && blk * SBT / a.Mx == a.Nz / 2) {
-        if (blockIdx.y == 0 && blk * SBT == (a.Nz / 2) * a.Mx) mean();
+    const bool clear = a.nyq_mean && blk * SBT / a.Mx == a.Nz / 2;
+    if ((clear || blk == a.nblk) && stop) return;
+    if (clear)
         for (int mb = 0; mb < nmb; ++mb)
             nyquist_clear<SBT>(a, var, par, blk, C + (m0 + mb) * a.ms_c);
+    if (clear || blk == a.nblk) {
+        if ((cv & 3) == 0 && (blk == nyq || !clear)) solve_mean(a, m0, nmb, C, Cs, lds_solve);
         return;
     }
     if (var == 0)
-        solve_block<4, SBT, VR, MB>(a, 0, par, blk, m0, nmb, C, Cs, lds_solve);
+        solve_block<4, SBT, VR, MB>(a, 0, par, blk, m0, nmb, stop, C, Cs, lds_solve);
     else
-        solve_block<2, SBT, VR, MB>(a, 1, par, blk, m0, nmb, C, Cs, lds_solve);
+        solve_block<2, SBT, VR, MB>(a, 1, par, blk, m0, nmb, stop, C, Cs, lds_solve);
 }
 
 // coefficient tables for the stages
@@ -2522,10 +2250,17 @@ static const double BD_[3] = {0., -2. / 3, -1. / 6};
 
 size_t solve_lds_bytes(int dimR, int sbt, int mb)
 {
-    const size_t nr = (size_t) (dimR + 1) / 2;
-    const size_t blk = nr * sbt * (9 * 8 + 32 * (size_t) mb);
-    const size_t mean = (size_t) dimR * (4 * 16 + 5 * 8) + SOLVE_THREADS * 8;
+    const size_t nrp = solve_rows(dimR), vrows = SOLVE_LEAD + nrp + SOLVE_TAIL;
+    const size_t blk = nrp * sbt * 9 * 8 + mb * vrows * sbt * 16;
+    const size_t mean = 2 * nrp * 5 * 8 + mb * 2 * vrows * 2 * 16 + SOLVE_THREADS * 8;
     return blk > mean ? blk : mean;
+}
+
+// Row slots of a worker: the chains' rows over the workers' rows of a pass
+static int solve_slots(int dimR, int sbt)
+{
+    const int step = SOLVE_WORKERS / sbt;
+    return ((dimR + 1) / 2 + step - 1) / step;
 }
 
 // Columns per solve block: 8, 4 or 2 (an even count keeps every block's
@@ -2533,26 +2268,44 @@ size_t solve_lds_bytes(int dimR, int sbt, int mb)
 // a row slot for every chain row; 0 when none fits.
 int solve_columns_per_block(int dimR)
 {
-    const int nr = (dimR + 1) / 2;
     for (int sbt = 8; sbt >= 2; sbt >>= 1)
-        if (solve_lds_bytes(dimR, sbt, 1) <= 64 * 1024 && nr <= SOLVE_VR_MAX * (SOLVE_THREADS / sbt))
+        if (solve_lds_bytes(dimR, sbt, 1) <= 64 * 1024 && solve_slots(dimR, sbt) <= SOLVE_VR_MAX)
             return sbt;
     return 0;
 }
 
-// Members per solve block (1, 2 or 4): the tuning's choice when set, else 4;
-// fewer when the run has fewer members or their vectors and the factor image
-// would not fit twice in the LDS of a CU.
+// Members per solve block (1, 2 or 4): the tuning's choice when set, else 2 (32
+// members at 64x97x64: 232 us a launch, 262 with one: the second member's vectors
+// come while the first's chain runs, and a third would take the LDS of a block);
+// fewer when the run has fewer members, when a worker would hold more than six
+// rows of them in registers, or when two blocks would not fit a CU's LDS.
 int solve_members_per_block(const Context &c)
 {
-    int mb = tuning().solve_mb > 0 ? tuning().solve_mb : 4;
-    // several members only with two row slots per thread (the four-slot
-    // form would spill its registers)
-    const bool two = (c.d.dimR + 1) / 2 <= 2 * (SOLVE_THREADS / c.sbt);
-    if (!two) mb = 1;
-    while (mb > 1 && (mb > c.nrun || 2 * solve_lds_bytes(c.d.dimR, c.sbt, mb) > 160 * 1024))
+    int mb = tuning().solve_mb > 0 ? tuning().solve_mb : 2;
+    while (mb > 1 && (mb > c.nrun || mb * solve_slots(c.d.dimR, c.sbt) > 6 ||
+                      2 * solve_lds_bytes(c.d.dimR, c.sbt, mb) > 160 * 1024))
         mb /= 2;
     return mb;
+}
+
+typedef void (*SolveKernel)(SolveArgs, cplx *, cplx *);
+
+template <int SBT, int VR>
+static SolveKernel solve_kernel_mb(int mb)
+{
+    if constexpr (4 * VR <= 6)
+        if (mb == 4) return k_solve<SBT, VR, 4>;
+    if constexpr (2 * VR <= 6)
+        if (mb == 2) return k_solve<SBT, VR, 2>;
+    return k_solve<SBT, VR, 1>;
+}
+
+template <int SBT>
+static SolveKernel solve_kernel(int slots, int mb)
+{
+    if (SBT == 8 && slots == 1) return solve_kernel_mb<SBT, 1>(mb);
+    if (slots <= 2) return solve_kernel_mb<SBT, 2>(mb);
+    return slots == 3 ? solve_kernel_mb<SBT, 3>(mb) : solve_kernel_mb<SBT, 4>(mb);
 }
 
 void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cplx *Fa2,
@@ -2589,7 +2342,6 @@ void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cp
     a.exact_mean = adj && exact_mean;
     a.add_mass = c.dAdd[0][k];
     a.abort_flag = c.abort_flag;
-    a.err = c.abort_flag + 2;
     a.ms_c = mstride(c, Ccarry);
     a.ms_cs = mstride(c, Csol);
     a.ms_fa = mstride(c, a.Fa);
@@ -2607,28 +2359,19 @@ void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cp
                    fcols * 8.0 * (9.0 * d.dimQ + 5.0 * d.dimR);
     const int sbt = c.sbt;
     const int ncol = d.Nz * d.Mx;
-    // members per block: the staged factor image feeds the chains of up to
-    // four members (2 sbt lanes each), within 160 KB of LDS per CU
     const int mb = solve_members_per_block(c);
     const size_t lds = solve_lds_bytes(d.dimR, sbt, mb);
     a.nm = c.nrun;
+    a.ngrp = (c.nrun + mb - 1) / mb;
     a.nblk = (ncol + sbt - 1) / sbt;
     a.mirror = c.factor_mirror;
     a.nyq_mean = d.Mx % sbt == 0;
-    const dim3 grid(a.nblk + (a.nyq_mean ? 0 : 1), 4, (c.nrun + mb - 1) / mb);
+    const dim3 grid(xcd_grid((a.nblk + (a.nyq_mean ? 0 : 1)) * 4 * a.ngrp));
     const hipStream_t st = c.stream;
-    // row slots per thread: the chains have at most (dimR + 1) / 2 rows
-    const bool two = (d.dimR + 1) / 2 <= 2 * (SOLVE_THREADS / sbt);
-    typedef void (*SolveKernel)(SolveArgs, cplx *, cplx *);
-    SolveKernel kern;
-    if (mb == 4)
-        kern = sbt == 8 ? k_solve<8, 2, 4> : sbt == 4 ? k_solve<4, 2, 4> : k_solve<2, 2, 4>;
-    else if (mb == 2)
-        kern = sbt == 8 ? k_solve<8, 2, 2> : sbt == 4 ? k_solve<4, 2, 2> : k_solve<2, 2, 2>;
-    else
-        kern = sbt == 8 ? (two ? k_solve<8, 2, 1> : k_solve<8, 4, 1>)
-             : sbt == 4 ? (two ? k_solve<4, 2, 1> : k_solve<4, 4, 1>)
-                        : (two ? k_solve<2, 2, 1> : k_solve<2, 4, 1>);
+    const int slots = solve_slots(d.dimR, sbt);
+    const SolveKernel kern = sbt == 8   ? solve_kernel<8>(slots, mb)
+                             : sbt == 4 ? solve_kernel<4>(slots, mb)
+                                        : solve_kernel<2>(slots, mb);
     if (lds > 64 * 1024)
         (void) hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int) lds);

@@ -23,9 +23,6 @@ namespace sc {
 
 typedef double2 cplx;
 
-// kernel error bits in abort_flag[2]
-constexpr int SC_KERR_SOLVE_WAIT = 1;   // band solve: factor staging never signalled
-
 // doubles between the planes' CFL maxima: a cache line each, as the blocks of a
 // launch update them with atomics (145 planes in 10 lines: 4 us of the primal x
 // kernel's 27 at 64x64x97)
@@ -152,16 +149,20 @@ struct Context {
     bool ypar = false;
     unsigned *rb_queue = nullptr;               // rebuild task queues [8][nyt][2], zero between launches
     // LU factors of the implicit operators, per (direction, stage), as the
-    // LDS images of the solve's blocks of sbt columns (col = z Mx + x):
-    //   alpha: [nblk][2 parities][(dimQ+1)/2 chain rows][9][sbt]
-    //   beta:  [nblk][2 parities][(dimR+1)/2 chain rows][5][sbt]
-    // (j<DL: L(i,i-2(DL-j)); j=DL: 1/U(i,i); j>DL: U(i,i+2(j-DL)); chain row
-    // r of parity p is matrix row p + 2r; zero outside the matrix and for the
-    // columns without a chain)
+    // images the solve's blocks of sbt columns (col = z Mx + x) keep in LDS.
+    // Chain row r of parity p is matrix row p + 2r; an image has
+    // nrp = solve_rows(dim) rows and holds, one after the other,
+    //   [nrp][sbt][DL]  L(r+k, k+1) at k: what row r's solution is applied with
+    //   [nrp][sbt][DL]  U(r, r+1+k) at k
+    //   [nrp][sbt]      1/U(r, r)
+    // (L(i, m), U(i, i+m): the factor m chain rows away; zero outside the
+    // matrix and for the columns without a chain), as [nblk][2 parities],
+    // alpha (DL = 4) in dLa, beta (DL = 2) in dLb
     double *dLa[2][3] = {{nullptr}}, *dLb[2][3] = {{nullptr}};
     int sbt = 0;                                // columns per solve block
     bool factor_mirror = false;                 // images stored for kz rows <= Nz/2 only
-    // mean mode: factors [dimR][5] and flux-correction vector [dimR]
+    // mean mode: its two parities' images (one column, DL = 2) and the
+    // flux-correction vector [dimR]
     double *dLm[2][3] = {{nullptr}}, *dAdd[2][3] = {{nullptr}};
 
     // state
@@ -200,8 +201,8 @@ struct Context {
     double *dotpart = nullptr;                  // partial sums
     size_t ndotpart = 0;                        // doubles in dotpart
     double *scal = nullptr;                     // [8] device scalars
-    // [0] CFL stop (1 + plane), [1] first unwritten slot, [2] kernel error
-    // bits (SC_KERR_*, sticky until reported), [3] always zero (never written)
+    // [0] CFL stop (1 + plane), [1] first unwritten slot, [3] always zero
+    // (never written)
     int *abort_flag = nullptr;
     double *objscr = nullptr;                   // objectives and statistics (objective_scratch_doubles)
     double *dRwall = nullptr;                   // [2][dimR]: R_j'(-1), R_j'(+1)
@@ -333,6 +334,9 @@ void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cp
                   const cplx *Fb2, double target, double target_alt = 0.0,
                   unsigned alt_mask = 0, const cplx *Src = nullptr, int exact_mean = 0);
 int solve_columns_per_block(int dimR);
+// rows of a chain's factor image: those of the longer parity, in eights (eight
+// for an empty operator)
+__host__ __device__ constexpr int solve_rows(int n) { return n > 0 ? ((n + 1) / 2 + 7) / 8 * 8 : 8; }
 // Re-sensitivity forcing of state S: fa [Nz][dimQ][Mx], fb [Nz][dimR][Mx], f0 [2][dimR]
 void launch_tangent_forcing(Context &c, const cplx *S, cplx *fa, cplx *fb, cplx *f0);
 // wall plane of C: Uxb, Uzb [Nz][Mx]

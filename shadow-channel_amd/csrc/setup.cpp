@@ -369,17 +369,27 @@ int setup_host(Context &c)
     c.factor_mirror = mirror;
     const int zrows = mirror ? Nz / 2 + 1 : Nz;
     const size_t nblk = ((size_t) zrows * Mx + sbt - 1) / sbt;
-    const size_t rqa = (nQ + 1) / 2, rqb = (nR + 1) / 2;
-    // position of factor j of matrix row i of column col in the block images
-    auto image = [&](size_t rmax, int W, int col, int i, int j) {
-        const size_t b = col / sbt, cc = col % sbt, par = i & 1, r = i >> 1;
-        return (((b * 2 + par) * rmax + r) * W + j) * sbt + cc;
+    // factors A (n rows of 2 dl + 1, inverted pivots) of column cc of sbt into
+    // its block's two images
+    auto to_image = [](const std::vector<double> &A, int n, int dl, double *img, int cc, int w) {
+        const int nrp = solve_rows(n), W = 2 * dl + 1;
+        for (int i = 0; i < n; ++i) {
+            double *p = img + (size_t) (i & 1) * nrp * W * w;
+            double *U = p + (size_t) nrp * dl * w, *D = U + (size_t) nrp * dl * w;
+            const int r = i >> 1;
+            for (int m = 1; m <= dl; ++m) {
+                if (r >= m) p[((size_t) (r - m + 1) * w + cc) * dl + m - 1] = A[(size_t) i * W + dl - m];
+                U[((size_t) r * w + cc) * dl + m - 1] = A[(size_t) i * W + dl + m];
+            }
+            D[(size_t) r * w + cc] = A[(size_t) i * W + dl];
+        }
     };
+    const size_t ia = (size_t) 2 * solve_rows(nQ) * 9 * sbt, ib = (size_t) 2 * solve_rows(nR) * 5 * sbt;
     for (int dir = 0; dir < 2; ++dir)
         for (int k = 0; k < 3; ++k) {
             const double bk = dir == 0 ? FWD_B[k] : ADJ_B[k];
             const double coef = d.re * bk * d.dt;
-            std::vector<double> La(nblk * 2 * rqa * 9 * sbt, 0.0), Lb(nblk * 2 * rqb * 5 * sbt, 0.0);
+            std::vector<double> La(nblk * ia, 0.0), Lb(nblk * ib, 0.0);
             for (int z = 0; z < zrows; ++z)
                 for (int x = 0; x < Mx; ++x) {
                     if ((z == 0 && x == 0) || z == Nz / 2) continue;
@@ -390,16 +400,12 @@ int setup_host(Context &c)
                                 coef * (s * c.Qs[e] + 2. * k2 * c.Qps[e] + c.Qpps[e]);
                     band_factor(A9.data(), nQ, 4);
                     device_factors(A9.data(), nQ, 4);
-                    for (int i = 0; i < nQ; ++i)
-                        for (int j = 0; j < 9; ++j)
-                            La[image(rqa, 9, col, i, j)] = A9[(size_t) i * 9 + j];
+                    to_image(A9, nQ, 4, &La[col / sbt * ia], col % sbt, sbt);
                     for (int e = 0; e < 5 * nR; ++e)
                         A5[e] = c.Rs[e] + coef * (c.Rps[e] + k2 * c.Rs[e]);
                     band_factor(A5.data(), nR, 2);
                     device_factors(A5.data(), nR, 2);
-                    for (int i = 0; i < nR; ++i)
-                        for (int j = 0; j < 5; ++j)
-                            Lb[image(rqb, 5, col, i, j)] = A5[(size_t) i * 5 + j];
+                    to_image(A5, nR, 2, &Lb[col / sbt * ib], col % sbt, sbt);
                 }
             if (upload(&c.dLa[dir][k], La) || upload(&c.dLb[dir][k], Lb)) {
                 last_error() = "device allocation of factors failed";
@@ -407,9 +413,10 @@ int setup_host(Context &c)
             }
             // mean mode: LHS factors and the flux-correction vector
             for (int e = 0; e < 5 * nR; ++e) A5[e] = c.Rs[e] + coef * c.Rps[e];
-            std::vector<double> Lm(A5);
-            band_factor(Lm.data(), nR, 2);
-            device_factors(Lm.data(), nR, 2);
+            std::vector<double> Am(A5), Lm((size_t) 2 * solve_rows(nR) * 5, 0.0);
+            band_factor(Am.data(), nR, 2);
+            device_factors(Am.data(), nR, 2);
+            to_image(Am, nR, 2, Lm.data(), 0, 1);
             // primal and tangent use the mass matrix (channel/project0.c:85-98),
             // the adjoint the stage matrix (channel/adjproject0.c:82-95)
             std::vector<double> M = dir == 0 ? c.Rs : A5;
