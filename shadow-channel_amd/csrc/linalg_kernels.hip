@@ -1141,38 +1141,61 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_rows(ForceArgs a, int bpi,
 // weights are halved, so that S = 2 v(0) gives the weight once, and the
 // functions that D multiplies vanish there.  A block owns one pair of row
 // tiles (even rows 2(16p + n), odd rows 2(16p + n) + 1), stages their
-// weighted bases [NKS][2][NB][64] and runs tasks as k_force_rows.  Field
-// values are read with buffer loads over the whole field array: the points
-// past the half domain, whose staged weights are zero, read values in or
-// past the array (zero past its end) and need no clamp.
-template <bool ADJ, int NKS>
+// weighted bases [NKS][2][NB][64] and runs the (kz row, n-tile) tasks of a
+// contiguous range.  Field values are read with buffer loads over the whole
+// field array: the points past the half domain, whose staged weights are zero,
+// read values in or past the array (zero past its end) and need no clamp.
+//
+// What bounds it: the FP64 unit, which FP64 products and FP64 vector
+// instructions share (a product 65 clocks a SIMD, a multiply-add or add 4.5, a
+// conversion 6.5, one after the other), and with members the loads' way through
+// the L1.  So a k-step is held to the products and as few other FP64
+// instructions as the combinations need: their signs and the mean column's case
+// sit in per-lane coefficients.  The fields come through a ring of PD k-steps,
+// refilled for the k-step PD later, or for the next task's, as soon as a
+// k-step's combinations are formed; the first ring is requested before the
+// bases, and FP32 slots are converted when used (when loaded, the conversion
+// waited for the load).  Measured against chunks requested task by task, 104
+// instead of 55 vector instructions a k-step: 32 mixed members at 64x97x64 588
+// -> 460 us (adjoint) and 259 -> 206 us, two at 128x129x128 216 -> 193 and 95 ->
+// 77 us, nine FP64 members 50 -> 44.5 us, one FP64 solution 25.6 -> 24.7 and 13.4
+// -> 13.0 us.
+//
+// The sums of the two halves of the k-steps are added at the end (NH = 2).
+// KS = 2: two waves share a task, one half each, and add through LDS.  KS = 1: a
+// wave sums both halves, no barrier.
+template <bool ADJ, int NKS, bool P32, int KS>
 struct ForceParShape {
     static constexpr int NB = ADJ ? 5 : 3;
     static constexpr int NF = ADJ ? 5 : 3;
-    // KS waves share a task's k-steps (partial sums added through LDS)
-    // where the exchange area fits beside the staged bases
-    static constexpr int XCH1 = 4 * 4 * 64;                  // doubles of one wave's partials
-    static constexpr int KS = (NKS % 2 == 0 &&
-                               (NKS * 2 * NB * 64 + (FR_THREADS / 128) * XCH1) * 8 <= 160 * 1024) ? 2 : 1;
-    static constexpr int KW = NKS / KS;                      // k-steps per wave
+    // the bases of 28 adjoint k-steps leave no room for an exchange of halves
+    static constexpr int NH = ADJ && NKS == 28 ? 1 : 2;
+    static constexpr int KW = NKS / NH;                      // k-steps of a half
+    static constexpr int KT = NKS / KS;                      // k-steps of a wave's task
     static constexpr int TPR = FR_THREADS / 64 / KS;         // tasks per round of the block
-    static constexpr int XCH = KS > 1 ? TPR * (KS - 1) * XCH1 : 0;
-    static constexpr int CKMAX = ADJ ? 2 : 5;
-    static constexpr int pick(int ck) { return KW % ck == 0 ? ck : pick(ck - 1); }
-    static constexpr int CK = pick(CKMAX), NCH = KW / CK;
+    static constexpr int XCH1 = 4 * 4 * 64;                  // doubles of one wave's partials
+    static constexpr int XCH = KS > 1 ? TPR * XCH1 : 0;
+    // ring: 4, 5 or 7 k-steps, a divisor of KW; 2 where those would not leave
+    // the registers for two waves a SIMD (FP64 adjoint, FP64 28 k-steps)
+    static constexpr int PD = !P32 && (ADJ || NKS == 28) ? 2 : KW % 5 == 0 ? 5 : KW % 4 == 0 ? 4 : 7;
+    // k-steps of an unrolled group: whole turns of the ring and of the two
+    // buffers of basis fragments
+    static constexpr int UN = PD % 2 ? 2 * PD : PD;
+    static_assert(KT % UN == 0 && KW % PD == 0 && KS <= NH, "a task is whole groups");
     static constexpr size_t lds_bytes() { return sizeof(double) * ((size_t) NKS * 2 * NB * 64 + XCH); }
 };
 // P32: the product slots are FP32 complex (mixed precision; same element
-// index), converted to FP64 on load
-template <bool ADJ, int NKS, bool P32>
+// index), converted to FP64 when used
+template <bool ADJ, int NKS, bool P32, int KS>
 __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, int nprob,
                                                           const cplx *U0, cplx *Fa0, cplx *Fb0,
                                                           const cplx *U1, cplx *Fa1, cplx *Fb1)
 {
-    using SH = ForceParShape<ADJ, NKS>;
-    constexpr int NB = SH::NB, NF = SH::NF, CK = SH::CK, NCH = SH::NCH, KS = SH::KS;
+    using SH = ForceParShape<ADJ, NKS, P32, KS>;
+    constexpr int NB = SH::NB, NF = SH::NF, PD = SH::PD, UN = SH::UN, KT = SH::KT, NG = KT / UN;
     constexpr unsigned ESZ = P32 ? 8 : 16;                   // bytes of a slot value
-    constexpr int KW = SH::KW, TPR = SH::TPR, XCH1 = SH::XCH1;
+    constexpr int TPR = SH::TPR, XCH1 = SH::XCH1;
+    typedef typename std::conditional<P32, float, double>::type V;
     extern __shared__ double bsf[];
     if (*a.abort_flag) return;
     // XCD-aware: block b runs task range lb = (b / 8 / npair) 8 + b % 8 of
@@ -1188,29 +1211,15 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, 
     const int nnt = (Mx + 7) / 8;
     const int ntask = (a.Nz - 1) * nnt;
     const int nall = ntask * nprob * a.nm;
-    const int t0 = lb * nall / bpi, t1 = (lb + 1) * nall / bpi;
-    {
-        // fragQ [npair][NKS][2][5][64] -> [NKS][2][NB][64]
-        const double *frag = a.frag + (size_t) tp * NKS * 2 * 5 * 64;
-        constexpr int TOT = NKS * 2 * NB * 64, PT = (TOT + FR_THREADS - 1) / FR_THREADS;
-        double st[PT];
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            const int e = min((int) threadIdx.x + FR_THREADS * i, TOT - 1);
-            const int sp = e / (NB * 64), r = e - sp * NB * 64, m = r >> 6, l = r & 63;
-            const int mm = ADJ ? m : (m == 2 ? 3 : m);       // primal: Qpw, Qw, Rw
-            st[i] = frag[((size_t) sp * 5 + mm) * 64 + l];
-        }
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            const int e = threadIdx.x + FR_THREADS * i;
-            if (e < TOT) bsf[e] = st[i];
-        }
-    }
-    __syncthreads();
+    const int t0 = (int) ((long long) lb * nall / bpi), t1 = (int) ((long long) (lb + 1) * nall / bpi);
+    const int part = ncol_part(nl), half = KS > 1 ? wave % KS : 0, slot = wave / KS, kb = half * KT;
+    const unsigned ubytes = (unsigned) ((size_t) a.Nz * 5 * q * Mx * ESZ);
+    const unsigned rowb = (unsigned) Mx * ESZ, slotb = (unsigned) q * rowb;
     struct Task {
-        int z, nt, xcol, part, p, m;
-        unsigned off;                                         // bytes: row z, column xcol
+        int z, nt, p, m;
+        // bytes of the lane's column at its first point (row kb 4 + kq): the
+        // part that P, P2, Z, Z2 read and the part that Hy does
+        unsigned other, own;
     };
     auto task_of = [&](int t) {
         Task k;
@@ -1221,116 +1230,161 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, 
         const int zr = t / nnt;
         k.z = zr < a.Nz / 2 ? zr : zr + 1;
         k.nt = t - zr * nnt;
-        k.xcol = min(k.nt * 8 + ncol_x(nl), Mx - 1);
-        k.part = ncol_part(nl);
-        k.off = (unsigned) (((size_t) k.z * 5 * q * Mx + k.xcol) * ESZ);
+        const int xcol = min(k.nt * 8 + ncol_x(nl), Mx - 1);
+        const bool mean = k.z == 0 && xcol == 0;
+        const unsigned off = (unsigned) (((size_t) k.z * 5 * q * Mx + xcol) * ESZ) + (unsigned) (kb * 4 + kq) * rowb;
+        k.other = off + (mean ? 0 : 1 - part) * (ESZ / 2);
+        k.own = off + part * (ESZ / 2);
         return k;
     };
-    const unsigned ubytes = (unsigned) ((size_t) a.Nz * 5 * q * Mx * ESZ);
-    const unsigned rowb = (unsigned) Mx * ESZ, slotb = (unsigned) q * rowb;
-    // r[buf][0: y, 1: mirror][field][k-step]
-    double r[2][2][NF][CK];
-    auto load = [&](const Task &k, int ch, int buf) {
+    // r[slot of the ring][0: y, 1: mirror][field]
+    V r[PD][2][NF];
+    // k-step kb + s of task k (s = g PD + u) into slot u: uniform offsets for the
+    // field and the point; the mirror runs down from row q - 1 - (kb 4 + kq)
+    const unsigned md = (unsigned) (q - 1 - 2 * (kb * 4 + kq)) * rowb;
+    auto load = [&](const Task &k, int s, int u) {
         __amdgpu_buffer_rsrc_t rs =
             __builtin_amdgcn_make_buffer_rsrc((void *) ((k.p ? U1 : U0) + k.m * a.ms_u), 0, ubytes, 0x00020000);
-        const bool mean = k.z == 0 && k.xcol == 0;
-        const unsigned other = k.off + (mean ? 0 : 1 - k.part) * (ESZ / 2),
-                       own = k.off + k.part * (ESZ / 2);
-        // lane offsets for the point and the part, uniform slot offsets
-        auto ld = [&](unsigned v, unsigned slot) {
+        auto ld = [&](unsigned v, unsigned so) {
             if constexpr (P32)
-                return (double) __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int) v, (int) (slot * slotb), 0));
+                return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int) v, (int) so, 0));
             else
-                return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, (int) v, (int) (slot * slotb), 0));
+                return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, (int) v, (int) so, 0));
         };
+        const unsigned step = (unsigned) s * 4 * rowb;
 #pragma unroll
-        for (int s = 0; s < CK; ++s) {
-            const int y = (ch * CK + s) * 4 + kq, ym = q - 1 - y;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const unsigned e = (unsigned) (h ? ym : y) * rowb;
-                r[buf][h][1][s] = ld(e + other, 0);
-                r[buf][h][0][s] = ld(e + other, 1);
-                r[buf][h][2][s] = ld(e + own, 2);
-                if (ADJ) {
-                    r[buf][h][3 % NF][s] = ld(e + other, 3);
-                    r[buf][h][4 % NF][s] = ld(e + other, 4);
-                }
+        for (int h = 0; h < 2; ++h) {
+            const unsigned vo = h ? k.other + md - step : k.other, vw = h ? k.own + md - step : k.own;
+            const unsigned so = h ? 0 : step;
+            r[u][h][1] = ld(vo, so);
+            r[u][h][0] = ld(vo, so + slotb);
+            r[u][h][2] = ld(vw, so + 2 * slotb);
+            if constexpr (ADJ) {
+                r[u][h][3] = ld(vo, so + 3 * slotb);
+                r[u][h][4] = ld(vo, so + 4 * slotb);
             }
         }
     };
-    // Rounds of TPR tasks: task t + wave / KS, k-steps [kb, kb + KW) of it
-    // with kb = (wave % KS) KW.  The partial sums of the waves kb > 0 go
-    // through LDS to the wave kb = 0, which adds them in order and stores.
-    const int part = wave % KS, slot = wave / KS, kb = part * KW;
-    double *xch = bsf + (size_t) NKS * 2 * NB * 64;
-    for (int t = t0; t < t1; t += TPR) {
-        const int tk = t + slot;
-        const bool act = tk < t1;
-        mf4 aAe = mf4_zero(), aBe = mf4_zero(), aAo = mf4_zero(), aBo = mf4_zero();
-        const Task k = task_of(act ? tk : t0);
-        if (act) {
-            const bool mean = k.z == 0 && k.xcol == 0;
-            const double kz = wave_kz(k.z, a.Nz, a.az);
-            const double kx = wave_kx(k.xcol, a.ax), k2 = kz * kz + kx * kx;
-            const double sg = k.part ? 1.0 : -1.0;
-            auto chunk = [&](int ch, int buf) {
-                const double *bc = bsf + (size_t) (kb + ch * CK) * 2 * NB * 64 + lane;
+    int t = t0 + slot;
+    Task k = task_of(min(t, nall - 1));
+    if (t < t1) {
 #pragma unroll
-                for (int u = 0; u < CK; ++u) {
+        for (int u = 0; u < PD; ++u) load(k, u, u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        // fragQ [npair][NKS][2][5][64] -> [NKS][2][NB][64]
+        const double *frag = a.frag + (size_t) tp * NKS * 2 * 5 * 64;
+        constexpr int TOT = NKS * 2 * NB * 64, PT = (TOT + FR_THREADS - 1) / FR_THREADS;
+        double st[PT];
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            const int e = min((int) threadIdx.x + FR_THREADS * i, TOT - 1);
+            const int sp = e / (NB * 64), rr = e - sp * NB * 64, m = rr >> 6, l = rr & 63;
+            const int mm = ADJ ? m : (m == 2 ? 3 : m);       // primal: Qpw, Qw, Rw
+            st[i] = frag[((size_t) sp * 5 + mm) * 64 + l];
+        }
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            const int e = threadIdx.x + FR_THREADS * i;
+            if (e < TOT) bsf[e] = st[i];
+        }
+    }
+    __syncthreads();
+    double *xch = bsf + (size_t) NKS * 2 * NB * 64;
+    // the lane's basis fragments of a k-step: even rows' NB, then odd rows'
+    double bf[2][2 * NB];
+    auto fragments = [&](double *f, int s) {
+        const double *b = bsf + (size_t) (kb + s) * 2 * NB * 64 + lane;
+#pragma unroll
+        for (int e = 0; e < 2 * NB; ++e) f[e] = b[e * 64];
+    };
+    fragments(bf[0], 0);
+    // rounds of TPR tasks, the same count in every wave of a KS = 2 block
+    for (int tb = t0; KS > 1 ? tb < t1 : t < t1; tb += TPR, t += TPR) {
+        const bool act = t < t1, more = t + TPR < t1;
+        const Task kn = task_of(more ? t + TPR : min(t, nall - 1));
+        mf4 aAe = mf4_zero(), aBe = mf4_zero(), aAo = mf4_zero(), aBo = mf4_zero();
+        mf4 bAe, bBe, bAo, bBo;                              // the first half's sums (KS = 1)
+        if (act) {
+            // the lane's combinations, signs in the coefficients:
+            //   P = px hx + pz hz, Y = ky hy, P2 = qx hx - qz hz,
+            //   Z = px sz - pz sx, Z2 = wz sz + wx sx
+            // the mean column takes P = Y = Z = 0, P2 = hx (first part) or hz,
+            // Z2 = sz or -sx
+            const int xcol = min(k.nt * 8 + ncol_x(nl), Mx - 1);
+            const bool mean = k.z == 0 && xcol == 0;
+            const double kz = wave_kz(k.z, a.Nz, a.az);
+            const double kx = wave_kx(xcol, a.ax), k2 = __builtin_fma(kx, kx, kz * kz);
+            const double sg = part ? 1.0 : -1.0;
+            const double px = mean ? 0.0 : sg * kx, pz = mean ? 0.0 : sg * kz, ky = mean ? 0.0 : -k2;
+            const double qx = mean ? 1.0 - part : pz, qz = mean ? -part : px;
+            const double wz = mean ? 1.0 - part : pz, wx = mean ? -part : px;
+#pragma unroll 1
+            for (int g = 0; g < NG; ++g) {
+#pragma unroll
+                for (int u = 0; u < UN; ++u) {
+#pragma clang fp contract(off)   // Y is rounded before its sums
+                    const int w = u % PD;                    // ring slot
+                    if (KS < SH::NH && u == SH::KW % UN && g == SH::KW / UN) {
+                        bAe = aAe; bBe = aBe; bAo = aAo; bBo = aBo;
+                        aAe = aBe = aAo = aBo = mf4_zero();
+                    }
                     double vP[2], vY[2], vP2[2], vZ[2] = {0.0, 0.0}, vZ2[2] = {0.0, 0.0};
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        const double hx = r[buf][h][0][u], hz = r[buf][h][1][u], hy = r[buf][h][2][u];
-                        if (mean) {
-                            vP[h] = 0.0;
-                            vY[h] = 0.0;
-                            vP2[h] = k.part ? hz : hx;
-                            if (ADJ) vZ2[h] = k.part ? -r[buf][h][3 % NF][u] : r[buf][h][4 % NF][u];
-                        } else {
-                            vP[h] = sg * (kx * hx + kz * hz);
-                            vY[h] = -k2 * hy;
-                            vP2[h] = sg * (kz * hx - kx * hz);
-                            if (ADJ) {
-                                vZ[h] = -sg * (kz * r[buf][h][3 % NF][u] - kx * r[buf][h][4 % NF][u]);
-                                vZ2[h] = sg * (kz * r[buf][h][4 % NF][u] + kx * r[buf][h][3 % NF][u]);
-                            }
+                        const double hx = r[w][h][0], hz = r[w][h][1], hy = r[w][h][2];
+                        vP[h] = ADJ || NKS != 8 ? __builtin_fma(px, hx, pz * hz)
+                                                : __builtin_fma(pz, hz, px * hx);
+                        vY[h] = ky * hy;
+                        vP2[h] = __builtin_fma(qx, hx, -(qz * hz));
+                        if constexpr (ADJ) {
+                            const double sx = r[w][h][3], sz = r[w][h][4];
+                            vZ[h] = __builtin_fma(-pz, sx, px * sz);
+                            vZ2[h] = __builtin_fma(wx, sx, wz * sz);
                         }
                     }
                     const double sP = vP[0] + vP[1], dP = vP[0] - vP[1];
                     const double sY = vY[0] + vY[1], dY = vY[0] - vY[1];
                     const double sP2 = vP2[0] + vP2[1], dP2 = vP2[0] - vP2[1];
-                    const double *be = bc + u * 2 * NB * 64, *bo = be + NB * 64;
+                    const double sZ = vZ[0] + vZ[1], dZ = vZ[0] - vZ[1];
+                    const double sZ2 = vZ2[0] + vZ2[1], dZ2 = vZ2[0] - vZ2[1];
+                    __builtin_amdgcn_sched_barrier(0);
+                    // the k-step PD on, of this task or the next
+                    if (u + PD < UN || g + 1 < NG)
+                        load(k, g * UN + u + PD, w);
+                    else if (more)
+                        load(kn, u + PD - UN, w);
+                    // the next k-step's basis fragments
+                    fragments(bf[(u + 1) & 1], u + 1 < UN || g + 1 < NG ? g * UN + u + 1 : 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const double *be = bf[u & 1], *bo = be + NB;
                     aAe = mfma_f64(dP, be[0], aAe);
                     aAo = mfma_f64(sP, bo[0], aAo);
-                    aBe = mfma_f64(sP2, be[(ADJ ? 3 : 2) * 64], aBe);
-                    aBo = mfma_f64(dP2, bo[(ADJ ? 3 : 2) * 64], aBo);
-                    aAe = mfma_f64(sY, be[64], aAe);
-                    aAo = mfma_f64(dY, bo[64], aAo);
-                    if (ADJ) {
-                        const double sZ = vZ[0] + vZ[1], dZ = vZ[0] - vZ[1];
-                        const double sZ2 = vZ2[0] + vZ2[1], dZ2 = vZ2[0] - vZ2[1];
-                        aAe = mfma_f64(sZ, be[2 * 64], aAe);
-                        aAo = mfma_f64(dZ, bo[2 * 64], aAo);
-                        aBe = mfma_f64(dZ2, be[4 * 64], aBe);
-                        aBo = mfma_f64(sZ2, bo[4 * 64], aBo);
+                    aBe = mfma_f64(sP2, be[ADJ ? 3 : 2], aBe);
+                    aBo = mfma_f64(dP2, bo[ADJ ? 3 : 2], aBo);
+                    aAe = mfma_f64(sY, be[1], aAe);
+                    aAo = mfma_f64(dY, bo[1], aAo);
+                    if constexpr (ADJ) {
+                        aAe = mfma_f64(sZ, be[2], aAe);
+                        aAo = mfma_f64(dZ, bo[2], aAo);
+                        aBe = mfma_f64(dZ2, be[4], aBe);
+                        aBo = mfma_f64(sZ2, bo[4], aBo);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            };
-            // chunks of CK k-steps through two register buffers, the loads of
-            // chunk ch + 1 issued before the products of chunk ch
-            load(k, kb / CK, 0);
-#pragma unroll
-            for (int ch = 0; ch < NCH; ++ch) {
-                if (ch + 1 < NCH) load(k, kb / CK + ch + 1, (ch + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-                chunk(ch, ch & 1);
-                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (KS < SH::NH) {
+                aAe = bAe + aAe;
+                aBe = bBe + aBe;
+                aAo = bAo + aAo;
+                aBo = bBo + aBo;
             }
         }
-        if (KS > 1) {
-            double *xw = xch + (size_t) (slot * (KS - 1) + part - 1) * XCH1 + lane;
-            if (act && part > 0) {
+        if constexpr (KS > 1) {
+            // the second half's sums go through LDS to the first half's wave
+            double *xw = xch + (size_t) slot * XCH1 + lane;
+            if (act && half > 0) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     xw[(0 * 4 + e) * 64] = aAe[e];
@@ -1340,21 +1394,17 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, 
                 }
             }
             __syncthreads();
-            if (act && part == 0) {
+            if (act && half == 0) {
 #pragma unroll
-                for (int p2 = 1; p2 < KS; ++p2) {
-                    const double *xr = xch + (size_t) (slot * (KS - 1) + p2 - 1) * XCH1 + lane;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        aAe[e] += xr[(0 * 4 + e) * 64];
-                        aBe[e] += xr[(1 * 4 + e) * 64];
-                        aAo[e] += xr[(2 * 4 + e) * 64];
-                        aBo[e] += xr[(3 * 4 + e) * 64];
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    aAe[e] += xw[(0 * 4 + e) * 64];
+                    aBe[e] += xw[(1 * 4 + e) * 64];
+                    aAo[e] += xw[(2 * 4 + e) * 64];
+                    aBo[e] += xw[(3 * 4 + e) * 64];
                 }
             }
         }
-        if (act && part == 0) {
+        if (act && half == 0) {
             cplx *Fa = (k.p ? Fa1 : Fa0) + k.m * a.ms_fa, *Fb = (k.p ? Fb1 : Fb0) + k.m * a.ms_fb;
 #pragma unroll
             for (int par = 0; par < 2; ++par) {
@@ -1373,7 +1423,24 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, 
         }
         // the exchange area is reused by the next round
         if (KS > 1) __syncthreads();
+        k = kn;
     }
+}
+
+template <bool ADJ, int NKS, bool P32, int KS>
+static void launch_force_par_ks(const ForceArgs &a, int npair, int bpi, int nprob, const cplx *U0,
+                                cplx *Fa0, cplx *Fb0, const cplx *U1, cplx *Fa1, cplx *Fb1,
+                                hipStream_t st)
+{
+    const size_t lds = ForceParShape<ADJ, NKS, P32, KS>::lds_bytes();
+    static bool attr = false;
+    if (!attr) {
+        (void) hipFuncSetAttribute((const void *) k_force_par<ADJ, NKS, P32, KS>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+        attr = true;
+    }
+    hipLaunchKernelGGL((k_force_par<ADJ, NKS, P32, KS>), dim3(npair * bpi), dim3(FR_THREADS), lds, st, a, bpi,
+                       nprob, U0, Fa0, Fb0, U1, Fa1, Fb1);
 }
 
 template <bool ADJ, int NKS, bool P32>
@@ -1381,19 +1448,21 @@ static void launch_force_par(const ForceArgs &a, int npair, int ntask, int nprob
                              cplx *Fa0, cplx *Fb0, const cplx *U1, cplx *Fa1, cplx *Fb1,
                              hipStream_t st)
 {
-    using SH = ForceParShape<ADJ, NKS>;
-    const size_t lds = SH::lds_bytes();
-    static bool attr = false;
-    if (!attr) {
-        (void) hipFuncSetAttribute((const void *) k_force_par<ADJ, NKS, P32>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        attr = true;
-    }
     // blocks per pair: a multiple of 8 (XCD-aware mapping), one block per CU
     const int cap = tuning().force_blocks > 0 ? tuning().force_blocks : 256 / npair / 8 * 8;
-    const int bpi = std::max(8, std::min((ntask * nprob * a.nm + 7) / 8 * 8, cap));
-    hipLaunchKernelGGL((k_force_par<ADJ, NKS, P32>), dim3(npair * bpi), dim3(FR_THREADS), lds, st, a, bpi,
-                       nprob, U0, Fa0, Fb0, U1, Fa1, Fb1);
+    const int nall = ntask * nprob * a.nm;
+    const int bpi = std::max(8, std::min((nall + 7) / 8 * 8, cap));
+    // a task per wave where a block has eight tasks or more, for FP32 slots (32
+    // members: 460 us, with two waves a task 480; FP64 slots leave no registers
+    // for both halves' sums: nine members 73 us, with two waves 44.5); two waves
+    // a task otherwise
+    if constexpr (ForceParShape<ADJ, NKS, P32, 1>::NH > 1) {
+        if (!P32 || nall < 8 * bpi) {
+            launch_force_par_ks<ADJ, NKS, P32, 2>(a, npair, bpi, nprob, U0, Fa0, Fb0, U1, Fa1, Fb1, st);
+            return;
+        }
+    }
+    launch_force_par_ks<ADJ, NKS, P32, 1>(a, npair, bpi, nprob, U0, Fa0, Fb0, U1, Fa1, Fb1, st);
 }
 
 template <bool ADJ, int NKS>
