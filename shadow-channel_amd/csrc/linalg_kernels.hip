@@ -67,10 +67,10 @@ __device__ __forceinline__ int ncol_x(int n) { return 2 * (n & 3) + (n >> 3); }
 __device__ __forceinline__ int ncol_part(int n) { return (n >> 2) & 1; }
 
 
-// most blocks per XCD of the parity rebuild, split over its half-domain y-tiles
-#ifndef SC_RB_BLOCKS
-#define SC_RB_BLOCKS 64
-#endif
+// most blocks per XCD of the parity rebuild, split over its half-domain y-tiles:
+// two a CU for FP64 (61 KB of basis at 24 k-steps), three for FP32 (32 members at
+// 64x97x64: 216 us, 230 with two)
+constexpr int RB_BLOCKS = 64, RB_BLOCKS_F32 = 96;
 
 // wave index within the block, in a scalar register: the compiler then
 // treats everything derived from it as uniform across the wave
@@ -328,26 +328,40 @@ __device__ __forceinline__ void rebuild_store(const RebuildArgs &a, int zrow, in
         return;
     }
     O *Uz = Uo + (size_t) zrow * 5 * ss;
-    auto put = [&](size_t i, double re, double im) { Uz[i] = O{(S) re, (S) im}; };
     const double kz = wave_kz(zrow, a.Nz, a.az);
+    O v[2][5];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int x = nt * 8 + 2 * kq + h;
-        if (x >= Mx || (zrow == 0 && x == 0)) continue;
-        const size_t o = (size_t) y * Mx + x;
+        auto put = [&](int s, double re, double im) { v[h][s] = O{(S) re, (S) im}; };
         // one reciprocal per column instead of eight divisions
-        const double kx = wave_kx(x, a.ax), r2 = 1.0 / (kz * kz + kx * kx);
-        const double2 v = make_double2(acc[0][2 * h], acc[0][2 * h + 1]);
+        const double kx = wave_kx(nt * 8 + 2 * kq + h, a.ax), r2 = 1.0 / (kz * kz + kx * kx);
         const double2 f = make_double2(-acc[1][2 * h], -acc[1][2 * h + 1]);
         const double2 g = make_double2(acc[3][2 * h], acc[3][2 * h + 1]);
-        put(o + 1 * ss, v.x, v.y);
-        put(o + 0 * ss, (kx * f.y + kz * g.y) * r2, -(kx * f.x + kz * g.x) * r2);
-        put(o + 2 * ss, (-kx * g.y + kz * f.y) * r2, (kx * g.x - kz * f.x) * r2);
+        put(0, (kx * f.y + kz * g.y) * r2, -(kx * f.x + kz * g.x) * r2);
+        put(1, acc[0][2 * h], acc[0][2 * h + 1]);
+        put(2, (-kx * g.y + kz * f.y) * r2, (kx * g.x - kz * f.x) * r2);
         if (VEL) continue;
         const double2 q2 = make_double2(acc[2][2 * h], acc[2][2 * h + 1]);
         const double2 gp = make_double2(acc[4][2 * h], acc[4][2 * h + 1]);
-        put(o + 3 * ss, (-kx * q2.y + kz * gp.y) * r2, (kx * q2.x - kz * gp.x) * r2);
-        put(o + 4 * ss, -(kx * gp.y + kz * q2.y) * r2, (kx * gp.x + kz * q2.x) * r2);
+        put(3, (-kx * q2.y + kz * gp.y) * r2, (kx * q2.x - kz * gp.x) * r2);
+        put(4, -(kx * gp.y + kz * q2.y) * r2, (kx * gp.x + kz * q2.x) * r2);
+    }
+    // the lane's columns x0 and x0 + 1; (0, 0) is the mean task's
+    const int x0 = nt * 8 + 2 * kq;
+    const bool in0 = x0 < Mx && !(zrow == 0 && x0 == 0), in1 = x0 + 1 < Mx;
+    O *Ux = Uz + (size_t) y * Mx + x0;
+    // FP32: both columns in one 16-byte store where a row of slots is a whole
+    // number of them (Mx even: x0, y Mx and a slot's elements all are)
+    typedef S s4 __attribute__((ext_vector_type(4)));
+    const bool both = sizeof(S) == sizeof(float) && Mx % 2 == 0 && in0;
+#pragma unroll
+    for (int s = 0; s < (VEL ? 3 : 5); ++s) {
+        if (both) {
+            *(s4 *) (Ux + s * ss) = s4{v[0][s].x, v[0][s].y, v[1][s].x, v[1][s].y};
+        } else {
+            if (in0) Ux[s * ss] = v[0][s];
+            if (in1) Ux[s * ss + 1] = v[1][s];
+        }
     }
 }
 
@@ -557,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_rows(RebuildArgs a, const cp
 // w, w + 4 bpq, ..., and issues its first coefficient loads before it
 // stages the basis.
 template <int NKS, bool VEL, class T>
-__global__ __launch_bounds__(256, 2) void k_rebuild_par(RebuildArgs a, const cplx *C, cplx *U)
+__global__ __launch_bounds__(256, sizeof(T) == sizeof(float) ? 3 : 2) void k_rebuild_par(RebuildArgs a, const cplx *C, cplx *U)
 {
     using ACC = typename YAcc<T>::type;
     __shared__ T bs[NKS * 5 * 64];
@@ -590,7 +604,7 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_par(RebuildArgs a, const cpl
     };
     constexpr int NKH = NKS / 2, CK = NKS / 4;
     static_assert(CK % 2 == 0, "a quarter must be whole pairs of k-steps");
-    T ca[2][CK], cb[2][CK];
+    double ca[2][CK], cb[2][CK];
     // quarter ch: parity ch / 2, k-steps (ch % 2) CK .. + CK - 1 of that
     // parity, as buffer loads over the whole coefficient array: a lane
     // offset plus a uniform k-step offset.  Rows past dimR - 1 (whose basis
@@ -605,18 +619,18 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_par(RebuildArgs a, const cpl
 #pragma unroll
         for (int s = 0; s < CK; ++s) {
             const int so = (s0 + s) * 8 * M2 * 8;
-            ca[buf][s] = (T) __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, va, so, 0));
-            cb[buf][s] = (T) __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, vb, so, 0));
+            ca[buf][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, va, so, 0));
+            cb[buf][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, vb, so, 0));
         }
     };
     auto chunk = [&](bool mean, int ch, int buf, ACC *acc) {
-        const T *xa = ca[buf], *xb = cb[buf];
+        const double *xa = ca[buf], *xb = cb[buf];
         const int sb = (ch >> 1) * NKH + (ch & 1) * CK;
         if (mean) {
 #pragma unroll
             for (int t = 0; t < CK; ++t) {
-                acc[3] = mfma_t(xa[t], bs[((sb + t) * 5 + 3) * 64 + lane], acc[3]);
-                if (!VEL) acc[4] = mfma_t(xa[t], bs[((sb + t) * 5 + 4) * 64 + lane], acc[4]);
+                acc[3] = mfma_t((T) xa[t], bs[((sb + t) * 5 + 3) * 64 + lane], acc[3]);
+                if (!VEL) acc[4] = mfma_t((T) xa[t], bs[((sb + t) * 5 + 4) * 64 + lane], acc[4]);
             }
             return;
         }
@@ -630,11 +644,11 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_par(RebuildArgs a, const cpl
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int t = t0 + u;
-                acc[0] = mfma_t(xa[t], p[u * 5 + 0], acc[0]);
-                acc[1] = mfma_t(xa[t], p[u * 5 + 1], acc[1]);
-                if (!VEL) acc[2] = mfma_t(xa[t], p[u * 5 + 2], acc[2]);
-                acc[3] = mfma_t(xb[t], p[u * 5 + 3], acc[3]);
-                if (!VEL) acc[4] = mfma_t(xb[t], p[u * 5 + 4], acc[4]);
+                acc[0] = mfma_t((T) xa[t], p[u * 5 + 0], acc[0]);
+                acc[1] = mfma_t((T) xa[t], p[u * 5 + 1], acc[1]);
+                if (!VEL) acc[2] = mfma_t((T) xa[t], p[u * 5 + 2], acc[2]);
+                acc[3] = mfma_t((T) xb[t], p[u * 5 + 3], acc[3]);
+                if (!VEL) acc[4] = mfma_t((T) xb[t], p[u * 5 + 4], acc[4]);
             }
         };
         ldb(sb, p0);
@@ -750,21 +764,21 @@ void launch_rebuild2(Context &c, const cplx *C0, cplx *U0, const cplx *C1, cplx 
     const dim3 grows(8 * c.nyt * bpq), gchunk(xcd_grid(c.nyt * d.Nz), nm);
     const int nksp = c.nksP;
     const bool par = c.ypar && (nksp == 8 || nksp == 16 || nksp == 24);
+    // mixed precision: the parity rebuild's products on the FP32 matrix cores
+    // and FP32 slots, except for outputs such as spec2phys
+    const bool f32 = slots32(c);
     RebuildArgs ap = a;
     ap.frag = c.dFragP;
     ap.nyt = c.nht;
     ap.nks = nksp;
     {
         // enough waves for one task each (of one rebuild of all members), at
-        // most about two blocks per CU
+        // most about two (FP32: three) blocks per CU
         const int ntmax = nm * ((d.Nz + 7) / 8 * ((d.Mx + 7) / 8));
-        const int rbb = tuning().rebuild_blocks > 0 ? tuning().rebuild_blocks : SC_RB_BLOCKS;
+        const int rbb = tuning().rebuild_blocks > 0 ? tuning().rebuild_blocks : f32 ? RB_BLOCKS_F32 : RB_BLOCKS;
         ap.bpq = std::max(1, std::min((ntmax + 3) / 4, rbb / c.nht));
     }
     const dim3 gpar(8 * c.nht * ap.bpq);
-    // mixed precision: the parity rebuild's products on the FP32 matrix cores
-    // and FP32 slots, except for outputs such as spec2phys
-    const bool f32 = slots32(c);
     typedef void (*RebuildKernel)(RebuildArgs, const cplx *, cplx *);
 #define SC_RB_PAR(N, V) (f32 ? (RebuildKernel) k_rebuild_par<N, V, float> : (RebuildKernel) k_rebuild_par<N, V, double>)
     auto go = [=]() {
