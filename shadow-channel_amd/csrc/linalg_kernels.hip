@@ -308,7 +308,8 @@ __device__ __forceinline__ RebuildTask rebuild_task(const RebuildArgs &a, int zr
 // are stored as O: double2, or float2 for the FP32 instance (the mixed-
 // precision steps, whose z-inverse transform reads FP32 slots at the same
 // element index; the member base address stays that of the FP64 layout).
-template <bool VEL = false, class ACC = mf4, class O = double2>
+// DIV: divisions by kx^2 + kz^2 as k_rebuild's, not products with its inverse.
+template <bool VEL = false, class ACC = mf4, class O = double2, bool DIV = false>
 __device__ __forceinline__ void rebuild_store(const RebuildArgs &a, int zrow, int nt, int y, int kq,
                                               const ACC *acc, cplx *U)
 {
@@ -334,17 +335,18 @@ __device__ __forceinline__ void rebuild_store(const RebuildArgs &a, int zrow, in
     for (int h = 0; h < 2; ++h) {
         auto put = [&](int s, double re, double im) { v[h][s] = O{(S) re, (S) im}; };
         // one reciprocal per column instead of eight divisions
-        const double kx = wave_kx(nt * 8 + 2 * kq + h, a.ax), r2 = 1.0 / (kz * kz + kx * kx);
+        const double kx = wave_kx(nt * 8 + 2 * kq + h, a.ax), k2 = kz * kz + kx * kx, r2 = 1.0 / k2;
+        auto over = [&](double w) { return DIV ? w / k2 : w * r2; };
         const double2 f = make_double2(-acc[1][2 * h], -acc[1][2 * h + 1]);
         const double2 g = make_double2(acc[3][2 * h], acc[3][2 * h + 1]);
-        put(0, (kx * f.y + kz * g.y) * r2, -(kx * f.x + kz * g.x) * r2);
+        put(0, over(kx * f.y + kz * g.y), -over(kx * f.x + kz * g.x));
         put(1, acc[0][2 * h], acc[0][2 * h + 1]);
-        put(2, (-kx * g.y + kz * f.y) * r2, (kx * g.x - kz * f.x) * r2);
+        put(2, over(-kx * g.y + kz * f.y), over(kx * g.x - kz * f.x));
         if (VEL) continue;
         const double2 q2 = make_double2(acc[2][2 * h], acc[2][2 * h + 1]);
         const double2 gp = make_double2(acc[4][2 * h], acc[4][2 * h + 1]);
-        put(3, (-kx * q2.y + kz * gp.y) * r2, (kx * q2.x - kz * gp.x) * r2);
-        put(4, -(kx * gp.y + kz * q2.y) * r2, (kx * gp.x + kz * q2.x) * r2);
+        put(3, over(-kx * q2.y + kz * gp.y), over(kx * q2.x - kz * gp.x));
+        put(4, -over(kx * gp.y + kz * q2.y), over(kx * gp.x + kz * q2.x));
     }
     // the lane's columns x0 and x0 + 1; (0, 0) is the mean task's
     const int x0 = nt * 8 + 2 * kq;
@@ -548,6 +550,140 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_rows(RebuildArgs a, const cp
             atomicExch(&qc[0], 0u);
             atomicExch(&qc[1], 0u);
         }
+    }
+}
+
+// k_rebuild for dimR <= 4 NKS (NKS = 32: dimR 97 to 128), the whole basis of a
+// y-tile in LDS: the same products in the same order, so the same bits.  The
+// tasks of an XCD's kz rows, eight waves' at a time, are numbered y-tile by
+// y-tile and split evenly over its blocks, one a CU; a block stages the basis
+// of its first y-tile and, once or twice, of the next.  A wave's coefficients
+// move in four quarters through two register buffers, the next quarter's loads
+// (or the next task's first) issued before the current quarter's products.
+// Bound by the FP64 products (113 us for two members at 128x129x128); the form
+// that stages the basis chunk by chunk behind a barrier, for four waves that
+// start and end every n-tile together, took 262 us, this one 188: the products take
+// 72% of its clocks with the divisions and other FP64 instructions that share
+// their unit; the rest is the change of basis and re-reading coefficients.
+constexpr int RW_THREADS = 512;
+template <int NKS>
+__global__ __launch_bounds__(RW_THREADS) void k_rebuild_wide(RebuildArgs a, const cplx *C, cplx *U)
+{
+    constexpr int CK = NKS / 4, NW = RW_THREADS / 64;
+    static_assert(CK % 4 == 0, "a quarter is whole groups of four k-steps");
+    __shared__ double bs[NKS * 5 * 64];
+    if (*a.abort_flag) return;
+    const int xcd = blockIdx.x & 7, ib = blockIdx.x >> 3;
+    const int z0 = xcd * a.Nz / 8, z1 = (xcd + 1) * a.Nz / 8;
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int kq = lane >> 4, nl = lane & 15;
+    const int nnt = (a.Mx + 7) / 8, nR = a.dimR, M2 = a.Mx * 2;
+    const int zm = a.Nz / 2;
+    const bool has_mean = zm >= z0 && zm < z1;
+    const int ntask1 = (z1 - z0) * nnt - (has_mean ? nnt - 1 : 0);
+    const int ntask = ntask1 * a.nprob * a.nm;
+    // groups of NW tasks: ng a y-tile, this block's g0 .. g1 - 1 of all
+    const int ng = (ntask + NW - 1) / NW;
+    const int g0 = (int) ((long long) ib * a.nyt * ng / a.bpq), g1 = (int) ((long long) (ib + 1) * a.nyt * ng / a.bpq);
+    auto task_of = [&](int t, int &zrow, int &nt) {
+        t -= (t / ntask1) * ntask1;
+        const int tm = has_mean ? (zm - z0) * nnt : ntask1;
+        const int u = t <= tm ? t : t - tm - 1;
+        zrow = t == tm ? zm : (t < tm ? z0 : zm + 1) + u / nnt;
+        nt = t == tm ? 0 : u % nnt;
+    };
+    auto task_ops = [&](int t) {
+        int zr, nt;
+        task_of(t, zr, nt);
+        RebuildTask r = rebuild_task(a, zr, nt, nl);
+        r.cd = (const double *) rb_src(a, C, t / ntask1);
+        return r;
+    };
+    double ca[2][CK], cb[2][CK];
+    // quarter ch of a task's coefficients as buffer loads over the whole array
+    // (rows past dimR - 1, whose basis fragments are zero, read the next rows
+    // or zero past the end)
+    const unsigned cbytes = (unsigned) ((size_t) a.Nz * 2 * nR * M2 * sizeof(double));
+    auto load = [&](const RebuildTask &t, int ch) {
+        __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *) t.cd, 0, cbytes, 0x00020000);
+        const int va = (int) (unsigned) ((t.offA + kq * M2) * 8), vb = (int) (unsigned) ((t.offB + kq * M2) * 8);
+#pragma unroll
+        for (int s = 0; s < CK; ++s) {
+            const int so = (ch * CK + s) * 4 * M2 * 8;
+            ca[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, va, so, 0));
+            cb[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, vb, so, 0));
+        }
+    };
+    auto chunk = [&](int ch, mf4 *acc) {
+        const double *xa = ca[ch & 1], *xb = cb[ch & 1];
+        double p0[10], p1[10];
+        auto ldb = [&](int s0, double *p) {
+#pragma unroll
+            for (int e = 0; e < 10; ++e) p[e] = bs[(s0 * 5 + e) * 64 + lane];
+        };
+        auto mm = [&](int t0, const double *p) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                acc[0] = mfma_f64(xa[t0 + u], p[u * 5 + 0], acc[0]);
+                acc[1] = mfma_f64(xa[t0 + u], p[u * 5 + 1], acc[1]);
+                acc[2] = mfma_f64(xa[t0 + u], p[u * 5 + 2], acc[2]);
+                acc[3] = mfma_f64(xb[t0 + u], p[u * 5 + 3], acc[3]);
+                acc[4] = mfma_f64(xb[t0 + u], p[u * 5 + 4], acc[4]);
+            }
+        };
+        const int sb = ch * CK;
+        ldb(sb, p0);
+#pragma unroll
+        for (int t0 = 0; t0 < CK; t0 += 4) {
+            ldb(sb + t0 + 2, p1);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(t0, p0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t0 + 4 < CK) ldb(sb + t0 + 4, p0);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(t0 + 2, p1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int gs = g0; gs < g1;) {
+        const int yt = gs / ng, ge = min(g1, (yt + 1) * ng);
+        int t = (gs - yt * ng) * NW + wave;
+        const int te = min(ntask, (ge - yt * ng) * NW);
+        if (t < te) load(task_ops(t), 0);
+        if (gs > g0) __syncthreads();                          // the last y-tile's products
+        {
+            const double *frag = a.frag + (size_t) yt * NKS * 5 * 64;
+            constexpr int PT = NKS * 5 * 64 / RW_THREADS;
+            static_assert(NKS * 5 * 64 % RW_THREADS == 0, "basis must split over the block");
+            double st[PT];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) st[i] = frag[threadIdx.x + RW_THREADS * i];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) bs[threadIdx.x + RW_THREADS * i] = st[i];
+        }
+        __syncthreads();
+        for (; t < te; t += NW) {
+            const RebuildTask cur = task_ops(t);
+            mf4 acc[5];
+#pragma unroll
+            for (int m = 0; m < 5; ++m) acc[m] = mf4_zero();
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch) {
+                if (ch < 3)
+                    load(cur, ch + 1);
+                else if (t + NW < te)
+                    load(task_ops(t + NW), 0);
+                __builtin_amdgcn_sched_barrier(0);
+                // (the mean task's alpha and beta fragments are one load's, and
+                // its first three sums are not used)
+                chunk(ch, acc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            int zr, nt;
+            task_of(t, zr, nt);
+            rebuild_store<false, mf4, double2, true>(a, zr, nt, yt * 16 + nl, kq, acc, rb_dst(a, U, t / ntask1));
+        }
+        gs = ge;
     }
 }
 
@@ -779,6 +915,11 @@ void launch_rebuild2(Context &c, const cplx *C0, cplx *U0, const cplx *C1, cplx 
         ap.bpq = std::max(1, std::min((ntmax + 3) / 4, rbb / c.nht));
     }
     const dim3 gpar(8 * c.nht * ap.bpq);
+    // whole basis of a y-tile in LDS (80 KB at 32 k-steps): a block a CU, never
+    // more than there are tasks for its first wave
+    RebuildArgs aw = a;
+    aw.bpq = std::max(1, std::min(32, c.nyt * (nm * nprob * ((d.Nz + 7) / 8) * ((d.Mx + 7) / 8) + 7) / 8));
+    const dim3 gwide(8 * aw.bpq);
     typedef void (*RebuildKernel)(RebuildArgs, const cplx *, cplx *);
 #define SC_RB_PAR(N, V) (f32 ? (RebuildKernel) k_rebuild_par<N, V, float> : (RebuildKernel) k_rebuild_par<N, V, double>)
     auto go = [=]() {
@@ -802,6 +943,8 @@ void launch_rebuild2(Context &c, const cplx *C0, cplx *U0, const cplx *C1, cplx 
             hipLaunchKernelGGL(k_rebuild_rows<16>, grows, dim3(256), 0, st, a, C0, U0);
         else if (nks == 24)
             hipLaunchKernelGGL(k_rebuild_rows<24>, grows, dim3(256), 0, st, a, C0, U0);
+        else if (nks == 32)
+            hipLaunchKernelGGL(k_rebuild_wide<32>, gwide, dim3(RW_THREADS), 0, st, aw, C0, U0);
         else
             for (int p = 0; p < nprob; ++p)
                 hipLaunchKernelGGL(k_rebuild, gchunk, dim3(256), 0, st, a, p ? C1 : C0, p ? U1 : U0);
