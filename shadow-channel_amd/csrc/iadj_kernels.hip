@@ -38,10 +38,8 @@ namespace sc {
 
 namespace {
 
-#ifndef SC_IA_XG
-#define SC_IA_XG 4
-#endif
-constexpr int IA_XG = SC_IA_XG;   // kx columns per block
+constexpr int IA_XG = 4;          // kx columns per block
+typedef double v2d __attribute__((ext_vector_type(2)));   // stays in registers in arrays
 constexpr int IA_THREADS = 256;   // rows: alpha on threads 0..127, beta on 128..255
 
 // adjoint RK3/CN coefficients (channel/increadjproject.c:34-37)
@@ -80,178 +78,299 @@ struct IadjArgs {
 __device__ __forceinline__ cplx cadd(cplx a, cplx b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ cplx cscale(cplx a, double s) { return make_double2(a.x * s, a.y * s); }
 
-// Forward and back substitution on the rows of parity p of a stride-2 band
-// system, in place on vec (row i at vec[i]), with column cc of a factor image
-// of the setup (sbt columns, both parities one after the other: see dLa in
-// sc_internal.h; no pivoting).  The last DL values stay in registers, so one
-// row waits only on the row before it.
-template <int DL>
-__device__ void chain_subst(cplx *vec, const double *img, int sbt, int cc, int N, int p)
+// Forward and back substitution of one part (real or imaginary) of the nr rows
+// of one parity of a stride-2 band system (no pivoting), in LDS: row r at v[4 r],
+// its factors at L[r XG DL + m - 1] = L(r + m - 1, m), U[r XG DL + m - 1] =
+// U(r, r + m) and D[r XG] = 1 / U(r, r), for rows up to the next multiple of
+// eight (zero past the chain).  Nearest terms first in both sweeps; the last DL
+// values stay in registers, and the operands of eight rows are read while the
+// eight before them are computed.
+template <int DL, int XG>
+__device__ __forceinline__ void chain_subst(double *v, const double *L, const double *U, const double *D, int nr)
 {
-    const int nr = (N - p + 1) / 2, nrp = solve_rows(N);
-    const double *L = img + (size_t) p * nrp * sbt * (2 * DL + 1) + cc * DL;
-    const double *U = L + (size_t) nrp * sbt * DL, *D = U + (size_t) nrp * sbt * DL - cc * (DL - 1);
-    const size_t rs = (size_t) sbt * DL;
-    cplx y[DL];
+    constexpr int B = 8, FR = XG * DL;
+    const int nrp = (nr + B - 1) / B * B;
+    double y[DL], f[B][DL], b[B], d[B];
 #pragma unroll
-    for (int m = 0; m < DL; ++m) y[m] = make_double2(0.0, 0.0);
-#pragma unroll 4
-    for (int r = 0; r < nr; ++r) {
-        cplx b = vec[p + 2 * r];
+    for (int m = 0; m < DL; ++m) y[m] = 0.0;
+    auto fwd = [&](int r0) {
 #pragma unroll
-        for (int m = 1; m <= DL; ++m) {
-            // L(r, m); rows before the first multiply zeros
-            const double l = L[max(r - m + 1, 0) * rs + m - 1];
-            b.x -= l * y[m - 1].x;
-            b.y -= l * y[m - 1].y;
+        for (int i = 0; i < B; ++i) {
+            // rows before the first multiply zeros
+#pragma unroll
+            for (int m = 0; m < DL; ++m) f[i][m] = L[max(r0 + i - m, 0) * FR + m];
+            b[i] = v[4 * min(r0 + i, nr - 1)];
         }
+    };
+    if (nr > 0) fwd(0);
+    for (int r0 = 0; r0 < nrp; r0 += B) {
+        double fc[B][DL], bc[B];
 #pragma unroll
-        for (int m = DL - 1; m > 0; --m) y[m] = y[m - 1];
-        y[0] = b;
-        vec[p + 2 * r] = b;
+        for (int i = 0; i < B; ++i) {
+#pragma unroll
+            for (int m = 0; m < DL; ++m) fc[i][m] = f[i][m];
+            bc[i] = b[i];
+        }
+        if (r0 + B < nrp) fwd(r0 + B);
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            double x = bc[i];
+#pragma unroll
+            for (int m = 0; m < DL; ++m) x = __builtin_fma(-fc[i][m], y[m], x);
+#pragma unroll
+            for (int m = DL - 1; m > 0; --m) y[m] = y[m - 1];
+            y[0] = x;
+            if (r0 + i < nr) v[4 * (r0 + i)] = x;
+        }
     }
 #pragma unroll
-    for (int m = 0; m < DL; ++m) y[m] = make_double2(0.0, 0.0);
-#pragma unroll 4
-    for (int r = nr - 1; r >= 0; --r) {
-        cplx v = vec[p + 2 * r];
+    for (int m = 0; m < DL; ++m) y[m] = 0.0;
+    auto bwd = [&](int r0) {
 #pragma unroll
-        for (int t = 1; t <= DL; ++t) {
-            const double u = U[r * rs + t - 1];
-            v.x -= u * y[t - 1].x;
-            v.y -= u * y[t - 1].y;
+        for (int i = 0; i < B; ++i) {
+#pragma unroll
+            for (int m = 0; m < DL; ++m) f[i][m] = U[(r0 + i) * FR + m];
+            b[i] = r0 + i < nr ? v[4 * (r0 + i)] : 0.0;
+            d[i] = D[(r0 + i) * XG];
         }
-        v = cscale(v, D[(size_t) r * sbt]);
+    };
+    if (nr > 0) bwd(nrp - B);
+    for (int r0 = nrp - B; r0 >= 0; r0 -= B) {
+        double fc[B][DL], bc[B], dc[B];
 #pragma unroll
-        for (int m = DL - 1; m > 0; --m) y[m] = y[m - 1];
-        y[0] = v;
-        vec[p + 2 * r] = v;
+        for (int i = 0; i < B; ++i) {
+#pragma unroll
+            for (int m = 0; m < DL; ++m) fc[i][m] = f[i][m];
+            bc[i] = b[i];
+            dc[i] = d[i];
+        }
+        if (r0 >= B) bwd(r0 - B);
+#pragma unroll
+        for (int i = B - 1; i >= 0; --i) {
+            double x = bc[i];
+#pragma unroll
+            for (int m = 0; m < DL; ++m) x = __builtin_fma(-fc[i][m], y[m], x);
+            x *= dc[i];
+#pragma unroll
+            for (int m = DL - 1; m > 0; --m) y[m] = y[m - 1];
+            y[0] = x;
+            if (r0 + i < nr) v[4 * (r0 + i)] = x;
+        }
     }
 }
 
-// One block row of the band operators: the Gram rows of row i in registers
-// (alpha: Qs, Qps, Qpps; beta: Rs, Rps, entries (i, i + 2o), zero outside
-// the matrix), combined per mode.
-struct GramRow {
-    double s[9], p[9], pp[9];
+// Row i of the operator (alpha: -(k2 Qs + Qps) + cv V, V = k2^2 Qs + 2 k2 Qps +
+// Qpps; beta: Rs - cv V, V = -(Rps + k2 Rs)) on v and of the viscous part V on m
+// (rows in LDS): e, mm.  The Gram bands are zero outside the
+// matrix, so columns are clamped and none is skipped; Qps reaches three off-diagonals of the four, Qpps two, Rps one of two.
+template <bool B>
+struct BandRow {
+    static constexpr int DL = B ? 2 : 4, W = 2 * DL + 1;
+    double s[W], p[W], pp[W];
+    __device__ __forceinline__ void load(const IadjArgs &a, int i)
+    {
+#pragma unroll
+        for (int o = 0; o < W; ++o) {
+            s[o] = (B ? a.Rs : a.Qs)[i * W + o];
+            p[o] = o > 0 && o < W - 1 ? (B ? a.Rps : a.Qps)[i * W + o] : 0.0;
+            pp[o] = !B && o > 1 && o < W - 2 ? a.Qpps[i * W + o] : 0.0;
+        }
+    }
+    __device__ __forceinline__ void apply(int i, int N, double k2, double cv, const cplx *v, const cplx *m,
+                                          cplx &e, cplx &mm) const
+    {
+        e = mm = make_double2(0.0, 0.0);
+        const double k4 = k2 * k2, t2 = 2. * k2;
+#pragma unroll
+        for (int o = 0; o < W; ++o) {
+            const int col = min(max(i + 2 * (o - DL), 0), N - 1);
+            const bool hp = o > 0 && o < W - 1;
+            const double ks = hp ? __builtin_fma(k2, s[o], p[o]) : k2 * s[o];     // k2 Qs + Qps
+            double vs, ex;
+            if (B) {
+                vs = -ks;
+                ex = __builtin_fma(cv, ks, s[o]);
+            } else {
+                vs = hp ? __builtin_fma(k4, s[o], t2 * p[o]) : k4 * s[o];
+                if (o > 1 && o < W - 2) vs += pp[o];
+                ex = __builtin_fma(cv, vs, -ks);
+            }
+            const cplx cv2 = v[col], mv = m[col];
+            e.x = __builtin_fma(ex, cv2.x, e.x);
+            e.y = __builtin_fma(ex, cv2.y, e.y);
+            mm.x = __builtin_fma(vs, mv.x, mm.x);
+            mm.y = __builtin_fma(vs, mv.y, mm.y);
+        }
+    }
 };
 
-__device__ __forceinline__ void load_gram(const IadjArgs &a, bool isb, int i, int N, GramRow &g)
+// Right-hand sides of row i of the alpha (B = false) or beta coefficients of the
+// block's columns
+template <bool B, class Valid>
+__device__ __forceinline__ void mode_rhs(const IadjArgs &a, int i, int z, int x0, double kz, const cplx *vec,
+                                         const cplx *smic, const Valid &valid, cplx *acc)
 {
-    const int dl = isb ? 2 : 4, w = 2 * dl + 1;
+    const int dQ = a.dQ, dR = a.dR, Mx = a.Mx, Nz = a.Nz, k = a.k, N = B ? dR : dQ;
+    const double dt = a.dt, re = a.re;
+    const size_t wp = (size_t) Nz * Mx;
+    BandRow<B> g;
+    if (k == 0) g.load(a, i);
 #pragma unroll
-    for (int o = 0; o < 9; ++o) {
-        g.s[o] = g.p[o] = g.pp[o] = 0.0;
-        if (o < w && i + 2 * (o - dl) >= 0 && i + 2 * (o - dl) < N) {
-            if (isb) {
-                g.s[o] = a.Rs[i * 5 + o];
-                g.p[o] = a.Rps[i * 5 + o];
-            } else {
-                g.s[o] = a.Qs[i * 9 + o];
-                g.p[o] = a.Qps[i * 9 + o];
-                g.pp[o] = a.Qpps[i * 9 + o];
-            }
+    for (int t = 0; t < IA_XG; ++t) {
+        acc[t] = make_double2(0.0, 0.0);
+        if (!valid(t)) continue;
+        const int x = x0 + t;
+        const double kx = a.Kx[x], k2 = kx * kx + kz * kz;
+        cplx c = vec[t * dR + i];
+        if (k == 0) {
+            cplx e, m;
+            g.apply(i, N, k2, B ? -re * kA[0] * dt : re * kA[0] * dt, vec + t * dR,
+                    smic + t * 2 * dR + (B ? dR : 0), e, m);
+            c = cadd(e, cscale(m, re * dt * (kA[0] + kB[0])));
         }
+        cplx gf = B ? a.Fb[((size_t) z * dR + i) * Mx + x] : a.Fa[((size_t) z * dQ + i) * Mx + x];
+        if (a.F) gf = cadd(gf, a.F[((((size_t) 0 * 2 + (B ? 1 : 0)) * Nz + z) * Mx + x) * dR + i]);
+        c = cadd(c, cscale(gf, dt * kC[k]));
+        const size_t wo = (size_t) z * Mx + x;
+        if (!B && i < 8) {
+            const cplx wb = a.W[wp + wo], wbt = a.W[3 * wp + wo], awb = a.W[5 * wp + wo];
+            const double mm = kLR[i] / 2. - k2 * kLX[i], vv = -k2 * kLR[i] + k2 * k2 * kLX[i];
+            c.x += mm * (wbt.x - wb.x) + dt * re * (kA[k] * wbt.x + kB[k] * wb.x) * vv +
+                   dt * re * (kA[k] + kB[k]) * awb.x * vv;
+            c.y += mm * (wbt.y - wb.y) + dt * re * (kA[k] * wbt.y + kB[k] * wb.y) * vv +
+                   dt * re * (kA[k] + kB[k]) * awb.y * vv;
+        }
+        if (B && i < 4) {
+            const cplx ub = a.W[wo], ubt = a.W[2 * wp + wo], aub = a.W[4 * wp + wo];
+            const double h = kLG[i] / 2.;
+            c.x += h * (ubt.x - ub.x) + dt * re * (kA[k] * ubt.x + kB[k] * ub.x) * (-k2 * h) +
+                   dt * re * (kA[k] + kB[k]) * aub.x * (-k2 * h);
+            c.y += h * (ubt.y - ub.y) + dt * re * (kA[k] * ubt.y + kB[k] * ub.y) * (-k2 * h) +
+                   dt * re * (kA[k] + kB[k]) * aub.y * (-k2 * h);
+        }
+        acc[t] = c;
     }
 }
 
-// entry o of row i: operator (alpha: -(k2 Qs + Qps) + cv V, beta: Rs + cv (Rps + k2 Rs))
-// and the viscous part V (alpha: k2^2 Qs + 2 k2 Qps + Qpps, beta: -(Rps + k2 Rs))
-__device__ __forceinline__ double g_op(const GramRow &g, bool isb, int o, double k2, double cv)
+// Row i of the next stage's explicit part: projections of LIU, forcing k + 1,
+// MIC[count - 1]
+template <bool B, class Valid>
+__device__ __forceinline__ void mode_next(const IadjArgs &a, int i, int z, int x0, double kz, const cplx *vec,
+                                          const cplx *smic, const Valid &valid)
 {
-    return isb ? g.s[o] + cv * (g.p[o] + k2 * g.s[o])
-               : -(k2 * g.s[o] + g.p[o]) + cv * (k2 * k2 * g.s[o] + 2. * k2 * g.p[o] + g.pp[o]);
-}
-__device__ __forceinline__ double g_visc(const GramRow &g, bool isb, int o, double k2)
-{
-    return isb ? -(g.p[o] + k2 * g.s[o]) : k2 * k2 * g.s[o] + 2. * k2 * g.p[o] + g.pp[o];
-}
-
-// sum_o op(i, o) v[i + 2o] and sum_o V(i, o) m[i + 2o] (v, m rows in LDS)
-__device__ __forceinline__ void band_pair(const GramRow &g, bool isb, int i, int N, double k2,
-                                          double cv, const cplx *v, const cplx *m, cplx &e, cplx &mm)
-{
-    const int dl = isb ? 2 : 4;
-    e = mm = make_double2(0.0, 0.0);
+    const int dQ = a.dQ, dR = a.dR, Mx = a.Mx, Nz = a.Nz, k = a.k, N = B ? dR : dQ;
+    const double dt = a.dt, re = a.re;
+    BandRow<B> g;
+    g.load(a, i);
 #pragma unroll
-    for (int o = 0; o < 9; ++o) {
-        if (o > 2 * dl) break;
-        const int col = i + 2 * (o - dl);
-        if (col < 0 || col >= N) continue;
-        const double ex = g_op(g, isb, o, k2, cv), vs = g_visc(g, isb, o, k2);
-        const cplx cv2 = v[col], mv = m[col];
-        e.x += ex * cv2.x; e.y += ex * cv2.y;
-        mm.x += vs * mv.x; mm.y += vs * mv.y;
+    for (int t = 0; t < IA_XG; ++t) {
+        if (!valid(t)) continue;
+        const int x = x0 + t;
+        const double kx = a.Kx[x], k2 = kx * kx + kz * kz;
+        cplx e, m;
+        g.apply(i, N, k2, B ? -re * kA[k + 1] * dt : re * kA[k + 1] * dt, vec + t * dR,
+                smic + t * 2 * dR + (B ? dR : 0), e, m);
+        cplx gf = B ? a.FLb[((size_t) z * dR + i) * Mx + x] : a.FLa[((size_t) z * dQ + i) * Mx + x];
+        if (a.F) gf = cadd(gf, a.F[((((size_t) 1 * 2 + (B ? 1 : 0)) * Nz + z) * Mx + x) * dR + i]);
+        const cplx c = cadd(cadd(e, cscale(gf, dt * kD[k + 1])), cscale(m, re * dt * (kA[k + 1] + kB[k + 1])));
+        a.IAC[((size_t) (z * 2 + (B ? 1 : 0)) * dR + i) * Mx + x] = c;
     }
 }
 
-// the (0, 0) mode (channel/increadjproject0.c:14-357), one block; wave-wide
-// sums over the Gauss points for its projections
+// the (0, 0) mode (channel/increadjproject0.c:14-357), one block.  It is the
+// longest of the launch, a chain of latencies, so whatever does not depend on the
+// solve is requested at once: both stages' products are projected in one pass over
+// the weights (32 Gauss points' in flight), the solve's factors wait in LDS.
 __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
 {
     const int q = a.q, dR = a.dR, Mx = a.Mx, Nz = a.Nz, k = a.k, tid = threadIdx.x;
     const int lane = tid & 63;
     const size_t plane = (size_t) q * Mx, wp = (size_t) Nz * Mx;
     const double dt = a.dt, re = a.re;
-    cplx *sal = sh, *sbe = sh + dR, *smic = sh + 2 * dR;          // smic [2][dR]
-    double *sp = (double *) (sh + 4 * dR);                        // [4][q]: Hx, Sz, Hz, Sx (real)
-    double *sf = sp + 4 * q;                                      // [2][dR]
+    const int nrp = solve_rows(dR);
+    cplx *sal = sh, *sbe = sh + dR, *smic = sh + 2 * dR;          // smic [2][2][dR]: MIC[count], MIC[count - 1]
+    double *sp = (double *) (sh + 6 * dR);                        // [2][4][q]: Hx, Sz, Hz, Sx (real) of IU, LIU
+    double *sfac = sp + 8 * q;                                    // [2][nrp][5]
     const cplx ub = a.W[0], wb = a.W[wp], ubt = a.W[2 * wp], wbt = a.W[3 * wp];
-    auto stage = [&](const cplx *U, const cplx *mic) {
-        for (int j = tid; j < q; j += IA_THREADS) {
-            sp[j] = U[plane + (size_t) j * Mx].x;
-            sp[q + j] = U[4 * plane + (size_t) j * Mx].x;
-            sp[2 * q + j] = U[(size_t) j * Mx].x;
-            sp[3 * q + j] = U[3 * plane + (size_t) j * Mx].x;
-        }
-        for (int r = tid; r < dR; r += IA_THREADS) {
-            smic[r] = mic[(size_t) r * Mx];
-            smic[dR + r] = mic[((size_t) dR + r) * Mx];
-        }
-    };
-    // f[r] = sum_j Rw Hx + Rpw Sz (alpha rows, threads < 128), Rw Hz - Rpw Sx
-    // (beta rows, threads >= 128): real parts; Rw, Rpw transposed ([q][dimR])
-    auto project = [&]() {
-        const bool b2 = tid >= 128;
-        const int r2 = b2 ? tid - 128 : tid;
-        if (r2 >= dR) return;
-        const double *p0 = sp + (b2 ? 2 * q : 0), *p1 = sp + (b2 ? 3 * q : q);
-        const double sg = b2 ? -1.0 : 1.0;
-        // batches of 8 Gauss points: 16 loads in flight before the sums
-        double f = 0.0;
-        for (int j0 = 0; j0 < q; j0 += 8) {
-            double w0[8], w1[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int j = min(j0 + u, q - 1);
-                w0[u] = a.tRw[(size_t) j * dR + r2];
-                w1[u] = a.tRpw[(size_t) j * dR + r2];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (j0 + u < q) f += w0[u] * p0[j0 + u] + sg * w1[u] * p1[j0 + u];
-        }
-        sf[b2 ? dR + r2 : r2] = f;
-    };
-    for (int r = tid; r < dR; r += IA_THREADS) {
-        sal[r] = a.IAC[(size_t) r * Mx];
-        sbe[r] = a.IAC[((size_t) dR + r) * Mx];
-    }
-    stage(a.IU, a.mic0);
-    __syncthreads();
-    project();
-    __syncthreads();
+    // alpha row r on threads < 128, beta row r on the others
     const bool isb = tid >= 128;
-    const int r = isb ? tid - 128 : tid;
-    GramRow g;
+    const int r = isb ? tid - 128 : tid, rc = min(r, dR - 1);
+    constexpr int PB = 32;
+    double w0[PB], w1[PB];                                        // weights of PB Gauss points
+    auto weights = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+            const size_t j = min(j0 + u, q - 1);
+            w0[u] = a.tRw[j * dR + rc];
+            w1[u] = a.tRpw[j * dR + rc];
+        }
+    };
+    BandRow<true> g;
+    cplx fk = make_double2(0.0, 0.0), fn = fk;
+    double ml;
+    {
+        // (q <= 195 and dR <= 128: one Gauss point and one row a thread)
+        const size_t o = (size_t) min(tid, q - 1) * Mx, o0 = (size_t) rc * Mx, os = (size_t) (isb ? dR : 0) * Mx;
+        const double u0 = a.IU[plane + o].x, u1 = a.IU[4 * plane + o].x, u2 = a.IU[o].x, u3 = a.IU[3 * plane + o].x;
+        double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
+        cplx m0 = make_double2(0.0, 0.0), m1 = m0;
+        const cplx c0 = a.IAC[os + o0];
+        if (k == 0) m0 = a.mic0[os + o0];
+        if (k < 2) {
+            l0 = a.LIU[plane + o].x;
+            l1 = a.LIU[4 * plane + o].x;
+            l2 = a.LIU[o].x;
+            l3 = a.LIU[3 * plane + o].x;
+            m1 = a.mic1[os + o0];
+        }
+        double lf[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) lf[i] = a.Lm[min(tid + i * IA_THREADS, 10 * nrp - 1)];
+        g.load(a, rc);
+        ml = a.mlift[rc];
+        if (a.F) {
+            fk = a.F[((size_t) (isb ? 1 : 0) * Nz * Mx) * dR + rc];
+            if (k < 2) fn = a.F[((size_t) (2 + (isb ? 1 : 0)) * Nz * Mx) * dR + rc];
+        }
+        weights(0);
+        if (tid < q) {
+            sp[tid] = u0; sp[q + tid] = u1; sp[2 * q + tid] = u2; sp[3 * q + tid] = u3;
+            sp[4 * q + tid] = l0; sp[5 * q + tid] = l1; sp[6 * q + tid] = l2; sp[7 * q + tid] = l3;
+        }
+        if (r < dR) {
+            (isb ? sbe : sal)[r] = c0;
+            smic[(isb ? dR : 0) + r] = m0;
+            smic[(isb ? 3 : 2) * dR + r] = m1;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (tid + i * IA_THREADS < 10 * nrp) sfac[tid + i * IA_THREADS] = lf[i];
+    }
+    __syncthreads();
+    // f[r] = sum_j Rw Hx + Rpw Sz (alpha), Rw Hz - Rpw Sx (beta): real parts;
+    // Rw, Rpw transposed ([q][dimR]); fl the same of LIU
+    double f = 0.0, fl = 0.0;
+    {
+        const double *p0 = sp + (isb ? 2 * q : 0), *p1 = sp + (isb ? 3 * q : q);
+        const double sg = isb ? -1.0 : 1.0;
+        for (int j0 = 0; j0 < q; j0 += PB) {
+            if (j0 > 0) weights(j0);
+#pragma unroll
+            for (int u = 0; u < PB; ++u)
+                if (j0 + u < q) {
+                    f += w0[u] * p0[j0 + u] + sg * w1[u] * p1[j0 + u];
+                    fl += w0[u] * p0[4 * q + j0 + u] + sg * w1[u] * p1[4 * q + j0 + u];
+                }
+        }
+    }
     cplx c = make_double2(0.0, 0.0);
     if (r < dR) {
-        load_gram(a, true, r, dR, g);
         const cplx *v = isb ? sbe : sal;
         c = v[r];
         if (k == 0) {
             // Rs - re a0 dt Rps on the coefficients, - re dt (a0 + b0) Rps MIC[count]
             cplx e = make_double2(0.0, 0.0), m = make_double2(0.0, 0.0);
+        #pragma unroll
             for (int o = 0; o < 5; ++o) {
                 const int col = r + 2 * (o - 2);
                 if (col < 0 || col >= dR) continue;
@@ -262,20 +381,24 @@ __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
             }
             c = cadd(e, cscale(m, -(dt * re * (kA[0] + kB[0]))));
         }
-        double f = sf[isb ? dR + r : r];
         // only the real part of the stage's forcing reaches the right-hand side
         // (channel/increadjproject0.c:130-141)
-        if (a.F) f += a.F[((size_t) (isb ? 1 : 0) * Nz * Mx) * dR + r].x;
+        if (a.F) f += fk.x;
         c.x += dt * kC[k] * f;
         const cplx dw = isb ? make_double2(wbt.x - wb.x, wbt.y - wb.y)
                             : make_double2(ubt.x - ub.x, ubt.y - ub.y);
-        c.x += a.mlift[r] * dw.x;
-        c.y += a.mlift[r] * dw.y;
+        c.x += ml * dw.x;
+        c.y += ml * dw.y;
     }
     __syncthreads();
     if (r < dR) (isb ? sbe : sal)[r] = c;
     __syncthreads();
-    if (tid < 4) chain_subst<2>(tid < 2 ? sal : sbe, a.Lm, 1, 0, dR, tid & 1);
+    // chains: alpha, beta (waves 0, 1), parity, part
+    if ((tid & 63) < 4 && tid < 128) {
+        const int pr = (tid >> 1) & 1, part = tid & 1;
+        const double *L = sfac + pr * nrp * 5, *U = L + nrp * 2, *D = U + nrp * 2;
+        chain_subst<2, 1>((double *) (tid < 64 ? sal : sbe) + 2 * pr + part, L, U, D, (dR - pr + 1) / 2);
+    }
     __syncthreads();
     // the mean's Gauss-point values sum all dimR coefficients
     for (int i = tid; i < dR; i += IA_THREADS) {
@@ -305,11 +428,6 @@ __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
         }
         return;
     }
-    __syncthreads();
-    stage(a.LIU, a.mic1);
-    __syncthreads();
-    project();
-    __syncthreads();
     if (r < dR) {
         const cplx *v = isb ? sbe : sal;
         cplx e = make_double2(0.0, 0.0), m = make_double2(0.0, 0.0);
@@ -317,12 +435,12 @@ __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
             const int col = r + 2 * (o - 2);
             if (col < 0 || col >= dR) continue;
             const double ex = g.s[o] - re * kA[k + 1] * dt * g.p[o];
-            const cplx vv = v[col], mv = smic[(isb ? dR : 0) + col];
+            const cplx vv = v[col], mv = smic[(isb ? 3 : 2) * dR + col];
             e.x += ex * vv.x; e.y += ex * vv.y;
             m.x += g.p[o] * mv.x; m.y += g.p[o] * mv.y;
         }
-        cplx gf = make_double2(sf[isb ? dR + r : r], 0.0);
-        if (a.F) gf = cadd(gf, a.F[((size_t) (2 + (isb ? 1 : 0)) * Nz * Mx) * dR + r]);
+        cplx gf = make_double2(fl, 0.0);
+        if (a.F) gf = cadd(gf, fn);
         const cplx c2 = cadd(cadd(e, cscale(gf, dt * kD[k + 1])),
                              cscale(m, -(dt * re * (kA[k + 1] + kB[k + 1]))));
         a.IAC[((size_t) (isb ? dR : 0) + r) * Mx] = c2;
@@ -332,6 +450,10 @@ __device__ void iadj_mean(const IadjArgs &a, cplx *sh)
 // Right-hand side, solve, wall values and next explicit part of the modes
 // (kx, kz) != (0, 0), kz row != Nz/2: IA_XG kx columns of one kz row per
 // block; the first block of the grid serves the mean mode (it runs longest).
+// Bound by latency and the FP64 band rows.  At 64x97x64 92 -> 51 us (modes alone
+// 72 -> 32, the mean alone 34 -> 32) with the factors requested at the start and the
+// chains fed from LDS, real and imaginary parts on lanes of their own, and the
+// band rows of alpha and beta in code of their own without a test per entry.
 __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
 {
     extern __shared__ double2 sh[];
@@ -356,15 +478,75 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
     }
     cplx *sal = sh;                          // [t][dR]
     cplx *sbe = sal + IA_XG * dR;            // [t][dR]
-    cplx *smic = sbe + IA_XG * dR;           // [t][2][dR]: MIC[count], then MIC[count - 1]
+    // MIC[count] for the right-hand sides, the factors for the solves, then
+    // MIC[count - 1]: [t][2][dR]
+    cplx *smic = sbe + IA_XG * dR;
     const double kz = a.Kz[z];
     auto valid = [&](int t) { return t < nx && !(z == 0 && x0 + t == 0); };
-    auto stage_mic = [&](const cplx *mic) {
-        for (int e = tid; e < 2 * dR * IA_XG; e += IA_THREADS) {
-            const int t = e % IA_XG, r = e / IA_XG;        // r over [2][dR]
-            if (t < nx) smic[t * 2 * dR + r] = mic[((size_t) z * 2 * dR + r) * Mx + x0 + t];
+    // MIC rows in registers, four values a thread (2 dR IA_XG <= 4 IA_THREADS)
+    v2d mv[4];
+    auto load_mic = [&](const cplx *mic) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = min(tid + i * IA_THREADS, 2 * dR * IA_XG - 1), r = e / IA_XG;     // r over [2][dR]
+            mv[i] = *(const v2d *) &mic[((size_t) z * 2 * dR + r) * Mx + x0 + min(e % IA_XG, nx - 1)];
         }
     };
+    auto put_mic = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = tid + i * IA_THREADS;
+            if (e < 2 * dR * IA_XG) smic[(e % IA_XG) * 2 * dR + e / IA_XG] = make_double2(mv[i].x, mv[i].y);
+        }
+    };
+    // The factors of the block's columns, eight rows of a parity at a time: a
+    // thread's role in a row is two L or two U values of one column or one
+    // inverse pivot (alpha: threads 0 .. 19 of 32, beta: the others).  They are
+    // requested here and put into LDS, [parity][L, U, D][row][t], once the
+    // right-hand sides no longer need it.
+    const int nrq = solve_rows(dQ), nrr = solve_rows(dR);
+    const int role = tid & 31, frow = tid >> 5;
+    const bool fb = role >= 20, fd = fb ? role >= 28 : role >= 16;         // beta, inverse pivot
+    const int fe = fb ? role - (fd ? 28 : role >= 24 ? 24 : 20) : role - (fd ? 16 : role >= 8 ? 8 : 0);
+    const int fdl = fb ? 2 : 4, frows = fb ? nrr : nrq, fsec = fd ? 2 : fb ? (role >= 24) : (role >= 8);
+    const int ft = fd || fb ? fe : fe >> 1, fm = fd || fb ? 0 : 2 * (fe & 1);
+    v2d fv[2][8];
+    {
+        const int zi = (a.mirror && z > Nz / 2) ? Nz - z : z;
+        const size_t col = (size_t) zi * Mx + x0 + min(ft, nx - 1), blk = col / a.sbt;
+        const int cc = (int) (col % a.sbt);
+        const size_t psize = (size_t) frows * a.sbt * (2 * fdl + 1);
+        const double *src = (fb ? a.Lb : a.La) + blk * 2 * psize + (size_t) fsec * frows * a.sbt * fdl +
+                            (fd ? cc : cc * fdl + fm);
+        const size_t rs = (size_t) a.sbt * (fd ? 1 : fdl);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int r = i * 8 + frow;
+                fv[p][i] = v2d{0.0, 0.0};
+                if (i * 8 < nrr && r < frows) {
+                    if (fd) fv[p][i].x = src[p * psize + r * rs];
+                    else fv[p][i] = *(const v2d *) (src + p * psize + r * rs);
+                }
+            }
+    }
+    double *fac = (double *) smic, *facb = fac + 2 * nrq * IA_XG * 9;
+    auto put_factors = [&]() {
+        double *dst = (fb ? facb : fac) + (size_t) fsec * frows * IA_XG * fdl + (fd ? ft : ft * fdl + fm);
+        const int psize = frows * IA_XG * (2 * fdl + 1), rs = IA_XG * (fd ? 1 : fdl);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int r = i * 8 + frow;
+                if (i * 8 < nrr && r < frows) {
+                    if (fd) dst[p * psize + r * rs] = fv[p][i].x;
+                    else *(v2d *) (dst + p * psize + r * rs) = fv[p][i];
+                }
+            }
+    };
+    if (k == 0) load_mic(a.mic0);
     for (int e = tid; e < dR * IA_XG; e += IA_THREADS) {
         const int i = e / IA_XG, t = e % IA_XG;
         if (t < nx) {
@@ -373,53 +555,17 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
             sbe[t * dR + i] = a.IAC[o + (size_t) dR * Mx];
         }
     }
-    if (k == 0) stage_mic(a.mic0);
+    if (k == 0) put_mic();
     __syncthreads();
     // right-hand sides: thread rows i (alpha: tid < 128, beta: tid >= 128)
     const bool isb = tid >= 128;
     const int i = isb ? tid - 128 : tid;
     const int N = isb ? dR : dQ;
-    const double dt = a.dt, re = a.re;
-    GramRow g;
     cplx acc[IA_XG];
-    if (i < N) {
-        load_gram(a, isb, i, N, g);
-#pragma unroll
-        for (int t = 0; t < IA_XG; ++t) {
-            acc[t] = make_double2(0.0, 0.0);
-            if (!valid(t)) continue;
-            const int x = x0 + t;
-            const double kx = a.Kx[x], k2 = kx * kx + kz * kz;
-            const cplx *v = (isb ? sbe : sal) + t * dR;
-            cplx c = v[i];
-            if (k == 0) {
-                cplx e, m;
-                band_pair(g, isb, i, N, k2, isb ? -re * kA[0] * dt : re * kA[0] * dt, v,
-                          smic + t * 2 * dR + (isb ? dR : 0), e, m);
-                c = cadd(e, cscale(m, re * dt * (kA[0] + kB[0])));
-            }
-            cplx gf = isb ? a.Fb[((size_t) z * dR + i) * Mx + x] : a.Fa[((size_t) z * dQ + i) * Mx + x];
-            if (a.F) gf = cadd(gf, a.F[((((size_t) 0 * 2 + (isb ? 1 : 0)) * Nz + z) * Mx + x) * dR + i]);
-            c = cadd(c, cscale(gf, dt * kC[k]));
-            const size_t wo = (size_t) z * Mx + x;
-            if (!isb && i < 8) {
-                const cplx wb = a.W[wp + wo], wbt = a.W[3 * wp + wo], awb = a.W[5 * wp + wo];
-                const double mm = kLR[i] / 2. - k2 * kLX[i], vv = -k2 * kLR[i] + k2 * k2 * kLX[i];
-                c.x += mm * (wbt.x - wb.x) + dt * re * (kA[k] * wbt.x + kB[k] * wb.x) * vv +
-                       dt * re * (kA[k] + kB[k]) * awb.x * vv;
-                c.y += mm * (wbt.y - wb.y) + dt * re * (kA[k] * wbt.y + kB[k] * wb.y) * vv +
-                       dt * re * (kA[k] + kB[k]) * awb.y * vv;
-            }
-            if (isb && i < 4) {
-                const cplx ub = a.W[wo], ubt = a.W[2 * wp + wo], aub = a.W[4 * wp + wo];
-                const double h = kLG[i] / 2.;
-                c.x += h * (ubt.x - ub.x) + dt * re * (kA[k] * ubt.x + kB[k] * ub.x) * (-k2 * h) +
-                       dt * re * (kA[k] + kB[k]) * aub.x * (-k2 * h);
-                c.y += h * (ubt.y - ub.y) + dt * re * (kA[k] * ubt.y + kB[k] * ub.y) * (-k2 * h) +
-                       dt * re * (kA[k] + kB[k]) * aub.y * (-k2 * h);
-            }
-            acc[t] = c;
-        }
+    if (isb) {
+        if (i < dR) mode_rhs<true>(a, i, z, x0, kz, sbe, smic, valid, acc);
+    } else {
+        if (i < dQ) mode_rhs<false>(a, i, z, x0, kz, sal, smic, valid, acc);
     }
     __syncthreads();
     if (i < N) {
@@ -427,23 +573,27 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
         for (int t = 0; t < IA_XG; ++t)
             if (valid(t)) (isb ? sbe : sal)[t * dR + i] = acc[t];
     }
-    if (k < 2) stage_mic(a.mic1);     // the rows of MIC[count] are no longer read
+    put_factors();                    // the rows of MIC[count] are no longer read
+    if (k < 2) load_mic(a.mic1);
     __syncthreads();
-    // implicit solves with the setup's factors: one parity chain per thread,
-    // neighbouring modes on neighbouring lanes (neighbouring image columns)
-    if (tid < 4 * IA_XG) {
-        const int kind = tid / IA_XG, t = tid % IA_XG;
+    // implicit solves: alpha chains on wave 0, beta chains on wave 1, one lane a
+    // parity, column and part
+    if ((tid & 63) < 4 * IA_XG && tid < 128) {
+        const int pr = (tid >> 3) & 1, t = (tid >> 1) & 3, part = tid & 1;
         if (valid(t)) {
-            const int zi = (a.mirror && z > Nz / 2) ? Nz - z : z;
-            const size_t col = (size_t) zi * Mx + x0 + t, blk = col / a.sbt;
-            const int cc = (int) (col % a.sbt);
-            if (kind < 2)
-                chain_subst<4>(sal + t * dR, a.La + blk * 2 * solve_rows(dQ) * 9 * a.sbt, a.sbt, cc, dQ, kind & 1);
-            else
-                chain_subst<2>(sbe + t * dR, a.Lb + blk * 2 * solve_rows(dR) * 5 * a.sbt, a.sbt, cc, dR, kind & 1);
+            if (tid < 64) {
+                const double *L = fac + pr * nrq * IA_XG * 9, *U = L + nrq * IA_XG * 4, *D = U + nrq * IA_XG * 4;
+                chain_subst<4, IA_XG>((double *) (sal + t * dR) + 2 * pr + part, L + 4 * t, U + 4 * t, D + t,
+                                      (dQ - pr + 1) / 2);
+            } else {
+                const double *L = facb + pr * nrr * IA_XG * 5, *U = L + nrr * IA_XG * 2, *D = U + nrr * IA_XG * 2;
+                chain_subst<2, IA_XG>((double *) (sbe + t * dR) + 2 * pr + part, L + 2 * t, U + 2 * t, D + t,
+                                      (dR - pr + 1) / 2);
+            }
         }
     }
     __syncthreads();
+    if (k < 2) put_mic();             // the factors are no longer read
     // solved coefficients for the y-transform: alpha rows beyond dimQ and
     // omega_y rows beyond dimQ cleared (channel/increadjproject.c:371-395 sum
     // the omega_y coefficients below dimQ)
@@ -500,23 +650,11 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
         }
         return;
     }
-    // the next stage's explicit part: projections of LIU, forcing k+1,
-    // MIC[count-1]
-    if (i < N) {
-#pragma unroll
-        for (int t = 0; t < IA_XG; ++t) {
-            if (!valid(t)) continue;
-            const int x = x0 + t;
-            const double kx = a.Kx[x], k2 = kx * kx + kz * kz;
-            cplx e, m;
-            band_pair(g, isb, i, N, k2, isb ? -re * kA[k + 1] * dt : re * kA[k + 1] * dt,
-                      (isb ? sbe : sal) + t * dR, smic + t * 2 * dR + (isb ? dR : 0), e, m);
-            cplx gf = isb ? a.FLb[((size_t) z * dR + i) * Mx + x] : a.FLa[((size_t) z * dQ + i) * Mx + x];
-            if (a.F) gf = cadd(gf, a.F[((((size_t) 1 * 2 + (isb ? 1 : 0)) * Nz + z) * Mx + x) * dR + i]);
-            const cplx c = cadd(cadd(e, cscale(gf, dt * kD[k + 1])),
-                                cscale(m, re * dt * (kA[k + 1] + kB[k + 1])));
-            a.IAC[((size_t) (z * 2 + (isb ? 1 : 0)) * dR + i) * Mx + x] = c;
-        }
+    __syncthreads();
+    if (isb) {
+        if (i < dR) mode_next<true>(a, i, z, x0, kz, sbe, smic, valid);
+    } else {
+        if (i < dQ) mode_next<false>(a, i, z, x0, kz, sal, smic, valid);
     }
 }
 
@@ -649,8 +787,12 @@ int launch_iadj(Context &c, int k, int count, cplx *IAC, const cplx *IU, const c
     a.re = d.re; a.dt = d.dt;
     a.La = c.dLa[1][k]; a.Lb = c.dLb[1][k]; a.Lm = c.dLm[1][k];
     a.sbt = c.sbt; a.mirror = c.factor_mirror ? 1 : 0;
-    const size_t lds_modes = sizeof(cplx) * 4 * IA_XG * (size_t) nR;
-    const size_t lds_mean = sizeof(cplx) * 4 * (size_t) nR + sizeof(double) * (4 * (size_t) q + 2 * (size_t) nR);
+    const size_t nrq = solve_rows(nQ), nrr = solve_rows(nR);
+    const size_t fac = sizeof(double) * 2 * IA_XG * (9 * nrq + 5 * nrr);
+    const size_t lds_modes = sizeof(cplx) * 2 * IA_XG * (size_t) nR +
+                             std::max(fac, sizeof(cplx) * 2 * IA_XG * (size_t) nR);
+    const size_t lds_mean = sizeof(cplx) * 6 * (size_t) nR +
+                            sizeof(double) * (8 * (size_t) q + 10 * nrr);
     const size_t lds = std::max(lds_modes, lds_mean);
     (void) hipFuncSetAttribute((const void *) k_iadj_modes, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int) lds);
