@@ -197,6 +197,9 @@ static void free_all(Context &c)
             if (c.dLm[a][k]) (void) hipFree(c.dLm[a][k]);
             if (c.dAdd[a][k]) (void) hipFree(c.dAdd[a][k]);
         }
+    if (c.pin) (void) hipHostFree(c.pin);
+    for (hipEvent_t e : c.pin_ev)
+        if (e) (void) hipEventDestroy(e);
     for (hipEvent_t e : c.ev_pool) (void) hipEventDestroy(e);
     for (auto &g : c.graphs) (void) hipGraphExecDestroy(g.exec);
     if (c.stream) (void) hipStreamDestroy(c.stream);
@@ -365,10 +368,132 @@ static void pass2_adjoint_pair(Context &c, const cplx *AUb, const cplx *wa, cons
     }
 }
 
-static int check_abort(Context &c, const char *what)
+// Host arrays pass through pinned memory of the context, a chunk at a time, the
+// host's copy of one chunk under the transfer of the others.  A pageable array of
+// 64 KB takes 34 us each way directly (the runtime pins it for the call) and 9 so;
+// 1 MB 60 to 140 us down, 40 so; the 5.4 MB of physical fields at 32x65x32 300 us
+// down, of which the link needs 101, 190 so (the host reads what the link has just
+// written at 35 GB/s; chunks of 512 KB end in 330 us instead of 275 to 300 for the call,
+// as every chunk costs a hand-over between queues, one chunk in 345).  The stop
+// flag costs 2 us behind a run's last kernel, 34 as a copy of its own.
+// Memory that the runtime knows (pinned, managed, a device's) is copied directly.
+static void alloc_pinned(Context &c)
 {
-    int flag = 0;
-    SC_HIP(hipMemcpy(&flag, c.abort_flag, sizeof(int), hipMemcpyDeviceToHost));
+    if (hipHostMalloc((void **) &c.pin, PIN_SLOTS * PIN_CHUNK + 4 * sizeof(int), 0) != hipSuccess) {
+        (void) hipGetLastError();
+        c.pin = nullptr;
+        return;
+    }
+    for (hipEvent_t &e : c.pin_ev)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            (void) hipGetLastError();
+            (void) hipHostFree(c.pin);
+            c.pin = nullptr;
+            return;
+        }
+}
+
+static bool through_pinned(const Context &c, const void *p)
+{
+    if (!c.pin) return false;
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void) hipGetLastError();                // not an address the runtime knows
+        return true;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
+static int wait_slot(Context &c, int s)
+{
+    if (c.pin_busy[s]) SC_HIP(hipEventSynchronize(c.pin_ev[s]));
+    c.pin_busy[s] = false;
+    return SC_OK;
+}
+
+// dst (device) <- src (host), in the order of the library's stream; src is free
+// on return where it went through pinned memory
+static int stage_in(Context &c, void *dst, const void *src, size_t n)
+{
+    if (!through_pinned(c, src)) {
+        SC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c.stream));
+        return SC_OK;
+    }
+    for (size_t o = 0; o < n; o += PIN_CHUNK) {
+        const size_t m = std::min(PIN_CHUNK, n - o);
+        const int s = c.pin_next++ % PIN_SLOTS;
+        char *slot = c.pin + s * PIN_CHUNK;
+        if (int rc = wait_slot(c, s)) return rc;
+        memcpy(slot, (const char *) src + o, m);
+        SC_HIP(hipMemcpyAsync((char *) dst + o, slot, m, hipMemcpyHostToDevice, c.stream));
+        SC_HIP(hipEventRecord(c.pin_ev[s], c.stream));
+        c.pin_busy[s] = true;
+    }
+    return SC_OK;
+}
+
+// dst (host) <- src (device) after the stream's work; dst is complete on return
+static int stage_out(Context &c, void *dst, const void *src, size_t n)
+{
+    if (!through_pinned(c, dst)) {
+        SC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c.stream));
+        SC_HIP(hipStreamSynchronize(c.stream));
+        return SC_OK;
+    }
+    const size_t nch = (n + PIN_CHUNK - 1) / PIN_CHUNK;
+    const unsigned base = c.pin_next;
+    auto len = [&](size_t i) { return std::min(PIN_CHUNK, n - i * PIN_CHUNK); };
+    for (size_t i = 0, put = 0; i < nch; ++i) {
+        // a slot is filled again once its chunk has been copied out (chunk put
+        // takes the slot of chunk put - PIN_SLOTS < i)
+        for (; put < nch && put < i + PIN_SLOTS; ++put) {
+            const int s = (base + put) % PIN_SLOTS;
+            SC_HIP(hipMemcpyAsync(c.pin + s * PIN_CHUNK, (const char *) src + put * PIN_CHUNK, len(put),
+                                  hipMemcpyDeviceToHost, c.stream));
+            SC_HIP(hipEventRecord(c.pin_ev[s], c.stream));
+            c.pin_busy[s] = true;
+        }
+        const int s = (base + i) % PIN_SLOTS;
+        if (int rc = wait_slot(c, s)) return rc;
+        memcpy((char *) dst + i * PIN_CHUNK, c.pin + s * PIN_CHUNK, len(i));
+    }
+    c.pin_next = base + (unsigned) nch;
+    return SC_OK;
+}
+
+// a run's input or output array, in host or device memory
+static int take(Context &c, void *dst, const void *src, size_t n, hipMemcpyKind kind)
+{
+    if (kind == hipMemcpyHostToDevice) return stage_in(c, dst, src, n);
+    SC_HIP(hipMemcpyAsync(dst, src, n, kind, c.stream));
+    return SC_OK;
+}
+
+static int stream_sync(Context &c)
+{
+    SC_HIP(hipStreamSynchronize(c.stream));
+    return 0;
+}
+
+// The end of a run: the result copied out where it stays on the device, the stop
+// flag fetched, the stream waited for.  flag[0], flag[1]: abort_flag's
+static int end_run(Context &c, void *out, const void *result, size_t n, hipMemcpyKind kind, int *flag)
+{
+    if (out && kind != hipMemcpyDeviceToHost) SC_HIP(hipMemcpyAsync(out, result, n, kind, c.stream));
+    int *host = c.pin ? (int *) (c.pin + PIN_SLOTS * PIN_CHUNK) : nullptr;
+    if (host && flag)
+        SC_HIP(hipMemcpyAsync(host, c.abort_flag, 2 * sizeof(int), hipMemcpyDeviceToHost, c.stream));
+    if (int rc = stream_sync(c)) return rc;
+    if (flag) {
+        if (host) memcpy(flag, host, 2 * sizeof(int));
+        else SC_HIP(hipMemcpy(flag, c.abort_flag, 2 * sizeof(int), hipMemcpyDeviceToHost));
+    }
+    return SC_OK;
+}
+
+// flag: abort_flag[0]
+static int check_abort(Context &c, const char *what, int flag)
+{
     if (flag) {
         int y = flag - 1;
         double m = 0.0;
@@ -450,11 +575,6 @@ static void host_gauss_to_coef(Context &c, const std::vector<cplx> &U, std::vect
     }
 }
 
-static int stream_sync(Context &c)
-{
-    SC_HIP(hipStreamSynchronize(c.stream));
-    return 0;
-}
 
 }  // namespace sc
 
@@ -760,6 +880,7 @@ int c_init(int Nx, int Ny, int Nz, double Lx, double Lz, double Re, double flux,
             c.wvalid.clear();
         }
     }
+    alloc_pinned(c);
     c.views.assign(nstep + 1, {});
     c.iviews.assign(nstep + 1, {});
     c.ok = true;
@@ -805,7 +926,7 @@ static int primal_run(int ru_steps, sc_complex *C_given, hipMemcpyKind in, hipMe
     const bool given = C_given != nullptr;
     const size_t cb = sizeof(cplx) * c.csize, cbm = cb * c.nrun;
     if (given) {
-        SC_HIP(hipMemcpyAsync(c.C, C_given, cbm, in, c.stream));
+        if (int rc = take(c, c.C, C_given, cbm, in)) return rc;
         launch_rebuild(c, c.C, c.U);
     } else {
         // laminar Poiseuille + rand() perturbation at Gauss points; C by
@@ -868,29 +989,29 @@ static int primal_run(int ru_steps, sc_complex *C_given, hipMemcpyKind in, hipMe
                 launch_rebuild(c, Cs, c.U);
             }
             if ((n & 63) == 63 && !capturing) {
-                int flag = 0;
-                SC_HIP(hipMemcpy(&flag, c.abort_flag, sizeof(int), hipMemcpyDeviceToHost));
-                if (flag) break;
+                int flag[2];
+                if (int rc = end_run(c, nullptr, nullptr, 0, in, flag)) return rc;
+                if (flag[0]) break;
             }
         }
         return SC_OK;
     });
-    if (!rc) rc = stream_sync(c);
+    int flag[2];
+    if (!rc) rc = end_run(c, given ? C_given : nullptr, c.C, cbm, out, flag);
     if (rc) return rc;
     // after an abort the queued launches did nothing: no cached field is
     // valid, and the states from the stopped step on were not written
-    if (check_abort(c, "Pass1")) {
+    if (check_abort(c, "Pass1", flag[0])) {
         std::fill(c.wvalid.begin(), c.wvalid.end(), 0);
         drop_graphs(c);
-        int slot = 1;
-        SC_HIP(hipMemcpy(&slot, c.abort_flag + 1, sizeof(int), hipMemcpyDeviceToHost));
+        const int slot = flag[1];
         const long last = 3L * d.nsteps;
         if (slot >= 1 && slot <= last)
             for (int m = 0; m < c.nrun; ++m)
                 SC_HIP(hipMemset((char *) mc(c, slot) + m * c.mcbytes, 0,
                                  cb * (size_t) (last - slot + 1)));
     }
-    if (given) SC_HIP(hipMemcpy(C_given, c.C, cbm, out));
+    if (given && out == hipMemcpyDeviceToHost) return stage_out(c, C_given, c.C, cbm);
     return SC_OK;
 }
 
@@ -931,7 +1052,7 @@ static int tangent_run(int start, int end, sc_complex *IC_given, unsigned inhomo
 {
     Context &c = ctx();
     const size_t cbm = sizeof(cplx) * c.csize * c.nrun;
-    SC_HIP(hipMemcpyAsync(c.IC, IC_given, cbm, in, c.stream));
+    if (int rc = take(c, c.IC, IC_given, cbm, in)) return rc;
     if (int rc = copy_to_slots(c, c.MIC, 3L * start, c.IC)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     // each CFL check clears the maxima it read; a run starts from zero
@@ -979,18 +1100,18 @@ static int tangent_run(int start, int end, sc_complex *IC_given, unsigned inhomo
                     launch_zero(c, member_at(c, c.IU, m), mstride_bytes(c, c.IU) / sizeof(cplx));
                 }
         if (((n - start) & 63) == 63 && !capturing) {
-            int flag = 0;
-            SC_HIP(hipMemcpy(&flag, c.abort_flag, sizeof(int), hipMemcpyDeviceToHost));
-            if (flag) break;
+            int flag[2];
+            if (int rc = end_run(c, nullptr, nullptr, 0, in, flag)) return rc;
+            if (flag[0]) break;
         }
     }
     return SC_OK;
     });
-    if (!rc) rc = stream_sync(c);
+    int flag[2];
+    if (!rc) rc = end_run(c, IC_given, c.IC, cbm, out, flag);
     if (rc) return rc;
-    check_abort(c, "Pass1");
-    SC_HIP(hipMemcpy(IC_given, c.IC, cbm, out));
-    return SC_OK;
+    check_abort(c, "Pass1", flag[0]);
+    return out == hipMemcpyDeviceToHost ? stage_out(c, IC_given, c.IC, cbm) : SC_OK;
 }
 
 extern "C" int sc_tangent_sources(int start, int end, sc_complex *IC, int inhomo, int re_source)
@@ -1109,7 +1230,7 @@ static int adjoint_run(int start, int end, sc_complex *AC_given, double strength
     Context &c = ctx();
     const Dims &d = c.d;
     const size_t cbm = sizeof(cplx) * c.csize * c.nrun;
-    SC_HIP(hipMemcpyAsync(c.AC, AC_given, cbm, in, c.stream));
+    if (int rc = take(c, c.AC, AC_given, cbm, in)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     // member windows: a member whose window ends before `start` waits at
     // zero and takes its given state at its window's end
@@ -1139,10 +1260,9 @@ static int adjoint_run(int start, int end, sc_complex *AC_given, double strength
         if (windows) zero_pending(c, end + 1);   // never started: win <= end
         return SC_OK;
     });
-    if (!rc) rc = stream_sync(c);
+    if (!rc) rc = end_run(c, AC_given, c.AC, cbm, out, nullptr);
     if (rc) return rc;
-    SC_HIP(hipMemcpy(AC_given, c.AC, cbm, out));
-    return SC_OK;
+    return out == hipMemcpyDeviceToHost ? stage_out(c, AC_given, c.AC, cbm) : SC_OK;
 }
 
 // The adjoint of J = weight sum_{m = end}^{start-1} tau(C_m), tau the lower
@@ -1156,7 +1276,7 @@ static int adjoint_objective_run(int start, int end, sc_complex *AC_given, doubl
 {
     Context &c = ctx();
     const size_t cbm = sizeof(cplx) * c.csize * c.nrun;
-    SC_HIP(hipMemcpyAsync(c.AC, AC_given, cbm, in, c.stream));
+    if (int rc = take(c, c.AC, AC_given, cbm, in)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     // member windows: a member waits at zero until its window's end
     const bool windows = windowed(c);
@@ -1172,10 +1292,8 @@ static int adjoint_objective_run(int start, int end, sc_complex *AC_given, doubl
         launch_add_mean(c, c.AC, c.dGwall, weight);
     }
     if (windows) zero_pending(c, end + 1);   // never started: win <= end
-    int rc = stream_sync(c);
-    if (rc) return rc;
-    SC_HIP(hipMemcpy(AC_given, c.AC, cbm, out));
-    return SC_OK;
+    if (int rc = end_run(c, AC_given, c.AC, cbm, out, nullptr)) return rc;
+    return out == hipMemcpyDeviceToHost ? stage_out(c, AC_given, c.AC, cbm) : SC_OK;
 }
 
 extern "C" {
@@ -1221,17 +1339,15 @@ double c_ddt_project(int i_step, sc_complex *IC_given, int Nz_dup, int Nvar_dup,
         return NAN;
     }
     const size_t cb = sizeof(cplx) * c.csize;
-    if (hipMemcpyAsync(c.Ctmp, IC_given, cb, hipMemcpyHostToDevice, c.stream) != hipSuccess ||
+    if (stage_in(c, c.Ctmp, IC_given, cb) != SC_OK ||
         hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream) != hipSuccess) {
         last_error() = "ddt_project: HIP transfer failed";
         return NAN;
     }
     if (ddt_project_dev(c, i_step, c.Ctmp, c.Ctmp) != SC_OK) return NAN;
     double scal[3] = {0, 0, 0};
-    if (hipMemcpyAsync(IC_given, c.Ctmp, cb, hipMemcpyDeviceToHost, c.stream) != hipSuccess) return NAN;
-    if (hipMemcpyAsync(scal, c.scal, sizeof(scal), hipMemcpyDeviceToHost, c.stream) != hipSuccess) return NAN;
-    if (hipStreamSynchronize(c.stream) != hipSuccess) {
-        last_error() = "ddt_project: HIP synchronisation failed";
+    if (stage_out(c, IC_given, c.Ctmp, cb) != SC_OK || stage_out(c, scal, c.scal, sizeof(scal)) != SC_OK) {
+        last_error() = "ddt_project: HIP transfer failed";
         return NAN;
     }
     return scal[2];
@@ -1248,8 +1364,7 @@ static int get_view(int i_step, bool incre, sc_complex **ptr, int *Nz, int *Nvar
     auto &v = incre ? c.iviews[i_step] : c.views[i_step];
     v.resize(c.csize);
     const cplx *src = incre ? mic(c, 3L * i_step) : mc(c, 3L * i_step);
-    SC_HIP(hipStreamSynchronize(c.stream));
-    SC_HIP(hipMemcpy(v.data(), src, sizeof(cplx) * c.csize, hipMemcpyDeviceToHost));
+    if (int rc = stage_out(c, v.data(), src, sizeof(cplx) * c.csize)) return rc;
     *ptr = (sc_complex *) v.data();
     *Nz = c.d.Nz;
     *Nvar = 2;
@@ -1280,7 +1395,7 @@ int c_spec2phys(sc_complex *C_ptr, int Nz_dup, int Nvar_dup, int Ny_dup, int Nx_
         last_error() = "spec2phys: flow must be (3, 3Nx/2, qpts, 3Nz/2)";
         return SC_EINVAL;
     }
-    SC_HIP(hipMemcpyAsync(c.Ctmp, C_ptr, sizeof(cplx) * c.csize, hipMemcpyHostToDevice, c.stream));
+    if (int rc = stage_in(c, c.Ctmp, C_ptr, sizeof(cplx) * c.csize)) return rc;
     SC_HIP(hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream));
     c.fp64_out = true;                          // an output: FP64 transforms
     launch_rebuild(c, c.Ctmp, c.Ut, true);    // spec2phys reads u, v, w only
@@ -1295,10 +1410,7 @@ int c_spec2phys(sc_complex *C_ptr, int Nz_dup, int Nvar_dup, int Ny_dup, int Nx_
     // physical fields in FP64 whatever the precision of the time steps
     fp64::launch_zinv(c, fs, c.W1);
     fp64::launch_xmix(c, XM_PHYS, c.W1, nullptr, 0, c.flowdev, nullptr, 0);
-    SC_HIP(hipMemcpyAsync(flow_ptr, c.flowdev, sizeof(double) * 3 * (size_t) d.Px * d.qpts * d.Pz,
-                          hipMemcpyDeviceToHost, c.stream));
-    SC_HIP(hipStreamSynchronize(c.stream));
-    return SC_OK;
+    return stage_out(c, flow_ptr, c.flowdev, sizeof(double) * 3 * (size_t) d.Px * d.qpts * d.Pz);
 }
 
 // save_solution / read_solution (channel/channel.c:791-1028) in the
@@ -1363,10 +1475,10 @@ int sc_tangent_forcing(int count, sc_complex *f_a, sc_complex *f_b, sc_complex *
     int rc = stream_sync(c);
     if (rc) return rc;
     const size_t na = (size_t) d.Nz * d.dimQ * d.Mx, nb = (size_t) d.Nz * d.dimR * d.Mx;
-    SC_HIP(hipMemcpy(f_a, c.Fa, sizeof(cplx) * na, hipMemcpyDeviceToHost));
-    SC_HIP(hipMemcpy(f_b, c.Fb, sizeof(cplx) * nb, hipMemcpyDeviceToHost));
-    SC_HIP(hipMemcpy(f0_a, c.Ctmp2, sizeof(cplx) * d.dimR, hipMemcpyDeviceToHost));
-    SC_HIP(hipMemcpy(f0_b, c.Ctmp2 + d.dimR, sizeof(cplx) * d.dimR, hipMemcpyDeviceToHost));
+    if (int rc = stage_out(c, f_a, c.Fa, sizeof(cplx) * na)) return rc;
+    if (int rc = stage_out(c, f_b, c.Fb, sizeof(cplx) * nb)) return rc;
+    if (int rc = stage_out(c, f0_a, c.Ctmp2, sizeof(cplx) * d.dimR)) return rc;
+    if (int rc = stage_out(c, f0_b, c.Ctmp2 + d.dimR, sizeof(cplx) * d.dimR)) return rc;
     return SC_OK;
 }
 
@@ -1380,10 +1492,10 @@ int sc_wall_plane(const sc_complex *C_ptr, sc_complex *Uxb, sc_complex *Uzb)
     }
     const Dims &d = c.d;
     const size_t np = (size_t) d.Nz * d.Mx;
-    SC_HIP(hipMemcpyAsync(c.Ctmp, C_ptr, sizeof(cplx) * c.csize, hipMemcpyHostToDevice, c.stream));
+    if (int rc = stage_in(c, c.Ctmp, C_ptr, sizeof(cplx) * c.csize)) return rc;
     launch_wall_plane(c, c.Ctmp, c.Ctmp2, c.Ctmp2 + np);
-    SC_HIP(hipMemcpyAsync(Uxb, c.Ctmp2, sizeof(cplx) * np, hipMemcpyDeviceToHost, c.stream));
-    SC_HIP(hipMemcpyAsync(Uzb, c.Ctmp2 + np, sizeof(cplx) * np, hipMemcpyDeviceToHost, c.stream));
+    if (int rc = stage_out(c, Uxb, c.Ctmp2, sizeof(cplx) * np)) return rc;
+    if (int rc = stage_out(c, Uzb, c.Ctmp2 + np, sizeof(cplx) * np)) return rc;
     return stream_sync(c);
 }
 
@@ -1398,11 +1510,11 @@ int sc_incre_boundary(sc_complex *Uxb, sc_complex *Uzb)
     }
     const size_t np = (size_t) d.Nz * d.Mx;
     // planes in Ctmp2 (2 Nz Mx <= one coefficient array), transforms in W1
-    SC_HIP(hipMemcpyAsync(c.Ctmp2, Uxb, sizeof(cplx) * np, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(c.Ctmp2 + np, Uzb, sizeof(cplx) * np, hipMemcpyHostToDevice, c.stream));
+    if (int rc = stage_in(c, c.Ctmp2, Uxb, sizeof(cplx) * np)) return rc;
+    if (int rc = stage_in(c, c.Ctmp2 + np, Uzb, sizeof(cplx) * np)) return rc;
     launch_incre_boundary(c, c.Ctmp2, c.Ctmp2 + np, c.W1);
-    SC_HIP(hipMemcpyAsync(Uxb, c.Ctmp2, sizeof(cplx) * np, hipMemcpyDeviceToHost, c.stream));
-    SC_HIP(hipMemcpyAsync(Uzb, c.Ctmp2 + np, sizeof(cplx) * np, hipMemcpyDeviceToHost, c.stream));
+    if (int rc = stage_out(c, Uxb, c.Ctmp2, sizeof(cplx) * np)) return rc;
+    if (int rc = stage_out(c, Uzb, c.Ctmp2 + np, sizeof(cplx) * np)) return rc;
     return stream_sync(c);
 }
 
@@ -1423,10 +1535,10 @@ int sc_pass2_incremental(const sc_complex *U, const sc_complex *IU, const sc_com
     }
     cplx *bU = c.p2ibuf, *bIU = bU + us, *bAU = bIU + us, *bIAU = bAU + us, *T1 = bIAU + us,
          *T2 = T1 + us;
-    SC_HIP(hipMemcpyAsync(bU, U, sizeof(cplx) * us, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(bIU, IU, sizeof(cplx) * us, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(bAU, AU, sizeof(cplx) * us, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(bIAU, IAU, sizeof(cplx) * us, hipMemcpyHostToDevice, c.stream));
+    if (int rc = stage_in(c, bU, U, sizeof(cplx) * us)) return rc;
+    if (int rc = stage_in(c, bIU, IU, sizeof(cplx) * us)) return rc;
+    if (int rc = stage_in(c, bAU, AU, sizeof(cplx) * us)) return rc;
+    if (int rc = stage_in(c, bIAU, IAU, sizeof(cplx) * us)) return rc;
     // bilinear in (state, lambda): the adjoint operator of (u, I lambda)
     // plus that of (Iu, lambda), in FP64 whatever the context's precision
     const bool mixed = c.mixed;
@@ -1435,7 +1547,7 @@ int sc_pass2_incremental(const sc_complex *U, const sc_complex *IU, const sc_com
     pass2_adjoint(c, bIU, bAU, T2);
     launch_gauss_sum(c, T1, T2);
     c.mixed = mixed;
-    SC_HIP(hipMemcpyAsync(IH, T1, sizeof(cplx) * us, hipMemcpyDeviceToHost, c.stream));
+    if (int rc = stage_out(c, IH, T1, sizeof(cplx) * us)) return rc;
     return stream_sync(c);
 }
 
@@ -1460,20 +1572,20 @@ int sc_increadjproject(int k, int count, sc_complex *IAC, const sc_complex *IU,
     const size_t np = (size_t) d.Nz * d.Mx, nf = 4 * np * d.dimR;
     cplx *bIAC = c.iadjbuf, *bIU = bIAC + c.csize, *bLIU = bIU + c.usize, *bIAU = bLIU + c.usize;
     cplx *bW = bIAU + c.usize, *bF = bW + 6 * np, *bIAUb = bF + nf;
-    SC_HIP(hipMemcpyAsync(bIAC, IAC, sizeof(cplx) * c.csize, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(bIU, IU, sizeof(cplx) * c.usize, hipMemcpyHostToDevice, c.stream));
+    if (int rc = stage_in(c, bIAC, IAC, sizeof(cplx) * c.csize)) return rc;
+    if (int rc = stage_in(c, bIU, IU, sizeof(cplx) * c.usize)) return rc;
     if (k < 2)
-        SC_HIP(hipMemcpyAsync(bLIU, LIU, sizeof(cplx) * c.usize, hipMemcpyHostToDevice, c.stream));
-    SC_HIP(hipMemcpyAsync(bW, walls, sizeof(cplx) * 6 * np, hipMemcpyHostToDevice, c.stream));
+        if (int rc = stage_in(c, bLIU, LIU, sizeof(cplx) * c.usize)) return rc;
+    if (int rc = stage_in(c, bW, walls, sizeof(cplx) * 6 * np)) return rc;
     if (force)
-        SC_HIP(hipMemcpyAsync(bF, force, sizeof(cplx) * nf, hipMemcpyHostToDevice, c.stream));
+        if (int rc = stage_in(c, bF, force, sizeof(cplx) * nf)) return rc;
     if (launch_iadj(c, k, count, bIAC, bIU, bLIU, bW, force ? bF : nullptr, bIAU, bIAUb)) {
         last_error() = "increadjproject: launch failed";
         return SC_EINIT;
     }
-    SC_HIP(hipMemcpyAsync(IAC, bIAC, sizeof(cplx) * c.csize, hipMemcpyDeviceToHost, c.stream));
-    SC_HIP(hipMemcpyAsync(IAU, bIAU, sizeof(cplx) * c.usize, hipMemcpyDeviceToHost, c.stream));
-    SC_HIP(hipMemcpyAsync(IAUb, bIAUb, sizeof(cplx) * 2 * np, hipMemcpyDeviceToHost, c.stream));
+    if (int rc = stage_out(c, IAC, bIAC, sizeof(cplx) * c.csize)) return rc;
+    if (int rc = stage_out(c, IAU, bIAU, sizeof(cplx) * c.usize)) return rc;
+    if (int rc = stage_out(c, IAUb, bIAUb, sizeof(cplx) * 2 * np)) return rc;
     return stream_sync(c);
 }
 
@@ -1613,8 +1725,7 @@ int sc_member_state(int incre, int member, int i_step, sc_complex *out)
     }
     const char *src = (const char *) ((incre ? c.MIC : c.MC) + 3 * c.csize * (size_t) i_step) +
                       (size_t) member * c.mcbytes;
-    SC_HIP(hipStreamSynchronize(c.stream));
-    SC_HIP(hipMemcpy(out, src, sizeof(cplx) * c.csize, hipMemcpyDeviceToHost));
+    if (int rc = stage_out(c, out, src, sizeof(cplx) * c.csize)) return rc;
     return SC_OK;
 }
 
@@ -1685,7 +1796,7 @@ double sc_member_ddt_project(int member, int i_step, sc_complex *v)
         P = (const cplx *) ((const char *) mc(c, 0) + (size_t) member * c.mcbytes);
         M = c.Cprev + (size_t) member * c.csize;
     }
-    if (hipMemcpyAsync(c.Ctmp, v, cb, hipMemcpyHostToDevice, c.stream) != hipSuccess ||
+    if (stage_in(c, c.Ctmp, v, cb) != SC_OK ||
         hipMemsetAsync(c.abort_flag, 0, sizeof(int), c.stream) != hipSuccess) {
         last_error() = "member_ddt_project: HIP transfer failed";
         return NAN;
@@ -1694,9 +1805,7 @@ double sc_member_ddt_project(int member, int i_step, sc_complex *v)
     if (nparts <= 0) return NAN;
     launch_ddt_apply(c, c.Ctmp, c.Ctmp, P, M, 1.0 / c.d.dt, c.csize, nullptr, 0.0, nparts, 0);
     double scal[3] = {0, 0, 0};
-    if (hipMemcpyAsync(v, c.Ctmp, cb, hipMemcpyDeviceToHost, c.stream) != hipSuccess ||
-        hipMemcpyAsync(scal, c.scal, sizeof(scal), hipMemcpyDeviceToHost, c.stream) != hipSuccess ||
-        hipStreamSynchronize(c.stream) != hipSuccess) {
+    if (stage_out(c, v, c.Ctmp, cb) != SC_OK || stage_out(c, scal, c.scal, sizeof(scal)) != SC_OK) {
         last_error() = "member_ddt_project: HIP transfer failed";
         return NAN;
     }

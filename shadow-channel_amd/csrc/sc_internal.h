@@ -27,6 +27,9 @@ typedef double2 cplx;
 // launch update them with atomics (145 planes in 10 lines: 4 us of the primal x
 // kernel's 27 at 64x64x97)
 constexpr int CFL_STRIDE = 16;
+// host arrays: chunks of pinned memory (see stage_in)
+constexpr int PIN_SLOTS = 4;
+constexpr size_t PIN_CHUNK = 1024 * 1024;
 constexpr int MAXF = 12;        // fields in one z-inverse launch
 constexpr int FFT_TILE = 2048;  // complex values (data + twiddles) in one transform block
 constexpr int FFT_BLOCK = 256;  // threads of a transform block
@@ -204,6 +207,12 @@ struct Context {
     // [0] CFL stop (1 + plane), [1] first unwritten slot, [3] always zero
     // (never written)
     int *abort_flag = nullptr;
+    // pinned host memory: PIN_SLOTS chunks that host arrays pass through, then
+    // the host's copy of abort_flag; null when it could not be allocated
+    char *pin = nullptr;
+    hipEvent_t pin_ev[PIN_SLOTS] = {};          // end of a chunk's transfer
+    bool pin_busy[PIN_SLOTS] = {};
+    unsigned pin_next = 0;
     double *objscr = nullptr;                   // objectives and statistics (objective_scratch_doubles)
     double *dRwall = nullptr;                   // [2][dimR]: R_j'(-1), R_j'(+1)
     // incremental adjoint stage (sc_increadjproject): transposed bases and
