@@ -309,6 +309,32 @@ __device__ __forceinline__ void fft_first(real2 *data, real sign, LD ld)
     }
 }
 
+// The same with the inputs in the memory that the outputs take: they wait in
+// registers for the block's barrier.
+template <int START, int N, int NSEQ, int SSTR, int ESTR, int T, class LD>
+__device__ __forceinline__ void fft_first_in_place(real2 *data, real sign, LD ld)
+{
+    constexpr int R = plan_radix(N, 0), NBS = N / R, TOTAL = NSEQ * NBS;
+    constexpr int NBT = (TOTAL + T - 1) / T;
+    real2 v[NBT][R];
+#pragma unroll
+    for (int i = 0; i < NBT; ++i) {
+        const int b = threadIdx.x + i * T, j = b / NSEQ, s = b - j * NSEQ;
+        if (TOTAL % T == 0 || b < TOTAL) ld(j, s, v[i]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NBT; ++i) {
+        const int b = threadIdx.x + i * T, j = b / NSEQ, s = b - j * NSEQ;
+        if (TOTAL % T == 0 || b < TOTAL) {
+            dft<R, START>(v[i], sign);
+            real2 *dst = data + s * SSTR + j * R * ESTR;
+#pragma unroll
+            for (int q = 0; q < R; ++q) dst[q * ESTR] = v[i][q];
+        }
+    }
+}
+
 // inputs of butterfly j of sequence src, twiddled, and their DFT
 template <int R, int N, int NS, int ESTR, int START = DS_ANY>
 __device__ __forceinline__ void fft_butterfly(const real2 *src, int j, int k, const real2 *tw,

@@ -62,6 +62,21 @@ constexpr XrowShape xrow_shape(int px, int nseq, int nso)
     return best;
 }
 
+// Whether the fields' bins come into LDS first, row by row as they lie in memory
+// (the first pass wants each bin twice, directly and mirrored, and a lane its own
+// sequence): lengths whose rows of Mx bins lie a multiple of 64 bytes apart, which
+// crowd the L1 when lanes read them side by side, as far as the two barriers and
+// the LDS traffic cost less.  FP32, direct / staged in us (64x97x64, 32 members):
+// primal 404 / 371, tangent 697 / 602, adjoint 628 / 562, merged adjoint 950 / 978;
+// 128x129x128, two members: merged adjoint 397 / 308, adjoint 235 / 207, primal 132 /
+// 137; other lengths within 3% either way.  FP64 at 48: primal 9.8 / 8.7, tangent
+// 12.5 / 10.8, merged adjoint 34.9 / 36.4; at 96 23.9 / 25.0 and 51.5 / 58.2.
+constexpr bool xrow_staged(int mode, int px)
+{
+    if (sizeof(real) == 4) return px == 24 || (px % 48 == 0 && (mode != XM_ADJ2 || px != 96));
+    return (px == 24 || px == 48) && (mode == XM_PRIMAL || mode == XM_TANGENT);
+}
+
 template <int MODE, int PX> struct XrowPlan {
     static constexpr int NF = XmixShape<MODE>::NF, NOUT = XmixShape<MODE>::NOUT;
     static constexpr int NSEQ = (NF + 1) / 2, NSO = (NOUT + 1) / 2;
@@ -100,19 +115,10 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
     auto plane = [&](int r) { return z0 + r >= Pz ? y0 + 1 : y0; };
     auto zrow = [&](int r) { return z0 + r >= Pz ? z0 + r - Pz : z0 + r; };
     stage_twiddles_c<PX, T>(a.tw, twl);
-    // Load stage = first inverse pass: bin n < Mx takes X[n] + i Y[n], bin
-    // n > Px - Mx the conjugates at Px - n, the bins between are zero (c2r
-    // uses Re only at kx = 0).  Groups of bins in the zero band are not loaded.
-    fft_first<DS_ANY, PX, ROWS * NSEQ, SP, 1, T>(lds, +1.0, [&](int j, int t, real2 *v) {
-        const int r = t / NSEQ, s2 = 2 * (t - r * NSEQ), rr = min(r, nr - 1);
-        const int nf1 = a.nf1, nf2 = MODE == XM_ADJ2 ? a.nf2 : NF;
-        const int src = s2 < nf1 ? 0 : s2 < nf2 ? 1 : 2;
-        const int f0 = src == 0 ? 0 : src == 1 ? nf1 : nf2;
-        const int fn = src == 0 ? nf1 : src == 1 ? nf2 - nf1 : NF - nf2;
-        const real2 *B = src == 0 ? W1 : src == 1 ? a.W1b : a.W1c;
-        const real2 *X = B + ((size_t) plane(rr) * fn + (s2 - f0)) * PM + zrow(rr) * MX;
-        const bool hasy = NF % 2 == 0 || s2 + 1 < NF;
-        const real2 *Y = X + (hasy ? PM : 0);
+    // First inverse pass, the load stage: bin n < Mx takes X[n] + i Y[n], bin
+    // n > Px - Mx the conjugates at Px - n, the bins between are zero (c2r uses Re
+    // only at kx = 0).  Groups of bins in the zero band are not read.
+    auto bins = [&](int j, bool hasy, const real2 *X, const real2 *Y, real2 *v) {
         const real2 *Xd = X + j, *Yd = Y + j;            // direct bins
         const real2 *Xm = X - j, *Ym = Y - j;            // mirrored ones: Px - n = Px - q NB1 - j
 #pragma unroll
@@ -144,7 +150,51 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
             else if (n > PX - MX)
                 v[q] = mk2(xv.x + yv.y, -xv.y + yv.x);
         }
-    });
+    };
+    const int nf1 = a.nf1, nf2 = MODE == XM_ADJ2 ? a.nf2 : NF;
+    // field f of row r in its input array
+    auto field = [&](int f, int r) {
+        const int src = f < nf1 ? 0 : f < nf2 ? 1 : 2;
+        const int f0 = src == 0 ? 0 : src == 1 ? nf1 : nf2;
+        const int fn = src == 0 ? nf1 : src == 1 ? nf2 - nf1 : NF - nf2;
+        const real2 *B = src == 0 ? W1 : src == 1 ? a.W1b : a.W1c;
+        return B + ((size_t) plane(r) * fn + (f - f0)) * PM + zrow(r) * MX;
+    };
+    if constexpr (xrow_staged(MODE, PX)) {
+        // field f of row r at (r NF + f) SB (odd: as SP), inside the sequences' tile
+        constexpr int SB = MX | 1, NIN = NF * ROWS * MX, NLD = (NIN + T - 1) / T;
+        static_assert(NF * SB <= NSEQ * SP, "the bins fit the tile");
+        real bx[NLD], by[NLD];                           // (an array of real2 would go to scratch)
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int e = min((int) threadIdx.x + i * T, NIN - 1);
+            const int f = e / (ROWS * MX), rk = e - f * (ROWS * MX), r = rk / MX, k = rk - r * MX;
+            const real2 *B = field(f, min(r, nr - 1)) + k;
+            bx[i] = B->x;
+            by[i] = B->y;
+        }
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int e = threadIdx.x + i * T;
+            if (NIN % T != 0 && e >= NIN) break;
+            const int f = e / (ROWS * MX), rk = e - f * (ROWS * MX), r = rk / MX, k = rk - r * MX;
+            lds[(r * NF + f) * SB + k] = mk2(bx[i], by[i]);
+        }
+        __syncthreads();
+        fft_first_in_place<DS_ANY, PX, ROWS * NSEQ, SP, 1, T>(lds, +1.0, [&](int j, int t, real2 *v) {
+            const int r = t / NSEQ, s2 = 2 * (t - r * NSEQ);
+            const bool hasy = NF % 2 == 0 || s2 + 1 < NF;
+            const real2 *X = lds + (r * NF + s2) * SB;
+            bins(j, hasy, X, X + (hasy ? SB : 0), v);
+        });
+    } else {
+        fft_first<DS_ANY, PX, ROWS * NSEQ, SP, 1, T>(lds, +1.0, [&](int j, int t, real2 *v) {
+            const int r = t / NSEQ, s2 = 2 * (t - r * NSEQ);
+            const bool hasy = NF % 2 == 0 || s2 + 1 < NF;
+            const real2 *X = field(s2, min(r, nr - 1));
+            bins(j, hasy, X, X + (hasy ? PM : 0), v);
+        });
+    }
     __syncthreads();
     lds_fft_c<PX, ROWS * NSEQ, SP, 1, T, NP, 1, R1>(lds, twl, +1.0);
     // products: every field of a point read, then (after a barrier) the packed
