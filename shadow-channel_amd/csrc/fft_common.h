@@ -431,6 +431,7 @@ struct ZinvArgs {
 
 struct XmixArgs {
     int mode, nf, nout, Mx, Px, Pz, qpts, ZB, check_cfl;
+    int nm;                    // members (k_xrow_shared)
     const double2 *tw;
     int nf1;                   // fields 0..nf1-1 from the first source, the rest from W1b
     const real2 *W1b;
@@ -595,6 +596,8 @@ template <class K> struct Fixed {
     size_t lds = 0;            // bytes
 };
 template <int MODE> Fixed<XrowKernel> xrow_fixed(int Px, int Pz);
+// nm tangent members along one trajectory (fft_x.hip, k_xrow_shared)
+Fixed<XrowKernel> xrow_shared_fixed(int Px, int Pz, int nm);
 Fixed<ZinvKernel> zinv_fixed(int Pz, int Mx, bool s32);
 Fixed<ZfwdKernel> zfwd_fixed(int Pz, int Mx);
 Fixed<ZadjKernel> zadj_fixed(int Pz, int Mx);

@@ -716,7 +716,17 @@ void launch_xmix(Context &c, int mode, const cplx *W1, cplx *W2, int check_cfl,
     XmixArgs ar = a;
     ar.check_cfl = 0;
     std::function<void()> go, again;
-    if (const auto fx = xrow_kernel(mode, d); fx.kernel) {
+    a.nm = ar.nm = nm;
+    Fixed<XrowKernel> shared;
+    if (mode == XM_TANGENT && W1b && nf1 == 6 && a.ms_in == 0) shared = xrow_shared_fixed(d.Px, d.Pz, nm);
+    if (shared.kernel) {
+        // members along one trajectory: all of them in a block, unless that leaves
+        // fewer than four blocks a CU
+        const int blocks = (d.qpts * d.Pz + shared.group - 1) / shared.group;
+        const dim3 grid(blocks, std::max(1, std::min(nm, 1024 / blocks)));
+        go = [=]() { hipLaunchKernelGGL(shared.kernel, grid, dim3(shared.threads), shared.lds, st, a, W1r, W2r); };
+        again = [=]() { hipLaunchKernelGGL(shared.kernel, grid, dim3(shared.threads), shared.lds, st, ar, W1r, W2r); };
+    } else if (const auto fx = xrow_kernel(mode, d); fx.kernel) {
         const dim3 grid((d.qpts * d.Pz + fx.group - 1) / fx.group, nm);
         go = [=]() { hipLaunchKernelGGL(fx.kernel, grid, dim3(fx.threads), fx.lds, st, a, W1r, W2r); };
         again = [=]() { hipLaunchKernelGGL(fx.kernel, grid, dim3(fx.threads), fx.lds, st, ar, W1r, W2r); };

@@ -85,6 +85,46 @@ template <int MODE, int PX> struct XrowPlan {
     static constexpr size_t LDS = sizeof(real2) * ((size_t) ROWS * NSEQ * SP + PX);
 };
 
+// First inverse pass, the inputs of butterfly j: bin n < Mx takes X[n] + i Y[n],
+// bin n > Px - Mx the conjugates at Px - n, the bins between are zero (c2r uses Re
+// only at kx = 0).  Groups of bins in the zero band are not read.
+template <int PX>
+__device__ __forceinline__ void row_bins(int j, bool hasy, const real2 *X, const real2 *Y, real2 *v)
+{
+    constexpr int MX = PX / 3, R1 = plan_radix(PX, 0), NB1 = PX / R1;
+    const real2 *Xd = X + j, *Yd = Y + j;            // direct bins
+    const real2 *Xm = X - j, *Ym = Y - j;            // mirrored ones: Px - n = Px - q NB1 - j
+#pragma unroll
+    for (int q = 0; q < R1; ++q) {
+        const int lo = q * NB1, hi = lo + NB1 - 1, n = j + lo;
+        v[q] = mk2(0.0, 0.0);
+        if (lo >= MX && hi <= PX - MX) continue;     // zero band for every j
+        real2 xv, yl;
+        if (hi < MX) {
+            xv = Xd[lo];
+            yl = Yd[lo];
+        } else if (lo > PX - MX) {
+            xv = Xm[PX - lo];
+            yl = Ym[PX - lo];
+        } else {
+            const int k = min(n < MX ? n : PX - n, MX - 1);
+            xv = X[k];
+            yl = Y[k];
+        }
+        const real2 yv = hasy ? yl : mk2(0.0, 0.0);
+        if (hi < MX && lo > 0)
+            v[q] = mk2(xv.x - yv.y, xv.y + yv.x);
+        else if (lo > PX - MX)
+            v[q] = mk2(xv.x + yv.y, -xv.y + yv.x);
+        else if (n == 0)
+            v[q] = mk2(xv.x, yv.x);
+        else if (n < MX)
+            v[q] = mk2(xv.x - yv.y, xv.y + yv.x);
+        else if (n > PX - MX)
+            v[q] = mk2(xv.x + yv.y, -xv.y + yv.x);
+    }
+}
+
 // One block: ROWS consecutive rows of the flattened (y, z) index, so no block
 // has idle rows but the last (ROWS <= Pz: a block meets at most two planes).
 // grid (row blocks, members).  LDS: ROWS NSEQ packed sequences at a stride of
@@ -96,7 +136,7 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
     using P = XrowPlan<MODE, PX>;
     constexpr int NF = P::NF, NOUT = P::NOUT, NSEQ = P::NSEQ, NSO = P::NSO;
     constexpr int ROWS = P::ROWS, T = P::T, SP = P::SP, MX = PX / 3;
-    constexpr int R1 = plan_radix(PX, 0), NB1 = PX / R1, NP = plan_best(PX).passes;
+    constexpr int R1 = plan_radix(PX, 0), NP = plan_best(PX).passes;
     extern __shared__ __align__(16) char lds_raw[];
     if (*a.abort_flag) return;
     real2 *lds = (real2 *) lds_raw, *twl = lds + ROWS * NSEQ * SP;
@@ -115,42 +155,6 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
     auto plane = [&](int r) { return z0 + r >= Pz ? y0 + 1 : y0; };
     auto zrow = [&](int r) { return z0 + r >= Pz ? z0 + r - Pz : z0 + r; };
     stage_twiddles_c<PX, T>(a.tw, twl);
-    // First inverse pass, the load stage: bin n < Mx takes X[n] + i Y[n], bin
-    // n > Px - Mx the conjugates at Px - n, the bins between are zero (c2r uses Re
-    // only at kx = 0).  Groups of bins in the zero band are not read.
-    auto bins = [&](int j, bool hasy, const real2 *X, const real2 *Y, real2 *v) {
-        const real2 *Xd = X + j, *Yd = Y + j;            // direct bins
-        const real2 *Xm = X - j, *Ym = Y - j;            // mirrored ones: Px - n = Px - q NB1 - j
-#pragma unroll
-        for (int q = 0; q < R1; ++q) {
-            const int lo = q * NB1, hi = lo + NB1 - 1, n = j + lo;
-            v[q] = mk2(0.0, 0.0);
-            if (lo >= MX && hi <= PX - MX) continue;     // zero band for every j
-            real2 xv, yl;
-            if (hi < MX) {
-                xv = Xd[lo];
-                yl = Yd[lo];
-            } else if (lo > PX - MX) {
-                xv = Xm[PX - lo];
-                yl = Ym[PX - lo];
-            } else {
-                const int k = min(n < MX ? n : PX - n, MX - 1);
-                xv = X[k];
-                yl = Y[k];
-            }
-            const real2 yv = hasy ? yl : mk2(0.0, 0.0);
-            if (hi < MX && lo > 0)
-                v[q] = mk2(xv.x - yv.y, xv.y + yv.x);
-            else if (lo > PX - MX)
-                v[q] = mk2(xv.x + yv.y, -xv.y + yv.x);
-            else if (n == 0)
-                v[q] = mk2(xv.x, yv.x);
-            else if (n < MX)
-                v[q] = mk2(xv.x - yv.y, xv.y + yv.x);
-            else if (n > PX - MX)
-                v[q] = mk2(xv.x + yv.y, -xv.y + yv.x);
-        }
-    };
     const int nf1 = a.nf1, nf2 = MODE == XM_ADJ2 ? a.nf2 : NF;
     // field f of row r in its input array
     auto field = [&](int f, int r) {
@@ -185,14 +189,14 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
             const int r = t / NSEQ, s2 = 2 * (t - r * NSEQ);
             const bool hasy = NF % 2 == 0 || s2 + 1 < NF;
             const real2 *X = lds + (r * NF + s2) * SB;
-            bins(j, hasy, X, X + (hasy ? SB : 0), v);
+            row_bins<PX>(j, hasy, X, X + (hasy ? SB : 0), v);
         });
     } else {
         fft_first<DS_ANY, PX, ROWS * NSEQ, SP, 1, T>(lds, +1.0, [&](int j, int t, real2 *v) {
             const int r = t / NSEQ, s2 = 2 * (t - r * NSEQ);
             const bool hasy = NF % 2 == 0 || s2 + 1 < NF;
             const real2 *X = field(s2, min(r, nr - 1));
-            bins(j, hasy, X, X + (hasy ? PM : 0), v);
+            row_bins<PX>(j, hasy, X, X + (hasy ? PM : 0), v);
         });
     }
     __syncthreads();
@@ -296,6 +300,152 @@ __global__ __launch_bounds__((XrowPlan<MODE, PX>::T)) void k_xrow(XmixArgs a, co
     }
 }
 
+// The tangent's transforms and products for members along one trajectory: the
+// state's six fields, the same for every member, are transformed once for a group
+// of members and their point values kept in registers; each member then takes
+// three packed inverse transforms instead of six.  The same transforms and
+// products as k_xrow<XM_TANGENT>, so the same bits.
+// grid (row blocks, groups); group y takes the members y nm / ny ... .  Bound as
+// k_xrow is; the next member's bins are fetched while a member is transformed (207
+// us for nine FP64 members at 64x97x64, 255 without; k_xrow 279).
+template <int PX, bool EVEN>
+__global__ __launch_bounds__((XrowPlan<XM_PRIMAL, PX>::T)) void k_xrow_shared(XmixArgs a, const real2 *W1, real2 *W2)
+{
+    using P = XrowPlan<XM_PRIMAL, PX>;                   // six fields in, three out
+    constexpr int NF = 6, NSEQ = 3, NSO = 2;
+    constexpr int ROWS = P::ROWS, T = P::T, SP = P::SP, MX = PX / 3;
+    constexpr int R1 = plan_radix(PX, 0), NP = plan_best(PX).passes;
+    extern __shared__ __align__(16) char lds_raw[];
+    if (*a.abort_flag) return;
+    real2 *lds = (real2 *) lds_raw, *twl = lds + ROWS * NSEQ * SP;
+    const int Pz = a.Pz, nrow = a.qpts * Pz;
+    const int row0 = blockIdx.x * ROWS, y0 = row0 / Pz, z0 = row0 - y0 * Pz;
+    const int PM = Pz * MX;
+    const int nr = min(ROWS, nrow - row0);
+    auto plane = [&](int r) { return z0 + r >= Pz ? y0 + 1 : y0; };
+    auto zrow = [&](int r) { return z0 + r >= Pz ? z0 + r - Pz : z0 + r; };
+    stage_twiddles_c<PX, T>(a.tw, twl);
+    // the bins of six fields wait in registers, a member ahead, and come through
+    // the tile, field f of row r at (r NF + f) SB
+    constexpr int SB = MX | 1, NIN = NF * ROWS * MX, NLD = (NIN + T - 1) / T;
+    real bx[NLD], by[NLD];
+    auto fetch = [&](const real2 *B) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int e = min((int) threadIdx.x + i * T, NIN - 1);
+            const int f = e / (ROWS * MX), rk = e - f * (ROWS * MX), r = min(rk / MX, nr - 1), k = rk % MX;
+            const real2 *p = B + ((size_t) plane(r) * NF + f) * PM + zrow(r) * MX + k;
+            bx[i] = p->x;
+            by[i] = p->y;
+        }
+    };
+    // the fetched fields at the block's points, in the tile; next: fetched meanwhile
+    auto inverse = [&](const real2 *next) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int e = threadIdx.x + i * T;
+            if (NIN % T != 0 && e >= NIN) break;
+            const int f = e / (ROWS * MX), rk = e - f * (ROWS * MX), r = rk / MX, k = rk - r * MX;
+            lds[(r * NF + f) * SB + k] = mk2(bx[i], by[i]);
+        }
+        if (next) fetch(next);
+        __syncthreads();
+        fft_first_in_place<DS_ANY, PX, ROWS * NSEQ, SP, 1, T>(lds, +1.0, [&](int j, int t, real2 *v) {
+            const int r = t / NSEQ;
+            const real2 *X = lds + (r * NF + 2 * (t - r * NSEQ)) * SB;
+            row_bins<PX>(j, true, X, X + SB, v);
+        });
+        __syncthreads();
+        lds_fft_c<PX, ROWS * NSEQ, SP, 1, T, NP, 1, R1>(lds, twl, +1.0);
+    };
+    const int m0 = blockIdx.y * a.nm / gridDim.y, m1 = (blockIdx.y + 1) * a.nm / gridDim.y;
+    const real2 *Wb = a.W1b + (size_t) m0 * a.ms_inb;
+    constexpr int NPT = ROWS * PX, MAXP = (NPT + T - 1) / T;
+    auto point = [&](int i, real *f) {
+        const int e = min((int) threadIdx.x + i * T, NPT - 1), r = e / PX, n = e - r * PX;
+        const real2 *row = lds + r * NSEQ * SP + n;
+#pragma unroll
+        for (int s = 0; s < NSEQ; ++s) {
+            f[2 * s] = row[s * SP].x;
+            f[2 * s + 1] = row[s * SP].y;
+        }
+    };
+    fetch(W1);
+    inverse(Wb);
+    real fb[MAXP][NF];
+    double cmax[2] = {0.0, 0.0};                         // CFL maxima of planes y0, y0 + 1
+#pragma unroll
+    for (int i = 0; i < MAXP; ++i) {
+        point(i, fb[i]);
+        const int e = threadIdx.x + i * T, r = e / PX;
+        if (a.check_cfl && e < NPT && r < nr) {
+            const int y = plane(r);
+            const double t = fabs(fb[i][0]) * a.cfl1 + fabs(fb[i][1]) * a.cfl2[y] + fabs(fb[i][2]) * a.cfl3;
+            cmax[0] = fmax(cmax[0], y == y0 ? t : 0.0);
+            cmax[1] = fmax(cmax[1], y == y0 ? 0.0 : t);
+        }
+    }
+    if (a.check_cfl && blockIdx.y == 0) {
+        // as k_xrow; the state, and so the maximum, is the same for every group
+        __shared__ double cw[2][T / 64];
+        const int np = z0 + nr > Pz ? 2 : 1;
+        for (int p = 0; p < np; ++p) {
+            double m = cmax[p];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+            if ((threadIdx.x & 63) == 0) cw[p][threadIdx.x >> 6] = m;
+        }
+        __syncthreads();
+        if ((int) threadIdx.x < np) {
+            double b = cw[threadIdx.x][0];
+#pragma unroll
+            for (int w = 1; w < T / 64; ++w) b = fmax(b, cw[threadIdx.x][w]);
+            atomic_max_nonneg(&a.cflmax[(y0 + threadIdx.x) * CFL_STRIDE], b);
+        }
+    }
+    for (int m = m0; m < m1; ++m) {
+        __syncthreads();                                 // the tile's last reads
+        Wb += a.ms_inb;
+        inverse(m + 1 < m1 ? Wb : nullptr);
+        real outv[MAXP][3];
+#pragma unroll
+        for (int i = 0; i < MAXP; ++i) {
+            real f[12];
+#pragma unroll
+            for (int s = 0; s < NF; ++s) f[s] = fb[i][s];
+            point(i, f + NF);
+            xmix_products<XM_TANGENT>(f, outv[i]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MAXP; ++i) {
+            const int e = threadIdx.x + i * T;
+            if (NPT % T != 0 && e >= NPT) break;
+            const int r = e / PX, n = e - r * PX;
+            lds[(r * NSO) * SP + n] = mk2(outv[i][0], outv[i][1]);
+            lds[(r * NSO + 1) * SP + n] = mk2(outv[i][2], (real) 0);
+        }
+        __syncthreads();
+        lds_fft_c<PX, ROWS * NSO, SP, 1, T, NP, 0, 1, EVEN ? DS_FORWARD : DS_ANY>(lds, twl, -1.0);
+        constexpr int NU = ROWS * NSO * MX;
+        real2 *Wm = W2 + (size_t) m * a.ms_out;
+#pragma unroll
+        for (int i = 0; i < (NU + T - 1) / T; ++i) {
+            const int e = threadIdx.x + i * T;
+            if (NU % T != 0 && e >= NU) break;
+            const int q = e / MX, k = e - q * MX, r = q / NSO, t = q - r * NSO;
+            if (r >= nr) break;
+            const real2 *Z = lds + q * SP;
+            const real2 zk = Z[k], zm = Z[k == 0 ? 0 : PX - k];
+            const real2 X = mk2((real) 0.5 * (zk.x + zm.x), (real) 0.5 * (zk.y - zm.y));
+            const real2 Yv = mk2((real) 0.5 * (zk.y + zm.y), (real) -0.5 * (zk.x - zm.x));
+            real2 *D = Wm + ((size_t) plane(r) * 3 + 2 * t) * PM + zrow(r) * MX + k;
+            D[0] = X;
+            if (t == 0) D[PM] = Yv;
+        }
+    }
+}
+
 template <int MODE, int PX>
 static Fixed<XrowKernel> one(int Pz)
 {
@@ -323,6 +473,57 @@ Fixed<XrowKernel> xrow_fixed<SC_XMODE>(int Px, int Pz)
     default: return Fixed<XrowKernel>();
     }
 }
+
+// Where the shared form is taken: lengths 48 to 128 that are multiples of 12, from
+// four members on below 72.  Per member / shared in us, six members along one
+// trajectory, Ny = 41, Nz = 32: FP64 48 25.5 / 20.5, 72 35.1 / 32.6, 96 41.6 / 36.5,
+// 120 66.7 / 55.0, but 24 14.6 / 15.5, 54 29.0 / 30.7, 150 75.9 / 81.2; FP32 48 16.4 /
+// 14.4, 96 30.1 / 24.6, 120 50.1 / 32.4, but 24 10.5 / 12.3, 162 59.4 / 86.4, 192 52.7 /
+// 60.0 (longer rows leave few registers for the waves).  Three members: FP32 48
+// 11.3 / 11.8, FP64 60 18.3 / 19.1; two: FP64 72 17.5 / 16.3.
+constexpr bool xrow_shared_length(int px) { return px >= 48 && px <= 128 && px % 12 == 0; }
+
+// compiled with the tangent's kernels
+template <int PX>
+static Fixed<XrowKernel> one_shared(int Pz)
+{
+    using P = XrowPlan<XM_PRIMAL, PX>;
+    Fixed<XrowKernel> f;
+    if (P::ROWS > Pz) return f;
+    // the order of the forward transforms is that of the tangent's six sequences
+    if constexpr (start_length(PX))
+        f.kernel = even_rows(PX, Pz, 6) ? k_xrow_shared<PX, true> : k_xrow_shared<PX, false>;
+    else
+        f.kernel = k_xrow_shared<PX, false>;
+    f.group = P::ROWS;
+    f.threads = P::T;
+    f.lds = P::LDS;
+    return f;
+}
+
+template <int MODE>
+static Fixed<XrowKernel> shared_of(int Px, int Pz, int nm)
+{
+    if (nm < (Px < 72 ? 4 : 2)) return Fixed<XrowKernel>();
+    if constexpr (MODE == XM_TANGENT) {
+        switch (Px) {
+#define SC_ONE(N) \
+        case N: \
+            if constexpr (xrow_shared_length(N)) return one_shared<N>(Pz); \
+            break;
+            SC_X_LENGTHS(SC_ONE)
+#undef SC_ONE
+        }
+    }
+    return Fixed<XrowKernel>();
+}
+
+#define SC_IS_TANGENT_XM_TANGENT 1
+#define SC_IS(m) SC_IS_(m)
+#define SC_IS_(m) SC_IS_TANGENT_##m
+#if SC_IS(SC_XMODE)
+Fixed<XrowKernel> xrow_shared_fixed(int Px, int Pz, int nm) { return shared_of<SC_XMODE>(Px, Pz, nm); }
+#endif
 
 }  // namespace SC_FFT_NS
 }  // namespace sc
