@@ -600,18 +600,24 @@ __global__ __launch_bounds__(RW_THREADS) void k_rebuild_wide(RebuildArgs a, cons
         return r;
     };
     double ca[2][CK], cb[2][CK];
-    // quarter ch of a task's coefficients as buffer loads over the whole array
-    // (rows past dimR - 1, whose basis fragments are zero, read the next rows
-    // or zero past the end)
+    // quarter ch of a task's coefficients as buffer loads over the whole array.
+    // Rows past the matrix read as zero (an offset past the array), as whatever
+    // else lies there may not be finite: the alpha rows dimQ and dimQ + 1, which
+    // carry nothing, and the rows after a column's last.  Only the k-steps from
+    // RP on can hold one (dimQ >= 95 at 32 k-steps).
     const unsigned cbytes = (unsigned) ((size_t) a.Nz * 2 * nR * M2 * sizeof(double));
+    constexpr int RP = NKS - 9, PAST = 0x7ffffff8;
     auto load = [&](const RebuildTask &t, int ch) {
         __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *) t.cd, 0, cbytes, 0x00020000);
         const int va = (int) (unsigned) ((t.offA + kq * M2) * 8), vb = (int) (unsigned) ((t.offB + kq * M2) * 8);
+        // (the mean task's fragments are both R rows)
+        const int limA = t.offA == t.offB ? nR : a.dimQ;
 #pragma unroll
         for (int s = 0; s < CK; ++s) {
-            const int so = (ch * CK + s) * 4 * M2 * 8;
-            ca[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, va, so, 0));
-            cb[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, vb, so, 0));
+            const int ks = ch * CK + s, so = ks * 4 * M2 * 8, j = ks * 4 + kq;
+            const int oa = ks >= RP && j >= limA ? PAST : va, ob = ks >= RP && j >= nR ? PAST : vb;
+            ca[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, oa, so, 0));
+            cb[ch & 1][s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, ob, so, 0));
         }
     };
     auto chunk = [&](int ch, mf4 *acc) {
