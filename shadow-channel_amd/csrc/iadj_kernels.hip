@@ -161,8 +161,10 @@ __device__ __forceinline__ void chain_subst(double *v, const double *L, const do
 
 // Row i of the operator (alpha: -(k2 Qs + Qps) + cv V, V = k2^2 Qs + 2 k2 Qps +
 // Qpps; beta: Rs - cv V, V = -(Rps + k2 Rs)) on v and of the viscous part V on m
-// (rows in LDS): e, mm.  The Gram bands are zero outside the
-// matrix, so columns are clamped and none is skipped; Qps reaches three off-diagonals of the four, Qpps two, Rps one of two.
+// (rows in LDS): e, mm.  No column is skipped: the Gram bands are zero outside the
+// matrix, and what they meet there is a zero of its own (a clamped column would
+// be one of the other parity's, and that need not be finite).  Qps reaches three
+// off-diagonals of the four, Qpps two, Rps one of two.
 template <bool B>
 struct BandRow {
     static constexpr int DL = B ? 2 : 4, W = 2 * DL + 1;
@@ -177,13 +179,14 @@ struct BandRow {
         }
     }
     __device__ __forceinline__ void apply(int i, int N, double k2, double cv, const cplx *v, const cplx *m,
-                                          cplx &e, cplx &mm) const
+                                          const cplx *zero, cplx &e, cplx &mm) const
     {
         e = mm = make_double2(0.0, 0.0);
         const double k4 = k2 * k2, t2 = 2. * k2;
 #pragma unroll
         for (int o = 0; o < W; ++o) {
-            const int col = min(max(i + 2 * (o - DL), 0), N - 1);
+            const int col = i + 2 * (o - DL);
+            const bool in = o == DL || (o < DL ? col >= 0 : col < N);
             const bool hp = o > 0 && o < W - 1;
             const double ks = hp ? __builtin_fma(k2, s[o], p[o]) : k2 * s[o];     // k2 Qs + Qps
             double vs, ex;
@@ -195,7 +198,7 @@ struct BandRow {
                 if (o > 1 && o < W - 2) vs += pp[o];
                 ex = __builtin_fma(cv, vs, -ks);
             }
-            const cplx cv2 = v[col], mv = m[col];
+            const cplx cv2 = *(in ? v + col : zero), mv = *(in ? m + col : zero);
             e.x = __builtin_fma(ex, cv2.x, e.x);
             e.y = __builtin_fma(ex, cv2.y, e.y);
             mm.x = __builtin_fma(vs, mv.x, mm.x);
@@ -208,7 +211,7 @@ struct BandRow {
 // block's columns
 template <bool B, class Valid>
 __device__ __forceinline__ void mode_rhs(const IadjArgs &a, int i, int z, int x0, double kz, const cplx *vec,
-                                         const cplx *smic, const Valid &valid, cplx *acc)
+                                         const cplx *smic, const cplx *zero, const Valid &valid, cplx *acc)
 {
     const int dQ = a.dQ, dR = a.dR, Mx = a.Mx, Nz = a.Nz, k = a.k, N = B ? dR : dQ;
     const double dt = a.dt, re = a.re;
@@ -225,7 +228,7 @@ __device__ __forceinline__ void mode_rhs(const IadjArgs &a, int i, int z, int x0
         if (k == 0) {
             cplx e, m;
             g.apply(i, N, k2, B ? -re * kA[0] * dt : re * kA[0] * dt, vec + t * dR,
-                    smic + t * 2 * dR + (B ? dR : 0), e, m);
+                    smic + t * 2 * dR + (B ? dR : 0), zero, e, m);
             c = cadd(e, cscale(m, re * dt * (kA[0] + kB[0])));
         }
         cplx gf = B ? a.Fb[((size_t) z * dR + i) * Mx + x] : a.Fa[((size_t) z * dQ + i) * Mx + x];
@@ -256,7 +259,7 @@ __device__ __forceinline__ void mode_rhs(const IadjArgs &a, int i, int z, int x0
 // MIC[count - 1]
 template <bool B, class Valid>
 __device__ __forceinline__ void mode_next(const IadjArgs &a, int i, int z, int x0, double kz, const cplx *vec,
-                                          const cplx *smic, const Valid &valid)
+                                          const cplx *smic, const cplx *zero, const Valid &valid)
 {
     const int dQ = a.dQ, dR = a.dR, Mx = a.Mx, Nz = a.Nz, k = a.k, N = B ? dR : dQ;
     const double dt = a.dt, re = a.re;
@@ -269,7 +272,7 @@ __device__ __forceinline__ void mode_next(const IadjArgs &a, int i, int z, int x
         const double kx = a.Kx[x], k2 = kx * kx + kz * kz;
         cplx e, m;
         g.apply(i, N, k2, B ? -re * kA[k + 1] * dt : re * kA[k + 1] * dt, vec + t * dR,
-                smic + t * 2 * dR + (B ? dR : 0), e, m);
+                smic + t * 2 * dR + (B ? dR : 0), zero, e, m);
         cplx gf = B ? a.FLb[((size_t) z * dR + i) * Mx + x] : a.FLa[((size_t) z * dQ + i) * Mx + x];
         if (a.F) gf = cadd(gf, a.F[((((size_t) 1 * 2 + (B ? 1 : 0)) * Nz + z) * Mx + x) * dR + i]);
         const cplx c = cadd(cadd(e, cscale(gf, dt * kD[k + 1])), cscale(m, re * dt * (kA[k + 1] + kB[k + 1])));
@@ -476,7 +479,8 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
         if (tid < 2 * nx) a.IAUb[(tid / nx) * wp + (size_t) z * Mx + x0 + tid % nx] = make_double2(0.0, 0.0);
         return;
     }
-    cplx *sal = sh;                          // [t][dR]
+    cplx *zero = sh;                         // a zero (BandRow)
+    cplx *sal = zero + 1;                    // [t][dR]
     cplx *sbe = sal + IA_XG * dR;            // [t][dR]
     // MIC[count] for the right-hand sides, the factors for the solves, then
     // MIC[count - 1]: [t][2][dR]
@@ -556,6 +560,7 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
         }
     }
     if (k == 0) put_mic();
+    if (tid == 0) *zero = make_double2(0.0, 0.0);
     __syncthreads();
     // right-hand sides: thread rows i (alpha: tid < 128, beta: tid >= 128)
     const bool isb = tid >= 128;
@@ -563,9 +568,9 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
     const int N = isb ? dR : dQ;
     cplx acc[IA_XG];
     if (isb) {
-        if (i < dR) mode_rhs<true>(a, i, z, x0, kz, sbe, smic, valid, acc);
+        if (i < dR) mode_rhs<true>(a, i, z, x0, kz, sbe, smic, zero, valid, acc);
     } else {
-        if (i < dQ) mode_rhs<false>(a, i, z, x0, kz, sal, smic, valid, acc);
+        if (i < dQ) mode_rhs<false>(a, i, z, x0, kz, sal, smic, zero, valid, acc);
     }
     __syncthreads();
     if (i < N) {
@@ -652,9 +657,9 @@ __global__ __launch_bounds__(IA_THREADS) void k_iadj_modes(IadjArgs a)
     }
     __syncthreads();
     if (isb) {
-        if (i < dR) mode_next<true>(a, i, z, x0, kz, sbe, smic, valid);
+        if (i < dR) mode_next<true>(a, i, z, x0, kz, sbe, smic, zero, valid);
     } else {
-        if (i < dQ) mode_next<false>(a, i, z, x0, kz, sal, smic, valid);
+        if (i < dQ) mode_next<false>(a, i, z, x0, kz, sal, smic, zero, valid);
     }
 }
 
@@ -789,7 +794,7 @@ int launch_iadj(Context &c, int k, int count, cplx *IAC, const cplx *IU, const c
     a.sbt = c.sbt; a.mirror = c.factor_mirror ? 1 : 0;
     const size_t nrq = solve_rows(nQ), nrr = solve_rows(nR);
     const size_t fac = sizeof(double) * 2 * IA_XG * (9 * nrq + 5 * nrr);
-    const size_t lds_modes = sizeof(cplx) * 2 * IA_XG * (size_t) nR +
+    const size_t lds_modes = sizeof(cplx) * (2 * IA_XG * (size_t) nR + 1) +
                              std::max(fac, sizeof(cplx) * 2 * IA_XG * (size_t) nR);
     const size_t lds_mean = sizeof(cplx) * 6 * (size_t) nR +
                             sizeof(double) * (8 * (size_t) q + 10 * nrr);
