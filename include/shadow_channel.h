@@ -294,8 +294,11 @@ int sc_precision(void);
 /* Launch shapes (no counterpart in the reference).  sc_set_tuning(name,
    value) sets, for all later launches of the process, one of
      "solve_members_per_block"  1, 2 or 4 members whose band solves share a
-                                block and its staged factor image (0: 2, or
-                                one where they do not fit);
+                                block and its staged factor image (4 run as
+                                2 where no more fit a block's registers and
+                                LDS: Ny 131 to 178, 275 to 354 and from 451
+                                on; 0: 2, or 1 where a thread would hold
+                                more than six of their rows);
      "rebuild_blocks"           blocks per XCD of the parity rebuild (<= 256);
      "force_blocks"             blocks per pair of i-tiles of the parity
                                 projection (multiple of 8, <= 256);

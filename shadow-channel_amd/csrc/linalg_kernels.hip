@@ -2506,16 +2506,18 @@ int solve_columns_per_block(int dimR)
     return 0;
 }
 
-// Members per solve block (1, 2 or 4): the tuning's choice when set, else 2 (32
-// members at 64x97x64: 232 us a launch, 262 with one: the second member's vectors
-// come while the first's chain runs, and a third would take the LDS of a block);
-// fewer when the run has fewer members, when a worker would hold more than six
-// rows of them in registers, or when two blocks would not fit a CU's LDS.
-int solve_members_per_block(const Context &c)
+// Members per solve block (1, 2 or 4) of a run of nrun members: the tuning's choice
+// when set, else 2 (32 members at 64x97x64: 232 us a launch, 262 with one: the second
+// member's vectors come while the first's chain runs, and a third would take the LDS
+// of a block) while a worker holds no more than six rows of them in registers; fewer
+// when the run has fewer members, when two blocks would not fit a CU's LDS, or when a
+// worker's rows would not fit its registers (four members of more than three rows).
+int solve_members(int dimR, int sbt, int nrun, int tuned)
 {
-    int mb = tuning().solve_mb > 0 ? tuning().solve_mb : 2;
-    while (mb > 1 && (mb > c.nrun || mb * solve_slots(c.d.dimR, c.sbt) > 6 ||
-                      2 * solve_lds_bytes(c.d.dimR, c.sbt, mb) > 160 * 1024))
+    const int slots = solve_slots(dimR, sbt);
+    int mb = tuned > 0 ? tuned : 2;
+    while (mb > 1 && (mb > nrun || (tuned > 0 ? mb == 4 && slots > 3 : mb * slots > 6) ||
+                      2 * solve_lds_bytes(dimR, sbt, mb) > 160 * 1024))
         mb /= 2;
     return mb;
 }
@@ -2525,11 +2527,9 @@ typedef void (*SolveKernel)(SolveArgs, cplx *, cplx *);
 template <int SBT, int VR>
 static SolveKernel solve_kernel_mb(int mb)
 {
-    if constexpr (4 * VR <= 6)
+    if constexpr (VR <= 3)
         if (mb == 4) return k_solve<SBT, VR, 4>;
-    if constexpr (2 * VR <= 6)
-        if (mb == 2) return k_solve<SBT, VR, 2>;
-    return k_solve<SBT, VR, 1>;
+    return mb == 2 ? k_solve<SBT, VR, 2> : k_solve<SBT, VR, 1>;
 }
 
 template <int SBT>
@@ -2591,7 +2591,7 @@ void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cp
                    fcols * 8.0 * (9.0 * d.dimQ + 5.0 * d.dimR);
     const int sbt = c.sbt;
     const int ncol = d.Nz * d.Mx;
-    const int mb = solve_members_per_block(c);
+    const int mb = solve_members(d.dimR, sbt, c.nrun, tuning().solve_mb);
     const size_t lds = solve_lds_bytes(d.dimR, sbt, mb);
     a.nm = c.nrun;
     a.ngrp = (c.nrun + mb - 1) / mb;
