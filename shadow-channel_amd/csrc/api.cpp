@@ -368,14 +368,21 @@ static void pass2_adjoint_pair(Context &c, const cplx *AUb, const cplx *wa, cons
     }
 }
 
-// Host arrays pass through pinned memory of the context, a chunk at a time, the
-// host's copy of one chunk under the transfer of the others.  A pageable array of
-// 64 KB takes 34 us each way directly (the runtime pins it for the call) and 9 so;
-// 1 MB 60 to 140 us down, 40 so; the 5.4 MB of physical fields at 32x65x32 300 us
-// down, of which the link needs 101, 190 so (the host reads what the link has just
-// written at 35 GB/s; chunks of 512 KB end in 330 us instead of 275 to 300 for the call,
-// as every chunk costs a hand-over between queues, one chunk in 345).  The stop
-// flag costs 2 us behind a run's last kernel, 34 as a copy of its own.
+// Host arrays pass through pinned memory of the context where a copy of the pageable
+// array takes longer: downloads, a chunk at a time with the host's copy of one under
+// the transfer of the others, and uploads of up to one chunk.  Larger uploads are
+// left to the runtime, which pins the array: the host's copy into the chunks takes
+// longer.  Direct / through chunks in us, a call about it included; the runtime stages
+// up to 1 MB itself, several times slower until 16 MB have passed (in brackets):
+//   up: 16 KB 52 / 40, 64 KB 60 (83) / 56, 254 KB 65 (159) / 62, 1 MB 106 (474) / 102,
+//     but 1.3 MB 126 / 155, 2.9 MB 163 / 220, 6.2 MB 267 / 332, 33 MB 1246 / 1325;
+//   down: 16 KB 22 / 14, 64 KB 12 (36) / 12, 254 KB 21 (113) / 21, 1 MB 54 (116) / 53,
+//     1.3 MB 81 / 75, 6.2 MB 338 / 245, 33 MB 1900 / 1260.
+// One chunk takes no events (7 us of each call).  The 5.4 MB of physical fields at
+// 32x65x32 come in 190 us, of which the link needs 101: the host reads what the link
+// has just written at 35 GB/s.  Chunks of 512 KB end in 330 us instead of 275 to 300
+// for the call, as every chunk costs a hand-over between queues, one chunk in 345.
+// The stop flag costs 2 us behind a run's last kernel, 34 as a copy of its own.
 // Memory that the runtime knows (pinned, managed, a device's) is copied directly.
 static void alloc_pinned(Context &c)
 {
@@ -415,17 +422,16 @@ static int wait_slot(Context &c, int s)
 // on return where it went through pinned memory
 static int stage_in(Context &c, void *dst, const void *src, size_t n)
 {
-    if (!through_pinned(c, src)) {
-        SC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c.stream));
-        return SC_OK;
-    }
-    for (size_t o = 0; o < n; o += PIN_CHUNK) {
-        const size_t m = std::min(PIN_CHUNK, n - o);
-        const int s = c.pin_next++ % PIN_SLOTS;
-        char *slot = c.pin + s * PIN_CHUNK;
+    const void *from = src;
+    const int s = c.pin_next % PIN_SLOTS;
+    const bool pinned = n <= PIN_CHUNK && through_pinned(c, src);
+    if (pinned) {
+        ++c.pin_next;
         if (int rc = wait_slot(c, s)) return rc;
-        memcpy(slot, (const char *) src + o, m);
-        SC_HIP(hipMemcpyAsync((char *) dst + o, slot, m, hipMemcpyHostToDevice, c.stream));
+        from = memcpy(c.pin + s * PIN_CHUNK, src, n);
+    }
+    SC_HIP(hipMemcpyAsync(dst, from, n, hipMemcpyHostToDevice, c.stream));
+    if (pinned) {
         SC_HIP(hipEventRecord(c.pin_ev[s], c.stream));
         c.pin_busy[s] = true;
     }
@@ -438,6 +444,13 @@ static int stage_out(Context &c, void *dst, const void *src, size_t n)
     if (!through_pinned(c, dst)) {
         SC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c.stream));
         SC_HIP(hipStreamSynchronize(c.stream));
+        return SC_OK;
+    }
+    if (n <= PIN_CHUNK) {
+        char *slot = c.pin + c.pin_next % PIN_SLOTS * PIN_CHUNK;
+        SC_HIP(hipMemcpyAsync(slot, src, n, hipMemcpyDeviceToHost, c.stream));
+        SC_HIP(hipStreamSynchronize(c.stream));
+        memcpy(dst, slot, n);
         return SC_OK;
     }
     const size_t nch = (n + PIN_CHUNK - 1) / PIN_CHUNK;

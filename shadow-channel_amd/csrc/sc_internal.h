@@ -27,7 +27,7 @@ typedef double2 cplx;
 // launch update them with atomics (145 planes in 10 lines: 4 us of the primal x
 // kernel's 27 at 64x64x97)
 constexpr int CFL_STRIDE = 16;
-// host arrays: chunks of pinned memory (see stage_in)
+// host arrays: chunks of pinned memory (see alloc_pinned)
 constexpr int PIN_SLOTS = 4;
 constexpr size_t PIN_CHUNK = 1024 * 1024;
 constexpr int MAXF = 12;        // fields in one z-inverse launch
