@@ -259,7 +259,9 @@ int sc_adjoint_dev(int start_step, int end_step, sc_complex *AC_dev, double stre
 /* The primal keeps, per stored stage state, its velocity and vorticity after
    the z transform, so that the tangent and adjoint need not rebuild and
    transform that state again (capacity traded for recomputation; the results
-   are bitwise the same).  c_init allocates it when it fits in half of the
+   are bitwise the same, but for the adjoint's last bits at Nx = 32 when Nz / 2
+   is 4 more than a multiple of 8 and at Nx = 64 when it is 2 more than one of
+   4).  c_init allocates it when it fits in half of the
    free device memory and it is enabled (default 1); the setting applies to
    the next c_init.  sc_field_cache_active reports whether it is allocated. */
 int sc_set_field_cache(int enable);

@@ -147,8 +147,11 @@ template <int R> __device__ __forceinline__ void dft_prime(real2 *v, real sign)
 // How the first pass of a transform rounds its constant twiddles (see
 // rounds_by_y).  Two lengths, 48 and 96, have an order of their own on the grids
 // that tile evenly (even_columns, even_rows), the general one on the others.
-// Both are as accurate; each grid keeps its order, so that its results are the
-// same bits whatever kernel computes them.
+// Both are as accurate; each grid keeps its order, so that a transform has the same
+// bits in whatever kernel of the same fields.  (The merged adjoint kernel packs
+// eight sequences, the single one five: on grids whose z rows come in the groups of
+// the one only, 4 against 8 at 48 points and 2 against 4 at 96, an adjoint with
+// cached fields and one without differ in the last bits.)
 enum DftStart : int {
     DS_ANY = 0,        // the general order; every pass but the first
     DS_FORWARD = 1,    // forward transforms
@@ -160,12 +163,13 @@ constexpr bool start_length(int n) { return n == 48 || n == 96; }
 inline bool even_columns(int Mx) { return Mx % 16 == 0; }
 // x transforms: the z rows come in groups of a 2048-value tile, nseq packed
 // sequences a row
-inline bool even_rows(int Px, int Pz, int nseq)
+constexpr int even_group(int px, int nseq)
 {
     int rows = 1;
-    while (2 * rows <= 64 && 2 * rows * nseq * (Px + 1) + Px <= 2048) rows *= 2;
-    return rows <= Pz && Pz % rows == 0;
+    while (2 * rows <= 64 && 2 * rows * nseq * (px + 1) + px <= 2048) rows *= 2;
+    return rows;
 }
+inline bool even_rows(int Px, int Pz, int nseq) { return Pz % even_group(Px, nseq) == 0; }
 
 // Whether the real (im = 0) or imaginary (im = 1) part of t w, w = (c, s) the
 // twiddle of (m2, k1) in a composite DFT, takes its t.y term (t.x otherwise) in

@@ -452,6 +452,8 @@ static Fixed<XrowKernel> one(int Pz)
     using P = XrowPlan<MODE, PX>;
     Fixed<XrowKernel> f;
     if (P::ROWS > Pz) return f;                          // a block would meet a third plane
+    // (the runtime-length kernel, which then runs, has the general order only)
+    static_assert(!start_length(PX) || P::ROWS <= even_group(PX, P::NSEQ), "a grid with an order of its own runs this kernel");
     if constexpr (start_length(PX) && P::NOUT > 0)
         f.kernel = even_rows(PX, Pz, P::NSEQ) ? k_xrow<MODE, PX, true> : k_xrow<MODE, PX, false>;
     else
