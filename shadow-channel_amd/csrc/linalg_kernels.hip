@@ -1497,6 +1497,9 @@ __global__ __launch_bounds__(FR_THREADS) void k_force_par(ForceArgs a, int bpi, 
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         const double hx = r[w][h][0], hz = r[w][h][1], hy = r[w][h][2];
+                        // which product is rounded: either is as accurate, and the
+                        // primal's results with eight k-steps (qpts <= 64) have been
+                        // those of the second form, which keeps their last bits
                         vP[h] = ADJ || NKS != 8 ? __builtin_fma(px, hx, pz * hz)
                                                 : __builtin_fma(pz, hz, px * hx);
                         vY[h] = ky * hy;
@@ -1619,13 +1622,15 @@ static void launch_force_par(const ForceArgs &a, int npair, int ntask, int nprob
     // members: 460 us, with two waves a task 480; FP64 slots leave no registers
     // for both halves' sums: nine members 73 us, with two waves 44.5); two waves
     // a task otherwise
-    if constexpr (ForceParShape<ADJ, NKS, P32, 1>::NH > 1) {
+    constexpr bool pairs = ForceParShape<ADJ, NKS, P32, 1>::NH > 1;
+    if constexpr (pairs) {
         if (!P32 || nall < 8 * bpi) {
             launch_force_par_ks<ADJ, NKS, P32, 2>(a, npair, bpi, nprob, U0, Fa0, Fb0, U1, Fa1, Fb1, st);
             return;
         }
     }
-    launch_force_par_ks<ADJ, NKS, P32, 1>(a, npair, bpi, nprob, U0, Fa0, Fb0, U1, Fa1, Fb1, st);
+    if constexpr (P32 || !pairs)
+        launch_force_par_ks<ADJ, NKS, P32, 1>(a, npair, bpi, nprob, U0, Fa0, Fb0, U1, Fa1, Fb1, st);
 }
 
 template <bool ADJ, int NKS>
@@ -2071,8 +2076,11 @@ __device__ __forceinline__ void solve_block(const SolveArgs &a, int var, int par
     }
 
     // L factors: every thread, in flight while the chain wave is chosen (LB and
-    // UB 16-byte loads a thread cover the rows that VR slots hold)
+    // UB 16-byte loads a thread cover the rows that VR slots hold, whole eights)
     constexpr int LB = DL == 4 ? (3 * VR + 1) / 2 : VR, UB = DL == 4 ? (5 * VR + 1) / 2 : (3 * VR + 1) / 2;
+    static_assert(RSTEP % 8 == 0 && 2 * LB * SOLVE_THREADS >= VR * RSTEP * DL * SBT &&
+                      2 * UB * SOLVE_WORKERS >= VR * RSTEP * (DL + 1) * SBT,
+                  "the loads cover the image");
     const v2d *src = (const v2d *) (var == 0 ? a.La : a.Lb) + ((size_t) fb * 2 + par) * (nrp * NE * SBT / 2);
     const int nl = nrp * DL * SBT / 2, nu = nrp * (DL + 1) * SBT / 2;
     v2d lt[LB], ut[UB];
@@ -2085,7 +2093,6 @@ __device__ __forceinline__ void solve_block(const SolveArgs &a, int var, int par
 #pragma unroll
         for (int i = 0; i < LB; ++i)
             if (tid + i * SOLVE_THREADS < nl) ((v2d *) fl)[tid + i * SOLVE_THREADS] = lt[i];
-        for (int e = tid + LB * SOLVE_THREADS; e < nl; e += SOLVE_THREADS) ((v2d *) fl)[e] = src[e];
     };
     // The chain wave and the workers take separate paths with the same barriers
     // (each is uniform in its waves), so that neither holds the other's values in
@@ -2207,7 +2214,6 @@ __device__ __forceinline__ void solve_block(const SolveArgs &a, int var, int par
 #pragma unroll
     for (int i = 0; i < UB; ++i)
         if (wt + i * SOLVE_WORKERS < nu) dst[wt + i * SOLVE_WORKERS] = ut[i];
-    for (int e = wt + UB * SOLVE_WORKERS; e < nu; e += SOLVE_WORKERS) dst[e] = src[nl + e];
     if (a.has_next && nr > 0) {
 #pragma unroll
         for (int t = 0; t < VR; ++t) {
@@ -2532,12 +2538,16 @@ static SolveKernel solve_kernel_mb(int mb)
     return mb == 2 ? k_solve<SBT, VR, 2> : k_solve<SBT, VR, 1>;
 }
 
+// the shapes that solve_columns_per_block leads to: one row slot only with 8
+// columns, four only with 8 or 4 (256 rows at most)
 template <int SBT>
 static SolveKernel solve_kernel(int slots, int mb)
 {
-    if (SBT == 8 && slots == 1) return solve_kernel_mb<SBT, 1>(mb);
-    if (slots <= 2) return solve_kernel_mb<SBT, 2>(mb);
-    return slots == 3 ? solve_kernel_mb<SBT, 3>(mb) : solve_kernel_mb<SBT, 4>(mb);
+    if constexpr (SBT == 8)
+        if (slots == 1) return solve_kernel_mb<SBT, 1>(mb);
+    if constexpr (SBT > 2)
+        if (slots == 4) return solve_kernel_mb<SBT, 4>(mb);
+    return slots == 3 ? solve_kernel_mb<SBT, 3>(mb) : solve_kernel_mb<SBT, 2>(mb);
 }
 
 void launch_solve(Context &c, cplx *Ccarry, cplx *Csol, int k, int adj, const cplx *Fa2,
