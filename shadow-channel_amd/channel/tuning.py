@@ -5,10 +5,10 @@ for bit) but do change speed with the grid and the number of members
 (sc_set_tuning): how many members' band solves share one block and its
 staged factor image, and how many blocks the parity y-transforms spread
 over.  autotune() times a short forward+adjoint window of the actual
-configuration for each candidate, one shape at a time (the others held at
-their best so far), keeps the fastest and leaves it set.  Results can be
-kept in a JSON file keyed by grid, member count and precision, so that a
-later process applies them without timing again.
+configuration for the library's own rule and each candidate, one shape at a
+time (the others held at their best so far), keeps the fastest and leaves it
+set.  Results can be kept in a JSON file keyed by grid, member count and
+precision, so that a later process applies them without timing again.
 """
 import json
 import os
@@ -22,10 +22,11 @@ import c_channel
 # an MI355X (a cache in the format autotune() writes)
 SHAPES_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "shapes.json")
 
+# candidates; 0 is the library's own rule
 SHAPES = {
-    "solve_members_per_block": (1, 2, 4),
-    "rebuild_blocks": (32, 64, 128),
-    "force_blocks": (64, 128, 256),
+    "solve_members_per_block": (0, 1, 2, 4),
+    "rebuild_blocks": (0, 32, 64, 128),
+    "force_blocks": (0, 64, 128, 256),
 }
 
 
