@@ -64,13 +64,17 @@ constexpr XrowShape xrow_shape(int px, int nseq, int nso)
 
 // Whether the fields' bins come into LDS first, row by row as they lie in memory
 // (the first pass wants each bin twice, directly and mirrored, and a lane its own
-// sequence): lengths whose rows of Mx bins lie a multiple of 64 bytes apart, which
-// crowd the L1 when lanes read them side by side, as far as the two barriers and
-// the LDS traffic cost less.  FP32, direct / staged in us (64x97x64, 32 members):
-// primal 404 / 371, tangent 697 / 602, adjoint 628 / 562, merged adjoint 950 / 978;
-// 128x129x128, two members: merged adjoint 397 / 308, adjoint 235 / 207, primal 132 /
-// 137; other lengths within 3% either way.  FP64 at 48: primal 9.8 / 8.7, tangent
-// 12.5 / 10.8, merged adjoint 34.9 / 36.4; at 96 23.9 / 25.0 and 51.5 / 58.2.
+// sequence): lengths whose rows of Mx bins lie a multiple of 128 bytes apart (64 at
+// 24 points in FP32), which crowd the L1 when lanes read them side by side, as far
+// as the two barriers and the LDS traffic cost less.  FP32, direct / staged in us
+// (64x97x64, 32 members): primal 404 / 371, tangent 697 / 602, adjoint 628 / 562,
+// merged adjoint 950 / 978; 128x129x128, two members: merged adjoint 397 / 308,
+// adjoint 235 / 207, primal 132 / 137; three members at Ny = 41: primal 9.0 / 8.1 at
+// 24, 14.9 / 12.0 at 48, 19.7 / 17.4 at 144, 22.7 / 22.4 at 192.  The other lengths
+// there are 8% slower (30, 90, 180) to 5% faster (72 and 120, whose rows lie 64 bytes
+// off a multiple of 128), the merged adjoint at 60 12%, and read directly.  FP64 at
+// 48: primal 9.8 / 8.7, tangent 12.5 / 10.8, merged adjoint 34.9 / 36.4; at 96 23.9 /
+// 25.0 and 51.5 / 58.2.
 constexpr bool xrow_staged(int mode, int px)
 {
     if (sizeof(real) == 4) return px == 24 || (px % 48 == 0 && (mode != XM_ADJ2 || px != 96));
@@ -479,10 +483,12 @@ Fixed<XrowKernel> xrow_fixed<SC_XMODE>(int Px, int Pz)
 // Where the shared form is taken: lengths 48 to 128 that are multiples of 12, from
 // four members on below 72.  Per member / shared in us, six members along one
 // trajectory, Ny = 41, Nz = 32: FP64 48 25.5 / 20.5, 72 35.1 / 32.6, 96 41.6 / 36.5,
-// 120 66.7 / 55.0, but 24 14.6 / 15.5, 54 29.0 / 30.7, 150 75.9 / 81.2; FP32 48 16.4 /
+// 120 66.7 / 55.0, but 24 14.6 / 15.5, 54 28.9 / 30.7, 150 75.9 / 81.2; FP32 48 16.4 /
 // 14.4, 96 30.1 / 24.6, 120 50.1 / 32.4, but 24 10.5 / 12.3, 162 59.4 / 86.4, 192 52.7 /
 // 60.0 (longer rows leave few registers for the waves).  Three members: FP32 48
-// 11.3 / 11.8, FP64 60 18.3 / 19.1; two: FP64 72 17.5 / 16.3.
+// 11.3 / 11.8, FP64 60 18.3 / 19.1; two: FP64 72 17.5 / 16.3.  Two lengths outside the
+// rule would gain, 90 (FP64 44.0 / 39.7, FP32 33.0 / 27.3) and, in FP32 alone, 54
+// (22.3 / 19.3).
 constexpr bool xrow_shared_length(int px) { return px >= 48 && px <= 128 && px % 12 == 0; }
 
 // compiled with the tangent's kernels
