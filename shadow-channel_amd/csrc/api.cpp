@@ -368,20 +368,22 @@ static void pass2_adjoint_pair(Context &c, const cplx *AUb, const cplx *wa, cons
     }
 }
 
-// Host arrays pass through pinned memory of the context where a copy of the pageable
-// array takes longer: downloads, a chunk at a time with the host's copy of one under
-// the transfer of the others, and uploads of up to one chunk.  Larger uploads are
-// left to the runtime, which pins the array: the host's copy into the chunks takes
-// longer.  Direct / through chunks in us, a call about it included; the runtime stages
-// up to 1 MB itself, several times slower until 16 MB have passed (in brackets):
-//   up: 16 KB 52 / 40, 64 KB 60 (83) / 56, 254 KB 65 (159) / 62, 1 MB 106 (474) / 102,
-//     but 1.3 MB 126 / 155, 2.9 MB 163 / 220, 6.2 MB 267 / 332, 33 MB 1246 / 1325;
-//   down: 16 KB 22 / 14, 64 KB 12 (36) / 12, 254 KB 21 (113) / 21, 1 MB 54 (116) / 53,
+// Host arrays pass through pinned memory of the context, a chunk at a time, the
+// host's copy of one chunk under the transfer of the others.  Left to itself the
+// runtime stages a pageable array of up to 1 MB and pins a larger one, and until 16 MB
+// have passed that way either takes several times longer.  Directly, first calls and
+// later ones / through the chunks, in us, a call about it included:
+//   up: 16 KB 52 / 40, 64 KB 83, 60 / 56, 254 KB 159, 65 / 62, 1 MB 474, 106 / 102,
+//     1.3 MB 530, 135 / 165, 2.9 MB 1100, 170 / 225, 6.2 MB 3000 and 2290 and 1600,
+//     265 / 335, 33 MB 1246 / 1325: beyond a chunk a program of many uploads would gain
+//     a little and one of fewer than fifty lose, as the host's copy into the chunks
+//     takes longer than pinning an array does once that is warm;
+//   down: 16 KB 22 / 14, 64 KB 36, 12 / 12, 254 KB 113, 21 / 21, 1 MB 116, 54 / 53,
 //     1.3 MB 81 / 75, 6.2 MB 338 / 245, 33 MB 1900 / 1260.
-// One chunk takes no events (7 us of each call).  The 5.4 MB of physical fields at
-// 32x65x32 come in 190 us, of which the link needs 101: the host reads what the link
-// has just written at 35 GB/s.  Chunks of 512 KB end in 330 us instead of 275 to 300
-// for the call, as every chunk costs a hand-over between queues, one chunk in 345.
+// A download of one chunk takes no events (7 us of each call).  The 5.4 MB of physical
+// fields at 32x65x32 come in 190 us, of which the link needs 101: the host reads what
+// the link has just written at 35 GB/s.  Chunks of 512 KB end in 330 us instead of 275
+// to 300 for the call, as every chunk costs a hand-over between queues, one chunk in 345.
 // The stop flag costs 2 us behind a run's last kernel, 34 as a copy of its own.
 // Memory that the runtime knows (pinned, managed, a device's) is copied directly.
 static void alloc_pinned(Context &c)
@@ -422,16 +424,17 @@ static int wait_slot(Context &c, int s)
 // on return where it went through pinned memory
 static int stage_in(Context &c, void *dst, const void *src, size_t n)
 {
-    const void *from = src;
-    const int s = c.pin_next % PIN_SLOTS;
-    const bool pinned = n <= PIN_CHUNK && through_pinned(c, src);
-    if (pinned) {
-        ++c.pin_next;
-        if (int rc = wait_slot(c, s)) return rc;
-        from = memcpy(c.pin + s * PIN_CHUNK, src, n);
+    if (!through_pinned(c, src)) {
+        SC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c.stream));
+        return SC_OK;
     }
-    SC_HIP(hipMemcpyAsync(dst, from, n, hipMemcpyHostToDevice, c.stream));
-    if (pinned) {
+    for (size_t o = 0; o < n; o += PIN_CHUNK) {
+        const size_t m = std::min(PIN_CHUNK, n - o);
+        const int s = c.pin_next++ % PIN_SLOTS;
+        char *slot = c.pin + s * PIN_CHUNK;
+        if (int rc = wait_slot(c, s)) return rc;
+        memcpy(slot, (const char *) src + o, m);
+        SC_HIP(hipMemcpyAsync((char *) dst + o, slot, m, hipMemcpyHostToDevice, c.stream));
         SC_HIP(hipEventRecord(c.pin_ev[s], c.stream));
         c.pin_busy[s] = true;
     }

@@ -1,6 +1,6 @@
-"""Host arrays about the size where their way to the device and back changes (1 MB:
-just below, exactly, just above) and about 64 KB.  A run of no steps returns its
-state and stores it, exactly; repeated, so that the chunks are used again.
+"""Host arrays about the size of a chunk of pinned memory (1 MB: just below, exactly,
+just above), where their way back changes, and about 64 KB.  A run of no steps returns
+its state and stores it, exactly; repeated, so that the chunks are used again.
 """
 import numpy as np
 import pytest
