@@ -562,9 +562,9 @@ __global__ __launch_bounds__(256, 2) void k_rebuild_rows(RebuildArgs a, const cp
 // (or the next task's first) issued before the current quarter's products.
 // Bound by the FP64 products (113 us for two members at 128x129x128); the form
 // that stages the basis chunk by chunk behind a barrier, for four waves that
-// start and end every n-tile together, took 262 us, this one 188: the products take
-// 72% of its clocks with the divisions and other FP64 instructions that share
-// their unit; the rest is the change of basis and re-reading coefficients.
+// start and end every n-tile together, took 262 us, this one 187: the products take
+// 61% of its clocks and the divisions and other vector instructions, which share
+// their unit, 12%; the rest is the change of basis and re-reading coefficients.
 constexpr int RW_THREADS = 512;
 template <int NKS>
 __global__ __launch_bounds__(RW_THREADS) void k_rebuild_wide(RebuildArgs a, const cplx *C, cplx *U)
